@@ -2,6 +2,7 @@
 // include/streams_mi355x.h) and the host-side ordering of the hot loop.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -246,7 +247,7 @@ hipError_t dalloc(T **p, size_t n) {
 void free_all(st_solver *s) {
     void *ptrs[] = {s->w_alloc ? s->w_alloc : (void *)s->w, s->w_aux_alloc ? s->w_aux_alloc : s->w_aux, s->F[0], s->F[1], s->wallprop, s->eoc[0], s->eoc[1], s->eoc[2], s->x, s->y,
                     s->z, s->yn, s->dcsidx, s->dcsidxs, s->dcsidx2, s->detady, s->detadys, s->detady2, s->dzitdz,
-                    s->dzitdzs, s->dzitdz2, s->ds, s->partials, s->dirty, s->counters, s->fixlist, s->rc_real, s->rc_maps,
+                    s->dzitdzs, s->dzitdz2, s->ds, s->partials, s->dirty, s->counters, s->fixlist, s->hot, s->hot_rec, s->hot_dirty, s->rc_real, s->rc_maps,
                     s->w_stat, s->rplane, s->rng_coef, s->rng_win, s->rng_ctl, s->wrecyc, s->fhat, s->fln};
     for (void *p : ptrs) {
         if (!p) continue;
@@ -288,6 +289,31 @@ struct TimeScope {
 // The mixed form with the Laplacian viscous terms refines the Ducros sensor
 // near the threshold in FP64 from w (its fluxes and stresses stay FP32).
 bool fp64_sensor(const st_solver *s) { return s->mixed && s->p.conservative_viscous != 1; }
+
+// one RK stage of rk_sync in four launches (st_stage.hip), plus the step's
+// WENO masks at its first stage; end: the last stage of a st_advance step
+int stage_one_pass(st_solver *s, int istep, bool end) {
+    using namespace st;
+    void *fprev = s->F[s->cur], *fcur = s->F[s->cur ^ 1];
+    const Geo &g = s->g;
+    const bool dt = istep == 0 && s->dt_in_stage && s->p.cfl > 0;
+    if (istep == 0) TIMED(ST_K_WENO_FIX, launch_hot_items(s));
+    TIMED(ST_K_AUX, launch_aux(s, 1 - g.ng, g.nx + g.ng, 1 - g.ng, g.ny + g.ng, 1 - g.ng, g.nz + g.ng, true, dt, true));
+    if (istep == 0) s->dt_in_stage = false;
+    TIMED(ST_K_EULER_XY, launch_flux(s, fcur, istep));
+    if (istep == 2 && fp64_sensor(s)) TIMED(ST_K_SENSOR, launch_sensor_refine(s, false, true));
+    TIMED(ST_K_WENO_FIX, launch_weno_items(s, fcur, istep, dt));
+    if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur));
+    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end));
+    if (s->p.channel_case && s->p.theta_wall >= -1.0)
+        TIMED(ST_K_FORCE_VAR, launch_force_var(s, one_pass_update_blocks(g)));
+    if (s->recyc) TIMED(ST_K_BC, launch_inflow_draws(s));
+    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s));
+    s->cur ^= 1;
+    s->last_stage = istep;
+    s->fln_current = false;
+    return ST_OK;
+}
 
 // one RK stage of rk_sync (singleideal_cpu.F90:352-406), fused
 int stage(st_solver *s, int istep) {
@@ -342,7 +368,7 @@ int stage(st_solver *s, int istep) {
     if (s->p.channel_case) TIMED(ST_K_FINISH, launch_force_finish(s, istep));
     if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur));  // bc_nr
     TIMED(ST_K_UPDATE, launch_update(s, fprev, fcur, istep));
-    if (s->p.channel_case && s->p.theta_wall >= -1.0) TIMED(ST_K_FORCE_VAR, launch_force_var(s));
+    if (s->p.channel_case && s->p.theta_wall >= -1.0) TIMED(ST_K_FORCE_VAR, launch_force_var(s, update_blocks(g)));
     // get_crandom_f of euler_z: the random inflow plane of this stage
     if (s->recyc) TIMED(ST_K_BC, launch_inflow_draws(s));
     if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s));  // update_ghost(do_swap=0)
@@ -352,17 +378,20 @@ int stage(st_solver *s, int istep) {
     return ST_OK;
 }
 
-int do_rk_sync(st_solver *s) {
+// end: the step of st_advance, which also moves time and the step counter
+int do_rk_sync(st_solver *s, bool end) {
+    const bool one = st::one_pass_stage(s);
     for (int istep = 0; istep < 3; istep++) {
-        int rc = stage(s, istep);
+        int rc = one ? stage_one_pass(s, istep, end && istep == 2) : stage(s, istep);
         if (rc) return rc;
     }
+    if (end && !one) TIMED(ST_K_STEP_END, st::launch_step_end(s));
     return ST_OK;
 }
 
 // The device arrays of one solve, in allocation order, and their sizes in
 // bytes (st_solver_footprint sums them, each rounded up to 256 bytes).
-constexpr int kNArrays = 26;
+constexpr int kNArrays = 29;
 constexpr size_t kArenaAlign = 256;
 size_t arena_align(size_t n) { return (n + kArenaAlign - 1) / kArenaAlign * kArenaAlign; }
 
@@ -373,6 +402,16 @@ int partial_slots(const st::Geo &g) {
     // 5 x 256 force_rhs partials, and the 128 x 8 second-level values at the end
     const int aux_blk = (int)((st::aux_lanes(g) + 255) / 256);
     return (7 * nblk > aux_blk ? 7 * nblk : aux_blk) + 256 * 5 + 128 * 8;
+}
+
+// the one-pass stage's scratch: the sums of k_flux share the head with the
+// partials above; the CFL maxima and the second-level values follow them
+int partial_head(const st::Geo &g, bool mixed) {
+    const int a = partial_slots(g) - 128 * 8, b = st::one_pass_flux_slots(g, mixed), c = st::one_pass_update_blocks(g);
+    return a > b ? (a > c ? a : c) : (b > c ? b : c);
+}
+int partial_total(const st::Geo &g, bool mixed) {
+    return partial_head(g, mixed) + st::aux_dt_blocks(g) + st::kStage2Slots + 128 * 8;
 }
 
 void array_sizes(const st_params &p, size_t n[kNArrays]) {
@@ -398,10 +437,13 @@ void array_sizes(const st_params &p, size_t n[kNArrays]) {
     for (int r = 0; r < 3; r++) n[q++] = d * g.ny;  // detady ...
     for (int r = 0; r < 3; r++) n[q++] = d * g.nz;  // dzitdz ...
     n[q++] = sizeof(st::DevScalars);       // ds
-    n[q++] = d * partial_slots(g);         // partials
+    n[q++] = d * partial_total(g, p.precision == ST_PREC_MIXED);         // partials
     n[q++] = nint + 64;                    // dirty flags + the any-dirty word
     n[q++] = sizeof(int) * (8 + 4096);     // counters (4096 = kFixMaxSeg)
     n[q++] = sizeof(int) * nint;           // fixlist
+    n[q++] = st::hot_bits_bytes(g);        // hot, hot_rec, hot_dirty
+    n[q++] = st::hot_rec_bytes(g);
+    n[q++] = st::hot_dirty_bytes(g);
 }
 
 // st_solver_create, or with mem the same solver inside memory the caller
@@ -438,7 +480,7 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
         return fail(ST_ERR_HIP, std::string("stream creation: ") + hipGetErrorString(e));
     }
     const size_t nvol = g.nvol, nint = g.nint;
-    s->npart = partial_slots(g);
+    s->npart = partial_total(g, s->mixed);
     size_t n[kNArrays];
     array_sizes(*p, n);
     void **dst[kNArrays] = {(void **)&s->w, &s->w_aux, &s->F[0], &s->F[1], (void **)&s->wallprop,
@@ -447,7 +489,8 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
                             (void **)&s->dcsidxs, (void **)&s->dcsidx2, (void **)&s->detady, (void **)&s->detadys,
                             (void **)&s->detady2, (void **)&s->dzitdz, (void **)&s->dzitdzs, (void **)&s->dzitdz2,
                             (void **)&s->ds, (void **)&s->partials, (void **)&s->dirty, (void **)&s->counters,
-                            (void **)&s->fixlist};
+                            (void **)&s->fixlist, (void **)&s->hot, (void **)&s->hot_rec,
+                            (void **)&s->hot_dirty};
     hipError_t ea = hipSuccess;
     if (mem) {
         size_t off = 0;
@@ -472,6 +515,8 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
             return fail(ST_ERR_NOMEM, std::string("device allocation failed: ") + hipGetErrorString(ea));
         }
     }
+    s->dtpart = s->partials + partial_head(g, s->mixed);
+    s->stage2 = s->dtpart + st::aux_dt_blocks(g);
     // the first points of w and w_aux sit lead_bytes into their allocations
     s->w_alloc = s->w;
     s->w_aux_alloc = s->w_aux;
@@ -609,6 +654,9 @@ int st_set_grid(st_solver *s, const double *x, const double *y, const double *z,
     s->jbl = 0;
     for (int j = 1; j <= g.ny; j++)
         if (s->p.l0 > y[j + g.ng - 1]) s->jbl = j;
+    // the metric of equal nodes agrees to their round-off
+    s->x_uniform = true;
+    for (int i = 1; i < g.nx; i++) s->x_uniform = s->x_uniform && std::fabs(dcsidx[i] / dcsidx[0] - 1.0) <= 1e-11;
     s->grid_set = true;
     return ST_OK;
 }
@@ -1139,7 +1187,7 @@ int st_rk_sync(st_solver *s) {
         if (rc) return rc;
         return rk_sync_pieces(s, s->hs->dt);
     }
-    return do_rk_sync(s);
+    return do_rk_sync(s, false);
 }
 
 int st_advance(st_solver *s, int32_t nsteps) {
@@ -1167,9 +1215,8 @@ int st_advance(st_solver *s, int32_t nsteps) {
             // therefore takes the reduction
             s->dt_in_stage = true;
         }
-        int rc = do_rk_sync(s);
+        int rc = do_rk_sync(s, true);
         if (rc) return rc;
-        TIMED(ST_K_STEP_END, st::launch_step_end(s));
     }
     return ST_OK;
 }

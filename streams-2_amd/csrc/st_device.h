@@ -1,0 +1,134 @@
+// st_device.h -- device helpers shared by the kernel files: wave and block
+// reductions, the isothermal-wall ghost of a point and the ghost images of an
+// interior value.
+#pragma once
+
+#include "st_internal.h"
+
+namespace st {
+
+constexpr int H = 3;           // stencil half width of the flux windows
+constexpr int RED_THREADS = 256;
+
+// -------------------------------------------------------------- utilities
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    return v;
+}
+__device__ __forceinline__ double wave_max(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
+    return v;
+}
+__device__ __forceinline__ double wave_min(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_down(v, off, 64));
+    return v;
+}
+
+// Block sum of NV values in a fixed order; result valid in thread 0.
+__device__ __forceinline__ int flat_block() { return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z); }
+__device__ __forceinline__ int flat_thread() { return threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z); }
+
+template <int NV>
+__device__ __forceinline__ void block_sum(double (&v)[NV], double (*lds)[NV]) {
+    const int ft = flat_thread();
+    const int lane = ft & 63;
+    const int wid = ft >> 6;
+    const int nw = (blockDim.x * blockDim.y * blockDim.z + 63) >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; q++) v[q] = wave_sum(v[q]);
+    if (lane == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; q++) lds[wid][q] = v[q];
+    }
+    __syncthreads();
+    if (ft == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; q++) {
+            double a = lds[0][q];
+            for (int w = 1; w < nw; w++) a += lds[w][q];
+            v[q] = a;
+        }
+    }
+}
+
+// bcwall_staggered_subroutine (kernels_cpu.F90:6612-6678) for one ghost
+// point: the mirror of interior point js, written at jg.
+template <typename R>
+__device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *__restrict__ w,
+                                           const R *__restrict__ wa, int i, int js, int jg, int k) {
+    const int s = gidx(g, i, js, k), d = gidx(g, i, jg, k);
+    const size_t nv = g.nvol;
+    double rho = w[s];
+    const double uu = w[nv + s] / rho;
+    const double vv = w[2 * nv + s] / rho;
+    const double ww = w[3 * nv + s] / rho;
+    const double rhoe = w[4 * nv + s];
+    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+    double ee = rhoe / rho - qq;
+    double tt = temperature_from_e(P, ee, double(wa[5 * nv + s]));
+    const double pp = rho * tt * P.rgas0;
+    tt = 2.0 * P.t_wall - tt;
+    ee = e_from_temperature(P, tt);
+    rho = pp / tt / P.rgas0;
+    w[d] = rho;
+    w[nv + d] = -rho * uu;
+    w[2 * nv + d] = -rho * vv;
+    w[3 * nv + d] = -rho * ww;
+    w[4 * nv + d] = rho * (ee + qq);
+}
+
+// exclusive prefix over the block's 256 threads of v; *total receives the sum
+__device__ __forceinline__ int block_excl_scan256(int v, int *wsum, int *total) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    int x = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d, 64);
+        if (lane >= d) x += y;
+    }
+    if (lane == 63) wsum[wv] = x;
+    __syncthreads();
+    int before = 0, tot = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        if (q < wv) before += wsum[q];
+        tot += wsum[q];
+    }
+    __syncthreads();
+    *total = tot;
+    return before + x - v;
+}
+
+// Ghost images of an interior value: periodic copy for periodic directions
+// (bcswap_var), zero-gradient copy otherwise (bcextr_var).
+template <typename R>
+__device__ __forceinline__ void write_images(const Geo &g, const KPar &P, R *__restrict__ a, int i, int j, int k,
+                                             R v, bool extrapolate) {
+    const int ng = g.ng;
+    if (P.periodic[0]) {
+        if (i <= ng) a[gidx(g, i + g.nx, j, k)] = v;
+        if (i > g.nx - ng) a[gidx(g, i - g.nx, j, k)] = v;
+    } else if (extrapolate) {
+        if (i == 1) for (int l = 1; l <= ng; l++) a[gidx(g, 1 - l, j, k)] = v;
+        if (i == g.nx) for (int l = 1; l <= ng; l++) a[gidx(g, g.nx + l, j, k)] = v;
+    }
+    if (P.periodic[1]) {
+        if (j <= ng) a[gidx(g, i, j + g.ny, k)] = v;
+        if (j > g.ny - ng) a[gidx(g, i, j - g.ny, k)] = v;
+    } else if (extrapolate) {
+        if (j == 1) for (int l = 1; l <= ng; l++) a[gidx(g, i, 1 - l, k)] = v;
+        if (j == g.ny) for (int l = 1; l <= ng; l++) a[gidx(g, i, g.ny + l, k)] = v;
+    }
+    if (P.periodic[2] && P.ndim == 3) {
+        if (k <= ng) a[gidx(g, i, j, k + g.nz)] = v;
+        if (k > g.nz - ng) a[gidx(g, i, j, k - g.nz)] = v;
+    } else if (extrapolate) {
+        if (k == 1) for (int l = 1; l <= ng; l++) a[gidx(g, i, j, 1 - l)] = v;
+        if (k == g.nz) for (int l = 1; l <= ng; l++) a[gidx(g, i, j, g.nz + l)] = v;
+    }
+}
+
+}  // namespace st

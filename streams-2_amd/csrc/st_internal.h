@@ -107,6 +107,7 @@ struct DevScalars {
     unsigned long long dtinv_bits;   // running max of the CFL spectral radii
     long long icyc;
     double cnt[3];                   // WENO face counts
+    double rhs_sum[2];               // bulk sums of the last stage's right-hand side 1:2 (one-pass stage)
 };
 
 // ------------------------------------------------------------- EOS helpers

@@ -1,6 +1,7 @@
 // st_kernels.hip -- gfx950 kernels of one RK stage and their launchers.
 //
-// Stage pipeline of the fused path (st_rk_sync), one kernel per line:
+// Stage pipeline of the separate sweeps (st_rk_sync for the solves that the
+// one-pass stage of st_stage.hip does not cover), one kernel per line:
 //   aux        w -> w_aux(1:7) over the ghosted box, periodic ghosts read
 //              from their images (replaces bcswap + compute_aux)
 //   euler_x    x faces + divergence, writes F[cur] (replaces init_flux's
@@ -17,57 +18,11 @@
 // Reductions use per-block partials summed in a fixed order, so a run is
 // bitwise reproducible; the CFL maximum uses an atomic max on the bit
 // pattern of non-negative doubles, which is order independent.
+#include "st_device.h"
 #include "st_flux.h"
 #include "st_solver.h"
 
 namespace st {
-
-constexpr int H = 3;           // stencil half width of the flux windows
-constexpr int RED_THREADS = 256;
-
-// -------------------------------------------------------------- utilities
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
-}
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
-    return v;
-}
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_down(v, off, 64));
-    return v;
-}
-
-// Block sum of NV values in a fixed order; result valid in thread 0.
-__device__ __forceinline__ int flat_block() { return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z); }
-__device__ __forceinline__ int flat_thread() { return threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z); }
-
-template <int NV>
-__device__ __forceinline__ void block_sum(double (&v)[NV], double (*lds)[NV]) {
-    const int ft = flat_thread();
-    const int lane = ft & 63;
-    const int wid = ft >> 6;
-    const int nw = (blockDim.x * blockDim.y * blockDim.z + 63) >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; q++) v[q] = wave_sum(v[q]);
-    if (lane == 0) {
-#pragma unroll
-        for (int q = 0; q < NV; q++) lds[wid][q] = v[q];
-    }
-    __syncthreads();
-    if (ft == 0) {
-#pragma unroll
-        for (int q = 0; q < NV; q++) {
-            double a = lds[0][q];
-            for (int w = 1; w < nw; w++) a += lds[w][q];
-            v[q] = a;
-        }
-    }
-}
 
 // ------------------------------------------------------------ ghost fills
 // Periodic copy of bcswap (base_cpu.F90:410-450, 669-745 with the local
@@ -137,32 +92,6 @@ __global__ void k_extrapolate_var(Geo g, T *__restrict__ a) {
         }
         a[dst] = a[src];
     }
-}
-
-// bcwall_staggered_subroutine (kernels_cpu.F90:6612-6678) for one ghost
-// point: the mirror of interior point js, written at jg.
-template <typename R>
-__device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *__restrict__ w,
-                                           const R *__restrict__ wa, int i, int js, int jg, int k) {
-    const int s = gidx(g, i, js, k), d = gidx(g, i, jg, k);
-    const size_t nv = g.nvol;
-    double rho = w[s];
-    const double uu = w[nv + s] / rho;
-    const double vv = w[2 * nv + s] / rho;
-    const double ww = w[3 * nv + s] / rho;
-    const double rhoe = w[4 * nv + s];
-    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-    double ee = rhoe / rho - qq;
-    double tt = temperature_from_e(P, ee, double(wa[5 * nv + s]));
-    const double pp = rho * tt * P.rgas0;
-    tt = 2.0 * P.t_wall - tt;
-    ee = e_from_temperature(P, tt);
-    rho = pp / tt / P.rgas0;
-    w[d] = rho;
-    w[nv + d] = -rho * uu;
-    w[2 * nv + d] = -rho * vv;
-    w[3 * nv + d] = -rho * ww;
-    w[4 * nv + d] = rho * (ee + qq);
 }
 
 template <typename R>
@@ -1758,28 +1687,6 @@ __device__ __forceinline__ unsigned dirty_bytes(unsigned long long wd, int bit, 
     return mine;
 }
 
-// exclusive prefix over the block's 256 threads of v; *total receives the sum
-__device__ __forceinline__ int block_excl_scan256(int v, int *wsum, int *total) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d, 64);
-        if (lane >= d) x += y;
-    }
-    if (lane == 63) wsum[wv] = x;
-    __syncthreads();
-    int before = 0, tot = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        if (q < wv) before += wsum[q];
-        tot += wsum[q];
-    }
-    __syncthreads();
-    *total = tot;
-    return before + x - v;
-}
-
 __device__ __forceinline__ void k_fix_compact_body(const dim3 blockIdx, const dim3 gridDim, unsigned char *__restrict__ flags, int ncell, int bit,
                                                      int anyidx, int wpb, int *__restrict__ list,
                                                      int *__restrict__ counts) {
@@ -1907,35 +1814,6 @@ __global__ __launch_bounds__(256) void k_fix_list(Geo g, KPar P, const R *__rest
 }
 
 // ---------------------------------------------------------------- viscous
-// Ghost images of an interior value: periodic copy for periodic directions
-// (bcswap_var), zero-gradient copy otherwise (bcextr_var).
-template <typename R>
-__device__ __forceinline__ void write_images(const Geo &g, const KPar &P, R *__restrict__ a, int i, int j, int k,
-                                             R v, bool extrapolate) {
-    const int ng = g.ng;
-    if (P.periodic[0]) {
-        if (i <= ng) a[gidx(g, i + g.nx, j, k)] = v;
-        if (i > g.nx - ng) a[gidx(g, i - g.nx, j, k)] = v;
-    } else if (extrapolate) {
-        if (i == 1) for (int l = 1; l <= ng; l++) a[gidx(g, 1 - l, j, k)] = v;
-        if (i == g.nx) for (int l = 1; l <= ng; l++) a[gidx(g, g.nx + l, j, k)] = v;
-    }
-    if (P.periodic[1]) {
-        if (j <= ng) a[gidx(g, i, j + g.ny, k)] = v;
-        if (j > g.ny - ng) a[gidx(g, i, j - g.ny, k)] = v;
-    } else if (extrapolate) {
-        if (j == 1) for (int l = 1; l <= ng; l++) a[gidx(g, i, 1 - l, k)] = v;
-        if (j == g.ny) for (int l = 1; l <= ng; l++) a[gidx(g, i, g.ny + l, k)] = v;
-    }
-    if (P.periodic[2] && P.ndim == 3) {
-        if (k <= ng) a[gidx(g, i, j, k + g.nz)] = v;
-        if (k > g.nz - ng) a[gidx(g, i, j, k - g.nz)] = v;
-    } else if (extrapolate) {
-        if (k == 1) for (int l = 1; l <= ng; l++) a[gidx(g, i, j, 1 - l)] = v;
-        if (k == g.nz) for (int l = 1; l <= ng; l++) a[gidx(g, i, j, g.nz + l)] = v;
-    }
-}
-
 // Point values of the viscous stencils: u, v, w, T, mu (w_aux 2, 3, 4, 6, 7).
 template <typename R>
 struct VP {
@@ -3442,7 +3320,11 @@ hipError_t launch_extrapolate_aux(st_solver *s, int var) {
     return hipGetLastError();
 }
 
-hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image, bool dt) {
+int aux_dt_blocks(const Geo &g) { return (int)((aux_lanes(g) + 255) / 256); }
+int update_blocks(const Geo &g) { return cell_blocks(g); }
+
+hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image, bool dt,
+                      bool defer_dt) {
     const int ni = i1 - i0 + 1, nj = j1 - j0 + 1, nk = k1 - k0 + 1;
     if (ni <= 0 || nj <= 0 || nk <= 0) return hipSuccess;
     const size_t tot = aux_whole_box(s->g, i0, ni, j0, nj, k0, nk) ? aux_lanes(s->g)
@@ -3451,12 +3333,12 @@ hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int 
 #define ST_LAUNCH_AUX(D_)                                                                                          \
     ST_DISPATCH(ST_GO(k_aux, ST_T(R, D_), 256, 0, dim3(nblk), dim3(256), s->g, s->kp, s->w, (R *)s->w_aux, i0, ni,  \
                       j0, nj, k0, nk, image ? 1 : 0, s->dcsidx, s->detady, s->dzitdz, s->dcsidxs, s->detadys,        \
-                      s->dzitdzs, s->partials))
+                      s->dzitdzs, defer_dt ? s->dtpart : s->partials))
     if (dt && s->p.cfl > 0) ST_LAUNCH_AUX(true);
     else ST_LAUNCH_AUX(false);
 #undef ST_LAUNCH_AUX
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !(dt && s->p.cfl > 0)) return e;
+    if (e != hipSuccess || !(dt && s->p.cfl > 0) || defer_dt) return e;
     ST_GO(k_dt_finish, , RED_THREADS, 0, dim3(red_blocks(nblk)), dim3(RED_THREADS), s->kp, s->partials, (int)nblk,
           s->partials + s->npart - RB * 8, s->counters + 1, &s->ds->dt);
     return hipGetLastError();
@@ -3844,11 +3726,11 @@ hipError_t launch_bc_nr(st_solver *s, void *fl) {
     return hipSuccess;
 }
 
-hipError_t launch_force_var(st_solver *s) {
+hipError_t launch_force_var(st_solver *s, int nblk) {
     ST_NOREC();
     const Geo &g = s->g;
-    hipLaunchKernelGGL(k_force_var_finish, dim3(red_blocks(cell_blocks(g))), dim3(RED_THREADS), 0, s->stream, s->kp,
-                       s->partials, cell_blocks(g), s->partials + s->npart - RB * 8, s->counters + 1, s->ds);
+    hipLaunchKernelGGL(k_force_var_finish, dim3(red_blocks(nblk)), dim3(RED_THREADS), 0, s->stream, s->kp,
+                       s->partials, nblk, s->partials + s->npart - RB * 8, s->counters + 1, s->ds);
     ST_DISPATCH(hipLaunchKernelGGL(k_force_var2<R>, cell_grid(g), kCellBlock, 0, s->stream, g, s->kp, s->w,
                                    (const R *)s->w_aux, s->ds));
     return launch_wall_ghosts(s);

@@ -46,6 +46,7 @@ struct st_solver {
     bool dt_in_stage;   // the CFL reduction of this step rides on the first stage's aux
     int visc_chunk;     // planes per tile of the z-marching viscous kernel (0: automatic)
     int march_chunk;    // points per thread of the y/z flux marches (0: automatic)
+    bool x_uniform;     // dcsidx is one value (set by st_set_grid)
     bool fuse_xy;       // x and y Euler fluxes in one pass
     bool fuse_zv;       // viscous divergence terms folded into the z march (Laplacian form)
     int force_nblk;     // force_rhs partials written in this stage (visc_div blocks, or z march + fix-up)
@@ -62,6 +63,11 @@ struct st_solver {
     int npart;           // capacity in doubles
     unsigned char *dirty;  // per-cell flag: a WENO face on either side (one sweep at a time)
     int *counters;         // [1] reduction ticket, [8 ..] segment counts of the WENO fix-up's lists
+    uint64_t *hot;         // sensor above the threshold, one bit per ghosted point (st_stage.hip)
+    uint64_t *hot_rec;     // lower/upper WENO face bits per cell and direction, 64 cells a record
+    uint3 *hot_dirty;      // cells with a WENO face, 32 cells an entry, one word a direction
+    double *dtpart;        // CFL block maxima of the aux pass of the one-pass stage (inside partials)
+    double *stage2;        // second-level values of k_weno_items (inside partials)
     int *fixlist;          // cells of one direction's WENO fix-up, in segments (nint entries)
     int cur;             // F[cur] is the right-hand side being built
     double rhork[3], gamrk[3];
@@ -158,8 +164,11 @@ constexpr int kDtStage2 = 128;
 hipError_t launch_fill_periodic(st_solver *s, double *arr, int nv);
 hipError_t launch_fill_periodic_aux(st_solver *s, int var);
 hipError_t launch_extrapolate_aux(st_solver *s, int var);
+// dt also takes the CFL reduction: its block maxima to dt itself, or with
+// defer_dt to dtpart, for launch_weno_items to finish
 hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image,
-                      bool dt = false);
+                      bool dt = false, bool defer_dt = false);
+int aux_dt_blocks(const Geo &g);  // block maxima of an aux pass over the ghosted box
 hipError_t launch_wall_ghosts(st_solver *s);
 // physical ghosts of every non-periodic face in the order xmin..zmax
 // (update_ghost without the periodic swap)
@@ -201,7 +210,25 @@ hipError_t launch_sensor(st_solver *s, bool ghost_images);
 hipError_t launch_visc_div(st_solver *s, void *fl, const void *fl_prev, int stage, bool reduce, bool ord2);
 hipError_t launch_force_finish(st_solver *s, int stage);
 hipError_t launch_update(st_solver *s, const void *fl_prev, const void *fl, int stage);
-hipError_t launch_force_var(st_solver *s);
+// nblk block sums of rho*u*T*dy from the update
+hipError_t launch_force_var(st_solver *s, int nblk);
+int update_blocks(const Geo &g);
+// ---- one-pass stage (st_stage.hip)
+bool one_pass_stage(const st_solver *s);
+size_t hot_bits_bytes(const Geo &g);
+size_t hot_rec_bytes(const Geo &g);
+size_t hot_dirty_bytes(const Geo &g);
+int one_pass_flux_slots(const Geo &g, bool mixed);
+int one_pass_update_blocks(const Geo &g);
+constexpr int kStage2Slots = 256 * 6;  // second-level values of k_weno_items
+// the step's WENO masks and work items from w_aux(8)
+hipError_t launch_hot_items(st_solver *s);
+// the whole right-hand side but grad(div/3) and the WENO faces
+hipError_t launch_flux(st_solver *s, void *fl, int stage);
+// WENO faces; bulk sums of force_rhs and, with dt, the CFL step finished
+hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt);
+// grad(div/3), update_flux, update_field, wall ghosts; the end of the step
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end);
 hipError_t launch_dt(st_solver *s);
 hipError_t launch_step_end(st_solver *s);
 hipError_t launch_residual(st_solver *s);

@@ -1,0 +1,1430 @@
+// st_stage.hip -- the one-pass stage: the kernels st_rk_sync / st_advance run
+// for the KEEP split (nkeep = 0) of a calorically perfect gas with the Roe
+// WENO split, three ghost layers and a periodic span (one_pass_stage below);
+// every other solve runs the separate sweeps of st_kernels.hip.
+//
+// One stage is
+//   aux      w -> w_aux(1:7) over the ghosted box (st_kernels.hip)
+//   flux     x, y and z central fluxes and the viscous terms of every cell in
+//            one march along z, the bulk sums of force_rhs, and at the third
+//            stage the Ducros sensor
+//   items    WENO faces of the flagged cells; the last workgroup finishes the
+//            bulk sums (dpdx) and, at the first stage, the CFL step
+//   update   grad(div/3) terms, w += fln with the forcing, wall ghosts
+// and at the first stage of a step two kernels turn the sensor into bit masks
+// and into the list of WENO work items, which the three stages share (the
+// reference switches on the sensor of the previous step's last stage).
+#include "st_device.h"
+#include "st_flux.h"
+#include "st_solver.h"
+
+namespace st {
+
+// ============================================================ sensor masks
+// Bit masks of the switch: the sensor of the ghosted box as one bit per point
+// (k_hot_bits), then per interior cell and direction whether its lower and
+// its upper face are WENO faces.  A face i of direction d takes the WENO flux
+// when a point i-ws+1 .. i+ws along d is above the threshold (the switch
+// window of the reference kernels, kernels_cpu.F90:466-470).
+//
+// Layouts: hot bits, ceil(rx/64) words per ghosted row, bit e of a row the
+// point i = e + 1 - ng.  Cell records, one per 64 cells of an interior row
+// (row-major over j, k): words 2d and 2d+1 hold the lower-face and
+// upper-face bits of direction d (words 6, 7 unused: a record is one 64-byte
+// sector).
+constexpr int kRecWords = 8;
+constexpr int kItemSeg = 4096;       // list segments at most
+constexpr int kItemBlocks = 256;     // workgroups of the item kernel at most (one per CU)
+
+__host__ __device__ __forceinline__ int hot_words(const Geo &g) { return (g.rx + 63) / 64; }
+__host__ __device__ __forceinline__ int rec_per_row(const Geo &g) { return (g.nx + 63) / 64; }
+
+// the cells with a WENO face, 32 cells of a row per entry, one word a direction
+__host__ __device__ __forceinline__ int dirty_per_row(const Geo &g) { return (g.nx + 31) / 32; }
+
+size_t hot_dirty_bytes(const Geo &g) { return sizeof(uint3) * (size_t)dirty_per_row(g) * g.ny * g.nz; }
+size_t hot_bits_bytes(const Geo &g) { return sizeof(uint64_t) * (size_t)hot_words(g) * g.sy * g.sz; }
+size_t hot_rec_bytes(const Geo &g) { return sizeof(uint64_t) * kRecWords * (size_t)rec_per_row(g) * g.ny * g.nz; }
+
+// One wave per word, bound by the read of the sensor (8 B a point).
+template <typename R>
+__device__ __forceinline__ void k_hot_bits_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
+                                                const R *__restrict__ wa, uint64_t *__restrict__ hot) {
+    const int lane = threadIdx.x & 63;
+    const int nwg = hot_words(g);
+    const int tot = nwg * g.sy * g.sz;
+    const R thr = R(P.sensor_threshold);
+    const R *S = wa + 7 * (size_t)g.nvol;
+    // four consecutive words a wave: their loads are in flight together
+    const int w0 = 4 * (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    R v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int wd = w0 + q;
+        const int row = wd / nwg, e = 64 * (wd - row * nwg) + lane;
+        v[q] = wd < tot && e < g.rx ? S[(size_t)row * g.sx + e] : thr;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const unsigned long long m = __ballot(v[q] > thr);
+        if (lane == 0 && w0 + q < tot) hot[w0 + q] = m;
+    }
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_hot_bits(Geo g, KPar P, const R *__restrict__ wa,
+                                                  uint64_t *__restrict__ hot) {
+    k_hot_bits_body<R>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, wa, hot);
+}
+
+// Record of 64 cells per thread (all directions by word operations), then the
+// work items of the block's segment of `256 * wpt` records, in cell order, x
+// before y before z of one cell.  An item is one flagged cell and direction:
+//   bits 0-23 cell, relative to the segment's first cell; 24-25 direction;
+//   26 lower face WENO; 27 upper face WENO.
+// The list of a segment starts at its first cell's index, so it has room for
+// one item per cell; a segment with more writes none and reports -3 * cells:
+// its items are then all (cell, direction) pairs, read from the records.
+__device__ __forceinline__ int seg_first_cell(const Geo &g, int nwx, int wd, int nwords) {
+    return wd >= nwords ? (int)g.nint : (wd / nwx) * g.nx + 64 * (wd % nwx);
+}
+
+__device__ __forceinline__ void k_hot_items_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
+                                                 const uint64_t *__restrict__ hot, uint64_t *__restrict__ rec,
+                                                 uint3 *__restrict__ dirty, int wpt, int *__restrict__ list, int *__restrict__ counts) {
+    __shared__ int wsum[4];
+    const int nwx = rec_per_row(g), nwg = hot_words(g);
+    const int nwords = nwx * g.ny * g.nz;
+    const int segw = 256 * wpt;
+    const int W0 = blockIdx.x * segw;
+    const int S0 = seg_first_cell(g, nwx, W0, nwords), S1 = seg_first_cell(g, nwx, W0 + segw, nwords);
+    const int ws = P.weno_scheme;
+    const int wa0 = W0 + (int)threadIdx.x * wpt, wa1 = min(wa0 + wpt, nwords);
+    int c = 0;
+    for (int wd = wa0; wd < wa1; wd++) {
+        const int q = wd % nwx, r = wd / nwx;
+        const int j = r % g.ny + 1, k = r / g.ny + 1;
+        // bits of the points 64q+1-3+s .. of ghosted row (j, k)
+        auto row = [&](int jj, int kk, int s) {
+            const size_t b = ((size_t)(kk + g.ng - 1) * g.sy + (jj + g.ng - 1)) * nwg + q;
+            const uint64_t lo = hot[b], hi = q + 1 < nwg ? hot[b + 1] : 0ull;
+            return s == 0 ? lo : (lo >> s) | (hi << (64 - s));
+        };
+        const int nc = g.nx - 64 * q;
+        const uint64_t in = nc >= 64 ? ~0ull : (1ull << nc) - 1ull;
+        uint64_t lh[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int o = -3; o <= 3; o++) {
+            const bool lower = o >= -ws && o <= ws - 1, upper = o >= -ws + 1 && o <= ws;
+            if (!lower && !upper) continue;
+            const uint64_t x = row(j, k, 3 + o), y = row(j + o, k, 3), z = row(j, k + o, 3);
+            if (lower) { lh[0] |= x; lh[2] |= y; lh[4] |= z; }
+            if (upper) { lh[1] |= x; lh[3] |= y; lh[5] |= z; }
+        }
+        // cells outside the Euler range of a direction get no flux there
+        uint64_t rx = in;
+        for (int d = 0; d < 2; d++) {
+            const int f = d == 0 ? P.eul_lo[0] - 1 - 64 * q : P.eul_hi[0] - 64 * q;  // cells below / up to f
+            const uint64_t below = f <= 0 ? 0ull : (f >= 64 ? ~0ull : (1ull << f) - 1ull);
+            rx &= d == 0 ? ~below : below;
+        }
+        const uint64_t msk[3] = {rx, j >= P.eul_lo[1] && j <= P.eul_hi[1] ? in : 0ull,
+                                 k >= P.eul_lo[2] && k <= P.eul_hi[2] ? in : 0ull};
+        uint64_t *o = rec + (size_t)kRecWords * wd;
+        uint64_t dd[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const uint64_t a = lh[2 * d] & msk[d], b = lh[2 * d + 1] & msk[d];
+            o[2 * d] = a;
+            o[2 * d + 1] = b;
+            dd[d] = a | b;
+            c += __popcll(dd[d]);
+        }
+        uint3 *dr = dirty + (size_t)r * dirty_per_row(g) + 2 * q;
+        dr[0] = make_uint3((unsigned)dd[0], (unsigned)dd[1], (unsigned)dd[2]);
+        if (nc > 32) dr[1] = make_uint3((unsigned)(dd[0] >> 32), (unsigned)(dd[1] >> 32), (unsigned)(dd[2] >> 32));
+    }
+    int total;
+    int off = block_excl_scan256(c, wsum, &total);
+    const bool dense = total > S1 - S0;
+    if (threadIdx.x == 0) counts[blockIdx.x] = dense ? -3 * (S1 - S0) : total;
+    if (c == 0 || dense) return;
+    int *seg = list + S0;
+    for (int wd = wa0; wd < wa1; wd++) {
+        const uint64_t *o = rec + (size_t)kRecWords * wd;
+        uint64_t lh[6], any = 0;
+#pragma unroll
+        for (int d = 0; d < 6; d++) {
+            lh[d] = o[d];
+            any |= lh[d];
+        }
+        const int cell0 = seg_first_cell(g, nwx, wd, nwords) - S0;
+        while (any) {
+            const int b = __ffsll((unsigned long long)any) - 1;
+            any &= any - 1ull;
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const int lo = (int)(lh[2 * d] >> b) & 1, hi = (int)(lh[2 * d + 1] >> b) & 1;
+                if (lo | hi) seg[off++] = (cell0 + b) | d << 24 | lo << 26 | hi << 27;
+            }
+        }
+    }
+}
+__global__ __launch_bounds__(256) void k_hot_items(Geo g, KPar P, const uint64_t *__restrict__ hot,
+                                                   uint64_t *__restrict__ rec, uint3 *__restrict__ dirty, int wpt, int *__restrict__ list,
+                                                   int *__restrict__ counts) {
+    k_hot_items_body(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, hot, rec, dirty, wpt, list, counts);
+}
+
+// ============================================================ one-pass fluxes
+// A value the optimizer cannot see through: address arithmetic of the rare
+// branches (edges, ghost images) built on it stays inside them instead of
+// being hoisted out of the march, where it would hold registers.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A point's stencil values: rho, u, v, w, T, mu, and in the mixed form the
+// stored deviation p - p_ref (in FP64 the pressure is rho*T*R).
+constexpr int VR = 0, VU = 1, VT = 4, VM = 5, VP_ = 6;
+template <typename R>
+constexpr int kNP = sizeof(R) == sizeof(double) ? 6 : 7;
+template <typename R>
+struct SP {
+    R a[kNP<R>];
+};
+// p/R in FP64, p - p_ref in the mixed form
+template <typename R>
+__device__ __forceinline__ R sp_press(const SP<R> &p) {
+    if constexpr (sizeof(R) == sizeof(double)) return p.a[VR] * p.a[VT];
+    else return p.a[VP_];
+}
+
+// What the three directions add up for one cell.  Every term of the right-hand
+// side has the form f_k = (u_k m + mk[k]) / 4 for the momenta (the pressure
+// and mu Laplacian terms ride in mk) and the energy takes u_k mk[k] / 4 of the
+// same sums, so five accumulators serve the convective, pressure, diffusion
+// and conduction terms of all directions.
+template <typename R>
+struct CellAcc {
+    R m, mk[3];  // sums of U = c (un_i + un_j)(rho_i + rho_j) and of U u_j, metric included; + 4 grad p - 4 mu lap u
+    R e;         // energy terms that are no u_k mk[k] / 4: U e_j / 4, p div u, conduction
+};
+
+// Velocity and viscosity derivatives along one direction.
+template <typename R>
+struct Grad {
+    R u[3], m;
+};
+
+// Uniform values of the flux arithmetic.
+template <typename R>
+struct FluxConst {
+    R c[H], c2[H + 1];  // first- and second-derivative weights (the viscous terms; Euler along z)
+    R rg, pref;         // pressure = rg * sp_press + pref
+    R ea, eb;           // internal energy = ea + eb T
+    R cpr;              // cp / Pr
+};
+
+// The central flux difference of the cell along direction D, and its viscous
+// derivatives.  The flux of the reference (kernels_cpu.F90:466-618, 1109-1257,
+// 1854-2004) at a face is a sum of pair terms G_l(a, b) over the pairs that
+// straddle it with b - a = l.  Between two faces of equal stencil order the
+// sums telescope: the difference is sum_l c_l (G_l(i, i+l) - G_l(i-l, i)), six
+// pairs that all hold the cell's own point i.  What depends on point i alone
+// then factors out of the sums (e.g. sum U (u_i + u_j) = u_i sum U + sum U u_j),
+// the pressure and velocity parts of the energy flux become the p and u_d
+// derivatives, and the internal energy, affine in T, needs only sum U T_j.
+// That is ~11 operations a pair and no face values to carry between cells or
+// lanes; the face form with its register march and lane moves issued ~2.5x
+// the instructions.  am is the metric of the Euler term (0: direction not
+// taken here), w the first-derivative weights of its stencil order (per lane
+// along x and y, see edge_cell), a1, s1, q1 the viscous metrics, pr the cell's
+// pressure.
+// The neighbours of a direction in the order +1, -1, +2, -2, +3, -3, each
+// read from LDS (D < 2) one step ahead of its use; a scheduler free to start
+// every read of a direction at once would hold 72 registers of them.
+template <typename R, int D, typename Get, typename Use>
+__device__ __forceinline__ void each_neighbour(const Get &at, const Use &use) {
+    SP<R> nb[2];
+    nb[0] = at(1);
+#pragma unroll
+    for (int q = 0; q < 2 * H; q++) {
+        if (q + 1 < 2 * H) nb[(q + 1) & 1] = at(q & 1 ? (q + 3) / 2 : -(q + 2) / 2);
+        if (D != 2) __builtin_amdgcn_sched_barrier(0);
+        use(nb[q & 1], q / 2, (q & 1) != 0);
+        if (D != 2) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <typename R, int D, typename Get>
+__device__ __forceinline__ R flux_dir(const FluxConst<R> &K, const SP<R> &o, const Get &at, const R (&w)[H], R pr, R am,
+                                      R a1, R s1, R q1, CellAcc<R> &A, Grad<R> &G) {
+    R m = R(0), mu_ = R(0), mv = R(0), mw = R(0), mt = R(0), ps = R(0);
+    R gu = R(0), gv = R(0), gw = R(0), gt = R(0), gm = R(0), gn = R(0);
+    R lu = K.c2[0] * o.a[VU], lv = K.c2[0] * o.a[VU + 1], lw = K.c2[0] * o.a[VU + 2], lt = K.c2[0] * o.a[VT];
+    each_neighbour<R, D>(at, [&](const SP<R> &p, int l, bool neg) {
+        const R c = neg ? -K.c[l] : K.c[l], c2 = K.c2[l + 1], cw = neg ? -w[l] : w[l];
+        const R U = (cw * (o.a[VU + D] + p.a[VU + D])) * (o.a[VR] + p.a[VR]);
+        m += U;
+        mu_ += U * p.a[VU];
+        mv += U * p.a[VU + 1];
+        mw += U * p.a[VU + 2];
+        mt += U * p.a[VT];
+        ps += cw * sp_press(p);
+        if (D != 2) gn += cw * p.a[VU + D];
+        gu += c * p.a[VU];
+        gv += c * p.a[VU + 1];
+        gw += c * p.a[VU + 2];
+        gt += c * p.a[VT];
+        gm += c * p.a[VM];
+        lu += c2 * p.a[VU];
+        lv += c2 * p.a[VU + 1];
+        lw += c2 * p.a[VU + 2];
+        lt += c2 * p.a[VT];
+    });
+    const R mu4 = R(-4) * o.a[VM];
+    (D == 0 ? mu_ : (D == 1 ? mv : mw)) += (R(4) * K.rg) * ps;
+    A.e += am * (R(0.25) * K.eb * mt + pr * (D == 2 ? gw : gn));
+    gu *= a1; gv *= a1; gw *= a1; gt *= a1; gm *= a1;
+    A.m += am * m;
+    A.mk[0] += am * mu_ + mu4 * (lu * s1 + gu * q1);
+    A.mk[1] += am * mv + mu4 * (lv * s1 + gv * q1);
+    A.mk[2] += am * mw + mu4 * (lw * s1 + gw * q1);
+    A.e -= K.cpr * (gm * gt + o.a[VM] * (lt * s1 + gt * q1));
+    G.u[0] = gu; G.u[1] = gv; G.u[2] = gw;
+    G.m = gm;
+    return gt;
+}
+
+// The same with the viscous terms of the second-order conservative form
+// (visflx_reduced_ord2 and visflx_x/y/z, kernels_cpu.F90:4623-4721, 4779-4999):
+// hc = 1/(x_{i+1} - x_{i-1}), hm = 1/(x_i - x_{i-1}), hp = 1/(x_{i+1} - x_i).
+// The face fluxes mu du/dx of the momenta go to mk, their kinetic part
+// mu d(|u|^2/2)/dx to e less the u_k mk[k] / 4 that the sums already carry:
+// (|u_p|^2 - |u_o|^2)/2 - u_o.(u_p - u_o) = |u_p - u_o|^2 / 2.
+template <typename R, int D, typename Get>
+__device__ __forceinline__ R flux_dir_cons(const FluxConst<R> &K, const SP<R> &o, const Get &at, const R (&w)[H], R pr, R am,
+                                           R hc, R hm, R hp, CellAcc<R> &A, Grad<R> &G) {
+    R m = R(0), mu_ = R(0), mv = R(0), mw = R(0), mt = R(0), ps = R(0), gn = R(0), gt = R(0);
+    G.u[0] = G.u[1] = G.u[2] = G.m = R(0);
+    each_neighbour<R, D>(at, [&](const SP<R> &p, int l, bool neg) {
+        const R c = neg ? -w[l] : w[l];
+        const R U = (c * (o.a[VU + D] + p.a[VU + D])) * (o.a[VR] + p.a[VR]);
+        m += U;
+        mu_ += U * p.a[VU];
+        mv += U * p.a[VU + 1];
+        mw += U * p.a[VU + 2];
+        mt += U * p.a[VT];
+        ps += c * sp_press(p);
+        gn += c * p.a[VU + D];
+        if (l == 0) {
+            const R h = neg ? -hc : hc;
+            const R f = (o.a[VM] + p.a[VM]) * ((neg ? hm : hp) * hc);
+            G.m += h * p.a[VM];
+            gt += h * p.a[VT];
+            R k2 = R(0);
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                const R d = p.a[VU + x] - o.a[VU + x];
+                G.u[x] += h * p.a[VU + x];
+                A.mk[x] -= R(4) * f * d;
+                k2 += d * d;
+            }
+            A.e -= f * ((p.a[VT] - o.a[VT]) * K.cpr + R(0.5) * k2);
+        }
+    });
+    (D == 0 ? mu_ : (D == 1 ? mv : mw)) += (R(4) * K.rg) * ps;
+    A.e += am * (R(0.25) * K.eb * mt + pr * gn);
+    A.m += am * m;
+    A.mk[0] += am * mu_;
+    A.mk[1] += am * mv;
+    A.mk[2] += am * mw;
+    return gt;
+}
+
+// Beside a non-periodic boundary the two faces of a cell can have different
+// half widths, or one is a zero-flux wall face.  flux_dir then works with the
+// weights d_l of the wider face, and this adds the difference at the other
+// one: sum_l (d_l - c_l) S_l, S_l the pairs that straddle it (zero flux: c_l
+// = 0, but the pressure part stays).  side is -1 (lower face) or +1; points
+// are taken at side * offset, so that both sides run the same code.  Only the
+// point pairs in flight are held in registers.
+template <typename R>
+struct EdgeW {
+    R e[H], p[H];  // d_l - c_l, for the convective and the pressure part
+};
+template <typename R, int D, typename Get>
+__device__ __forceinline__ void edge_cell(const Get &at, const SP<R> &o, unsigned edge, const R (*cd)[H],
+                                          const FluxConst<R> &K, R am, R f[5]) {
+    const int lo = (int)(edge & 15u), hi = (int)(edge >> 4) & 15;
+    const bool upper = (edge >> 9) & 1u || lo > hi;
+    const bool zero = upper ? (edge >> 9) & 1u : (edge >> 8) & 1u;
+    const int side = upper ? 1 : -1, small = upper ? hi : lo, big = max(lo, hi);
+    EdgeW<R> W;
+    am = upper ? -am : am;
+#pragma unroll
+    for (int l = 0; l < H; l++) {
+        const R d = am * cd[big - 1][l], c = am * cd[small - 1][l];
+        W.e[l] = d - (zero ? R(0) : c);
+        W.p[l] = d - c;
+    }
+    auto pair = [&](const SP<R> &A, const SP<R> &B, int l) {
+        const R una = A.a[VU + D], unb = B.a[VU + D];
+        const R pA = sp_press(A) * K.rg, pB = sp_press(B) * K.rg;
+        const R uv = R(0.25) * W.e[l - 1] * (una + unb) * (A.a[VR] + B.a[VR]);
+        f[0] += R(2) * uv;
+#pragma unroll
+        for (int x = 0; x < 3; x++) f[1 + x] += uv * (A.a[VU + x] + B.a[VU + x]);
+        f[1 + D] += W.p[l - 1] * (pA + pB);
+        f[4] += uv * (R(2) * K.ea + K.eb * (A.a[VT] + B.a[VT]) + A.a[VU] * B.a[VU] + A.a[VU + 1] * B.a[VU + 1] +
+                      A.a[VU + 2] * B.a[VU + 2]) +
+                W.e[l - 1] * (una * (pB + K.pref) + unb * (pA + K.pref));
+    };
+    {
+        const SP<R> m1 = at(side);
+        pair(m1, o, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        pair(m1, at(-side), 2);
+        __builtin_amdgcn_sched_barrier(0);
+        pair(m1, at(-2 * side), 3);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    {
+        const SP<R> m2 = at(2 * side);
+        pair(m2, o, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        pair(m2, at(-side), 3);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    pair(at(3 * side), o, 3);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <typename R>
+constexpr int kFluxWaves = sizeof(R) == sizeof(double) ? 2 : 3;
+
+constexpr int kFluxMaxChunk = 32;
+
+struct FluxArgs {
+    const double *dx1, *dxs, *dx2, *dy1, *dys, *dy2, *dz1, *dzs, *dz2;  // metrics
+    const double *xc, *yc, *zc, *yn;                                    // node coordinates, y faces
+    const int *eocx, *eocy;
+    const uint3 *dirty;   // cells with a WENO face (k_hot_items)
+    const double *w;
+    double *wallprop;
+    double *partials;     // 5 block sums of force_rhs (SUMS)
+    int chunk;
+    int last;             // third stage: |omega| and the sensor are written
+};
+
+// One workgroup marches a TX x TY column tile along z over `chunk` planes:
+// each lane keeps its 7-plane z stencil in registers, the x and y stencils
+// come from an LDS copy of the current plane with a 3-point halo (two
+// buffers, one barrier a plane).  All three directions read the same six
+// values of a point, so w_aux is read once a stage and the right-hand side is
+// written once; the separate passes (x + y sweep, viscous march, z march)
+// moved 96 + 120 + 152 B a cell, this one 48 + 48.  Two waves per SIMD: the z
+// window, the look-ahead and the accumulators fill 256 registers, so what a
+// lane can re-read (offsets, metrics, running sums) stays in LDS; a spilled
+// look-ahead load (waited for at once to be stored) cost 2x.
+// Bound by FP64 issue: ~830 vector instructions a wave and plane, 4.4 cycles
+// each at the ~2.0 GHz of a loaded chip (59 TFLOP/s of FMAs measured), 77 % of
+// the kernel's time.  512 x 256 x 256, with the bulk sums: 1.29 ms, where the
+// passes it replaces took 0.85 + 0.99 + 1.37; 128 x 96 x 64: 49 us for 38 + 35
+// + 41.  Mixed, 256 x 192 x 128: 189 us for 124 + 115 + 175.
+template <typename T>
+__device__ __forceinline__ T at_off(const T *__restrict__ base, unsigned bytes) {
+    return *(const T *)((const char *)base + bytes);
+}
+template <typename T>
+__device__ __forceinline__ void put_off(T *__restrict__ base, unsigned bytes, T v) {
+    *(T *)((char *)base + bytes) = v;
+}
+// a point of one plane: `plane` its (uniform) start, `off` the lane's byte
+// offset in it (a plane is far below 4 GiB)
+template <typename R>
+__device__ __forceinline__ SP<R> load_sp(const R *__restrict__ plane, size_t nv, unsigned off) {
+    SP<R> p;
+
+    p.a[VR] = at_off(plane, off);
+    p.a[VU] = at_off(plane + nv, off);
+    p.a[VU + 1] = at_off(plane + 2 * nv, off);
+    p.a[VU + 2] = at_off(plane + 3 * nv, off);
+    p.a[VT] = at_off(plane + 5 * nv, off);
+    p.a[VM] = at_off(plane + 6 * nv, off);
+    if constexpr (sizeof(R) != sizeof(double)) p.a[VP_] = at_off(plane + 10 * nv, off);
+    return p;
+}
+
+template <typename R, bool CONS, bool SUMS>
+__device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P, R *__restrict__ wa,
+                                            R *__restrict__ fl, FluxArgs F) {
+    constexpr int TX = 32, TY = 8, NP = kNP<R>;
+    static_assert(TX * TY >= 2 * H * (TX + TY), "fewer lanes than halo points");
+    __shared__ R tiles[2][NP][TY + 2 * H][TX + 2 * H];
+    // metrics of the tile: Euler, then the three viscous ones (read from memory
+    // inside the march they would wait behind the previous plane's stores)
+    __shared__ R smx[4][TX], smy[4][TY], smz[4][kFluxMaxChunk];
+    __shared__ double sred[SUMS ? 5 : 1][SUMS ? TX * TY : 1];
+    __shared__ double lds[4][5];
+    // byte offsets of this lane: its point and its halo point in a plane of
+    // w_aux, its cell in a plane of the right-hand side, its mask entry.  (A
+    // spilled register would come back through the vector memory counter,
+    // behind the look-ahead loads.)
+    __shared__ unsigned soff[4][TX * TY];
+    __shared__ unsigned sedge[2][TX * TY];  // edge_cell's face orders along x and y
+    __shared__ R scd[H][H];
+    __shared__ R swx[H][TX], swy[H][TY];    // Euler weights of the tile's columns and rows
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    // band of whole tile rows per XCD (workgroups are dealt round-robin to the
+    // 8 XCDs): the halo points then mostly come from the XCD's own L2
+    int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+    const int flat = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    if (gridDim.y % 8 == 0) {
+        const int band = gridDim.y / 8;
+        const int per = gridDim.x * band;
+        const int r = (flat >> 3) % per;
+        bz = (flat >> 3) / per;
+        bx = r % gridDim.x;
+        by = (flat & 7) * band + r / gridDim.x;
+    }
+    const int i = bx * TX + tx + 1, j = by * TY + ty + 1;
+    const int k0 = bz * F.chunk + 1, k1 = min(k0 + F.chunk - 1, g.nz);
+    const bool act = i <= g.nx && j <= g.ny;
+    const int ic = min(i, g.nx), jc = min(j, g.ny);
+    const int ng = g.ng;
+    const size_t nv = g.nvol, ni = g.nint;
+    const int tid = ty * TX + tx;
+    // offsets in a plane: this lane's point, its halo point (lanes 0 ..
+    // 2H*TX-1 the y halo rows, the next 2H*TY lanes the x halo columns, the
+    // rest none) and its cell of the right-hand side
+    soff[0][tid] = (unsigned)sizeof(R) * (unsigned)((min(i, g.nx + H) + ng - 1) + g.sx * (min(j, g.ny + H) + ng - 1));
+    soff[2][tid] = (unsigned)sizeof(R) * (unsigned)((ic - 1) + g.nx * (jc - 1));
+    const bool hl = tid < 2 * H * (TX + TY);
+    int hlx = tx + H, hly = ty + H;
+    if (tid < 2 * H * TX) {
+        const int r = tid / TX;
+        hly = r < H ? r : r + TY;
+        hlx = tid % TX + H;
+    } else if (hl) {
+        const int q = tid - 2 * H * TX, c6 = q % (2 * H);
+        hly = q / (2 * H) + H;
+        hlx = c6 < H ? c6 : c6 + TX;
+    }
+    soff[1][tid] = (unsigned)sizeof(R) *
+        (unsigned)((min(bx * TX + 1 - H + hlx, g.nx + H) + ng - 1) + g.sx * (min(by * TY + 1 - H + hly, g.ny + H) + ng - 1));
+    const int hslot = hly * (TX + 2 * H) + hlx;
+    // (indices for the rare branches, formed there)
+    auto li = [&]() { return bx * TX + opaque(tx) + 1; };
+    auto lj = [&]() { return by * TY + opaque(ty) + 1; };
+    auto plane = [&](int k) { return wa + (ptrdiff_t)(k + ng - 1) * g.sxy; };
+    // cells beside a non-periodic boundary: faces of lowered order or zero flux
+    const int lb = P.lmax_base;
+    const bool inx = i >= P.eul_lo[0] && i <= P.eul_hi[0], iny = j >= P.eul_lo[1] && j <= P.eul_hi[1];
+    bool edx, edy;
+    {
+        auto edge = [&](const int *eoc, int c, int n, int zlo, int zhi) {
+            return (unsigned)max(lb + eoc[c - 1], 1) | (unsigned)max(lb + eoc[c], 1) << 4 |
+                   (c == 1 && zlo == 1 ? 1u << 8 : 0u) | (c == n && zhi == 1 ? 1u << 9 : 0u);
+        };
+        const unsigned plain = (unsigned)(lb | lb << 4);
+        const unsigned ex = edge(F.eocx, ic, g.nx, P.fzf[0], P.fzf[1]), ey = edge(F.eocy, jc, g.ny, P.fzf[2], P.fzf[3]);
+        edx = act && inx && ex != plain;
+        edy = act && iny && ey != plain;
+        sedge[0][tid] = ex;
+        sedge[1][tid] = ey;
+    }
+    if (tid < H * H) scd[tid / H][tid % H] = R(P.cd1tab[tid / H][tid % H]);
+    if (tid < H * TX) {
+        const int c = min(bx * TX + tid % TX + 1, g.nx);
+        swx[tid / TX][tid % TX] = R(P.cd1tab[max(max(lb + F.eocx[c - 1], lb + F.eocx[c]), 1) - 1][tid / TX]);
+    } else if (tid >= 128 && tid < 128 + H * TY) {
+        const int q = tid - 128, c = min(by * TY + q % TY + 1, g.ny);
+        swy[q / TY][q % TY] = R(P.cd1tab[max(max(lb + F.eocy[c - 1], lb + F.eocy[c]), 1) - 1][q / TY]);
+    }
+    // ghost images of div/3 (and the sensor) are written from this column
+    const bool wall = j == 1;
+    const bool imgc = i <= ng || i > g.nx - ng || j <= ng || j > g.ny - ng;
+    FluxConst<R> K;
+#pragma unroll
+    for (int l = 0; l < H; l++) K.c[l] = R(P.vd1[l]);
+#pragma unroll
+    for (int l = 0; l <= H; l++) K.c2[l] = R(P.vd2[l]);
+    K.rg = R(sizeof(R) == sizeof(double) ? P.rgas0 : 1.0);
+    K.pref = R(sizeof(R) == sizeof(double) ? 0.0 : P.p_ref);
+    // e_from_temperature of a calorically perfect gas
+    K.eb = R(cvc(P, 0));
+    K.ea = R(P.t0 * (cvc(P, P.indx_cp_r + 1) - cvc(P, 0)));
+    K.cpr = R(cpc(P, 0) / P.prandtl);
+    if (tid < TX) {
+        const int q = min(bx * TX + tid + 1, g.nx);
+        smx[0][tid] = R(F.dx1[q - 1]);
+        if (CONS) {
+            smx[1][tid] = R(1.0 / (F.xc[q + ng] - F.xc[q + ng - 2]));
+            smx[2][tid] = R(1.0 / (F.xc[q + ng - 1] - F.xc[q + ng - 2]));
+            smx[3][tid] = R(1.0 / (F.xc[q + ng] - F.xc[q + ng - 1]));
+        } else {
+            smx[1][tid] = R(F.dxs[q - 1]);
+            smx[2][tid] = R(F.dx2[q - 1]);
+        }
+    } else if (tid >= 64 && tid < 64 + TY) {
+        const int q = min(by * TY + tid - 64 + 1, g.ny);
+        smy[0][tid - 64] = R(F.dy1[q - 1]);
+        if (CONS) {
+            smy[1][tid - 64] = R(1.0 / (F.yc[q + ng] - F.yc[q + ng - 2]));
+            smy[2][tid - 64] = R(1.0 / (F.yc[q + ng - 1] - F.yc[q + ng - 2]));
+            smy[3][tid - 64] = R(1.0 / (F.yc[q + ng] - F.yc[q + ng - 1]));
+        } else {
+            smy[1][tid - 64] = R(F.dys[q - 1]);
+            smy[2][tid - 64] = R(F.dy2[q - 1]);
+        }
+    }
+    else if (tid >= 128 && tid < 128 + min(F.chunk, kFluxMaxChunk)) {
+        const int z = tid - 128, q = min(k0 + z, g.nz);
+        smz[0][z] = R(F.dz1[q - 1]);
+        if (CONS) {
+            smz[1][z] = R(1.0 / (F.zc[q + ng] - F.zc[q + ng - 2]));
+            smz[2][z] = R(1.0 / (F.zc[q + ng - 1] - F.zc[q + ng - 2]));
+            smz[3][z] = R(1.0 / (F.zc[q + ng] - F.zc[q + ng - 1]));
+        } else {
+            smz[1][z] = R(F.dzs[q - 1]);
+            smz[2][z] = R(F.dz2[q - 1]);
+        }
+    }
+    if (SUMS) {
+#pragma unroll
+        for (int q = 0; q < 5; q++) sred[q][tid] = 0.0;
+    }
+    // masks of this lane's 32 cells (a tile row is 32 cells from a multiple of 32)
+    const int dpr = dirty_per_row(g);
+    soff[3][tid] = (unsigned)sizeof(uint3) * (unsigned)((jc - 1) * dpr + ((ic - 1) >> 5));
+    const size_t dirtyplane = (size_t)g.ny * dpr;
+    auto load_masks = [&](int k) { return at_off(F.dirty + (size_t)(k - 1) * dirtyplane, soff[3][tid]); };
+    // bit d: direction d of the cell has a WENO face
+    auto masks_of = [&](const uint3 &m) {
+        return ((m.x >> tx) & 1u) | (((m.y >> tx) & 1u) << 1) | (((m.z >> tx) & 1u) << 2);
+    };
+    auto fill = [&](int b, const SP<R> &centre, const SP<R> &halo) {
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            tiles[b][q][ty + H][tx + H] = centre.a[q];
+            if (hl) (&tiles[b][q][0][0])[hslot] = halo.a[q];
+        }
+    };
+    SP<R> win[2 * H + 1], nxt, hv;  // planes k-3 .. k+3; the look-ahead
+    uint3 mk;
+    unsigned wm;
+#pragma unroll
+    for (int q = 0; q < 2 * H + 1; q++) win[q] = load_sp(plane(min(k0 - H + q, g.nz + H)), nv, soff[0][tid]);
+    hv = load_sp(plane(k0), nv, soff[1][tid]);
+    mk = load_masks(k0);
+    wm = masks_of(mk);
+    fill(0, win[H], hv);
+    nxt = win[2 * H];
+    int buf = 0;
+    for (int k = k0; k <= k1; k++, buf ^= 1) {
+        const SP<R> &o = win[H];
+        R(*tile)[TY + 2 * H][TX + 2 * H] = tiles[buf];
+        __syncthreads();
+        auto at_x = [&](int l) {
+            SP<R> p;
+#pragma unroll
+            for (int q = 0; q < NP; q++) p.a[q] = tile[q][ty + H][tx + H + l];
+            return p;
+        };
+        auto at_y = [&](int l) {
+            SP<R> p;
+#pragma unroll
+            for (int q = 0; q < NP; q++) p.a[q] = tile[q][ty + H + l][tx + H];
+            return p;
+        };
+        auto at_z = [&](int l) { return win[H + l]; };
+        CellAcc<R> A;
+        A.m = A.e = R(0);
+#pragma unroll
+        for (int q = 0; q < 3; q++) A.mk[q] = R(0);
+        const R pr = K.rg * sp_press(o) + K.pref;
+        const R az = smz[0][k - k0], ax = smx[0][tx], ay = smy[0][ty];
+        const R amx = inx && !(wm & 1u) ? ax : R(0), amy = iny && !(wm & 2u) ? ay : R(0),
+                amz = (wm & 4u) ? R(0) : az;
+        // loads of plane k+1 (halo, masks) and k+1+H (centre): issued once the
+        // z terms are done and taken up before this plane's stores are issued
+        // (memory counters retire in order: a load waited for behind a store
+        // waits for the store), they overlap the x and y work
+        auto look_ahead = [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+            // (clamped, not skipped, behind the last plane: a load left in
+            // flight by one iteration only would make every iteration wait
+            // for its stores)
+            nxt = load_sp(plane(min(k + 1 + H, g.nz + H)), nv, soff[0][tid]);
+            hv = load_sp(plane(k + 1), nv, soff[1][tid]);
+            mk = load_masks(min(k + 1, g.nz));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // The stress terms of a pair of directions are added as soon as both
+        // have their derivatives (kernels_cpu.F90:3996-4180; in the
+        // conservative form their mu-gradient part, sig_xy = d(u_y)/dx_x):
+        // momentum in mk, dissipation in e, and the vorticity for the sensor.
+        R om2 = R(0);
+        auto cross = [&](int x, int y, const Grad<R> &X, const Grad<R> &Y) {
+            const R a = Y.u[x], b = X.u[y];  // d u_x / dy, d u_y / dx
+            om2 += (b - a) * (b - a);
+            if (CONS) {
+                A.mk[x] -= R(4) * (Y.m * b);
+                A.mk[y] -= R(4) * (X.m * a);
+                A.e -= R(2) * o.a[VM] * (a * b);
+            } else {
+                const R sxy = a + b;
+                A.mk[x] -= R(4) * (Y.m * sxy);
+                A.mk[y] -= R(4) * (X.m * sxy);
+                A.e -= o.a[VM] * (sxy * sxy);
+            }
+        };
+        R gty;
+        Grad<R> GX, GY, GZ;
+        auto weights = [&](const R *sw, int stride, R (&w)[H]) {
+#pragma unroll
+            for (int l = 0; l < H; l++) w[l] = sw[l * stride];
+        };
+        R ew[H];
+        if constexpr (CONS) {
+            flux_dir_cons<R, 2>(K, o, at_z, K.c, pr, amz, smz[1][k - k0], smz[2][k - k0], smz[3][k - k0], A, GZ);
+            look_ahead();
+            weights(&swx[0][tx], TX, ew);
+            flux_dir_cons<R, 0>(K, o, at_x, ew, pr, amx, smx[1][tx], smx[2][tx], smx[3][tx], A, GX);
+            cross(0, 2, GX, GZ);
+            weights(&swy[0][ty], TY, ew);
+            gty = flux_dir_cons<R, 1>(K, o, at_y, ew, pr, amy, smy[1][ty], smy[2][ty], smy[3][ty], A, GY);
+        } else {
+            flux_dir<R, 2>(K, o, at_z, K.c, pr, amz, az, smz[1][k - k0], smz[2][k - k0], A, GZ);
+            look_ahead();
+            weights(&swx[0][tx], TX, ew);
+            flux_dir<R, 0>(K, o, at_x, ew, pr, amx, ax, smx[1][tx], smx[2][tx], A, GX);
+            cross(0, 2, GX, GZ);
+            weights(&swy[0][ty], TY, ew);
+            gty = flux_dir<R, 1>(K, o, at_y, ew, pr, amy, ay, smy[1][ty], smy[2][ty], A, GY);
+        }
+        cross(0, 1, GX, GY);
+        cross(1, 2, GY, GZ);
+        const R u = o.a[VU], v = o.a[VU + 1], w = o.a[VU + 2], t = o.a[VT], mu = o.a[VM];
+        const R uy = GY.u[0], wy = GY.u[2];
+        const R d3 = (GX.u[0] + GY.u[1] + GZ.u[2]) * R(1.0 / 3.0);
+        {
+            // 2 (du_x/dx - div/3); the conservative form has its first half in the face fluxes
+            const R two = R(2);
+            const R s11 = CONS ? GX.u[0] - two * d3 : two * (GX.u[0] - d3);
+            const R s22 = CONS ? GY.u[1] - two * d3 : two * (GY.u[1] - d3);
+            const R s33 = CONS ? GZ.u[2] - two * d3 : two * (GZ.u[2] - d3);
+            A.mk[0] -= R(4) * (GX.m * s11);
+            A.mk[1] -= R(4) * (GY.m * s22);
+            A.mk[2] -= R(4) * (GZ.m * s33);
+            A.e -= mu * (s11 * GX.u[0] + s22 * GY.u[1] + s33 * GZ.u[2]);
+        }
+        R f[5];
+        f[0] = R(0.5) * A.m;
+        f[1] = R(0.25) * (u * A.m + A.mk[0]);
+        f[2] = R(0.25) * (v * A.m + A.mk[1]);
+        f[3] = R(0.25) * (w * A.m + A.mk[2]);
+        f[4] = R(0.25) * ((R(2) * K.ea + K.eb * t) * A.m + u * A.mk[0] + v * A.mk[1] + w * A.mk[2]) + A.e;
+        if (edx && !(wm & 1u)) edge_cell<R, 0>(at_x, o, sedge[0][tid], scd, K, ax, f);
+        if (edy && !(wm & 2u)) edge_cell<R, 1>(at_y, o, sedge[1][tid], scd, K, ay, f);
+        if (SUMS && act) {
+            // force_rhs: the grad(div/3) part of the rho*u sum by parts
+            // along the uniform periodic x: -sum mu d(D)/dx = +sum D d(mu)/dx
+            sred[0][tid] += double(f[0]);
+            sred[1][tid] += double(f[1]) + double(d3) * double(GX.m);
+            double w1, w2;
+            if constexpr (sizeof(R) == sizeof(double)) {
+                w1 = o.a[VR];
+                w2 = o.a[VR] * u;
+            } else {
+                const int c = gidx(g, li(), lj(), k);
+                w1 = F.w[c];
+                w2 = F.w[nv + c];
+            }
+            sred[2][tid] += w1;
+            sred[3][tid] += w2;
+            sred[4][tid] += w2 * double(t);
+        }
+        fill(buf ^ 1, win[H + 1], hv);
+        wm = masks_of(mk);
+#pragma unroll
+        for (int q = 0; q < 2 * H; q++) win[q] = win[q + 1];
+        win[2 * H] = nxt;
+        __builtin_amdgcn_sched_barrier(0);
+        if (act) {
+            const unsigned oc = soff[0][tid], of = soff[2][tid];
+            R *fk = fl + (size_t)(k - 1) * g.nx * g.ny;
+#pragma unroll
+            for (int q = 0; q < 5; q++) put_off(fk + q * ni, of, f[q]);
+            put_off(plane(k) + 9 * nv, oc, d3);
+            const bool img = imgc || k <= ng || k > g.nz - ng;
+            if (img) write_images(g, P, wa + 9 * nv, li(), lj(), k, d3, true);
+            if (F.last) {
+                // visflx(3): the sensor from the stored |omega| and div/3
+                // (sensor_subroutine, kernels_cpu.F90:4726-4744); the switch
+                // of this step works from the masks, so it can go in place
+                const R om = sqrt(om2);
+                put_off(plane(k) + 8 * nv, oc, om);
+                const R dv = R(3.0) * d3, ul = R(P.u0 / P.l0);
+                R sv = -dv / sqrt(om * om + dv * dv + ul * ul);
+                sv = fmax(sv, R(0.0));
+                put_off(plane(k) + 7 * nv, oc, sv * sv);
+                if (img) write_images(g, P, wa + 7 * nv, li(), lj(), k, sv * sv, false);
+            }
+            if (wall) {
+                const size_t wsz = (size_t)g.sx * g.sz;
+                const size_t wp = (size_t)(li() + ng - 1) + (size_t)g.sx * (k + ng - 1);
+                F.wallprop[wp] = double(mu * uy);
+                F.wallprop[wsz + wp] = double(mu * wy);
+                F.wallprop[2 * wsz + wp] = double(mu * gty * K.cpr);
+            }
+        }
+    }
+    if (SUMS) {
+        const int jy = min(lj(), g.ny);
+        const double dy = F.yn[jy] - F.yn[jy - 1];
+        double red[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) red[q] = sred[q][tid] * dy;
+        block_sum<5>(red, lds);
+        if (tid == 0) {
+#pragma unroll
+            for (int q = 0; q < 5; q++) F.partials[(size_t)flat * 5 + q] = red[q];
+        }
+    }
+}
+template <typename R, bool CONS, bool SUMS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFluxWaves<R>))) void k_flux(Geo g, KPar P, R *__restrict__ wa, R *__restrict__ fl, FluxArgs F) {
+    k_flux_body<R, CONS, SUMS>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, wa, fl, F);
+}
+
+// ============================================================ WENO items
+// Hybrid flux of one face in direction-aligned velocities (u normal, v and w
+// the tangential ones in the order of the eigenvector routines): the x
+// routines then serve all three directions, with the direction a property of
+// the lane.
+__device__ __forceinline__ void item_face(const KPar &P, const Pt (&q)[6], bool hot, int f, int e, int n, int dir,
+                                          double fh[5]) {
+    if (hot) {
+        weno_flux<0, 3>(P, q, e, fh);
+    } else {
+        Pc c[6];
+#pragma unroll
+        for (int s = 0; s < 6; s++) c[s] = pc_of(q[s]);
+        int lmax = P.lmax_base + e;
+        lmax = lmax < 1 ? 1 : lmax;
+        const int zlo = dir == 0 ? P.fzf[0] : (dir == 1 ? P.fzf[2] : P.fzf[4]);
+        const int zhi = dir == 0 ? P.fzf[1] : (dir == 1 ? P.fzf[3] : P.fzf[5]);
+        central_flux<0, 3, Pc, 0>(P, c, lmax, (f == 0 && zlo == 1) || (f == n && zhi == 1), fh);
+    }
+}
+
+struct ItemArgs {
+    const int *eoc[3];
+    const double *metric[3];
+    const uint64_t *rec;
+    const int *list, *counts;
+    int nseg, wpt;
+    // finish of the stage's reductions
+    const double *partials;  // 5 sums of each of nblk workgroups of k_flux
+    int nblk;
+    const double *dtpart;    // ndt block maxima of the CFL radii (ndt = 0: no new dt)
+    int ndt;
+    double *stage2;
+    int *ticket;
+    DevScalars *ds;
+    const double *yn;
+    double rkr, rkg;
+    int channel, first;
+};
+
+// The WENO work items of the stage: item (cell, direction) evaluates the two
+// faces of the cell along the direction, WENO or central as the masks say,
+// and gives the cell (fhat_hi - fhat_lo) * metric.  The items of one cell are
+// neighbours in the list: the lane of the first one adds them up in direction
+// order and stores, so a cell is written once and the result does not depend
+// on the schedule.  A wave takes 64 items and owns the cells that start in
+// the first 62.  All directions share one launch, and every face is hybrid
+// per lane; bound by the latency of the scattered stencil loads.
+//
+// The workgroups then finish the reductions of the stage (two levels, fixed
+// order): the bulk sums of k_flux with the items' changes, giving b1, b2,
+// dpdx and the bulk values of force_rhs (singleideal_cpu.F90:845-889), and
+// the CFL step (:1507-1514).  The sums of the previous stage's right-hand
+// side are those it finished with (DevScalars::rhs_sum).
+template <typename R>
+__device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
+                                                  const R *__restrict__ wa, const double *__restrict__ w,
+                                                  R *__restrict__ fl, ItemArgs A) {
+    __shared__ int pre[kItemSeg + 1];
+    __shared__ int wsum[4];
+    __shared__ double lds[4][5];
+    __shared__ double ldm[4];
+    __shared__ bool last;
+    const int t = threadIdx.x, lane = t & 63;
+    double red[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    int total;
+    {
+        int cs[16], sum = 0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int sgi = 16 * t + q;
+            cs[q] = sgi < A.nseg ? abs(A.counts[sgi]) : 0;
+            sum += cs[q];
+        }
+        int run = block_excl_scan256(sum, wsum, &total);
+#pragma unroll
+        for (int q = 0; q < 16; q++) {
+            const int sgi = 16 * t + q;
+            if (sgi < A.nseg) pre[sgi] = run;
+            run += cs[q];
+        }
+        if (t == 0) pre[A.nseg] = total;
+        __syncthreads();
+    }
+    const size_t nv = g.nvol, ni = g.nint;
+    const int nwx = rec_per_row(g), nwords = nwx * g.ny * g.nz;
+    // item e: its cell (linear) and code; in a segment without a list the
+    // (cell, direction) pairs in order, their masks from the records
+    auto item = [&](int e, int &cell, int &code) {
+        int lo = 0, hi = A.nseg;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (pre[mid] <= e) lo = mid;
+            else hi = mid;
+        }
+        const int S0 = seg_first_cell(g, nwx, lo * 256 * A.wpt, nwords);
+        const int x = e - pre[lo];
+        if (A.counts[lo] >= 0) {
+            code = A.list[S0 + x];
+            cell = S0 + (code & 0xffffff);
+        } else {
+            cell = S0 + x / 3;
+            const int d = x % 3, i0 = cell % g.nx;
+            const uint64_t *rc = A.rec + kRecWords * ((size_t)(cell / g.nx) * nwx + (i0 >> 6)) + 2 * d;
+            code = d << 24 | (int)((rc[0] >> (i0 & 63)) & 1ull) << 26 | (int)((rc[1] >> (i0 & 63)) & 1ull) << 27;
+        }
+    };
+    const int wave = (blockIdx.x * blockDim.x + t) >> 6;
+    const int nwaves = (gridDim.x * blockDim.x) >> 6;
+    for (int base = wave * 62; base < total; base += nwaves * 62) {
+        const int e = base + lane;
+        int cell = -1, code = 0;
+        if (e < total) item(e, cell, code);
+        const bool lo_hot = (code >> 26) & 1, hi_hot = (code >> 27) & 1;
+        const bool work = cell >= 0 && (lo_hot || hi_hot);
+        double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        int j = 1;
+        if (work) {
+            const int dir = (code >> 24) & 3;
+            const int i = cell % g.nx + 1, jk = cell / g.nx;
+            j = jk % g.ny + 1;
+            const int k = jk / g.ny + 1;
+            const int c = dir == 0 ? i : (dir == 1 ? j : k);
+            const int n = dir == 0 ? g.nx : (dir == 1 ? g.ny : g.nz);
+            const int stride = dir == 0 ? 1 : (dir == 1 ? g.sx : g.sxy);
+            const int *eoc = dir == 0 ? A.eoc[0] : (dir == 1 ? A.eoc[1] : A.eoc[2]);
+            const double *met = dir == 0 ? A.metric[0] : (dir == 1 ? A.metric[1] : A.metric[2]);
+            const size_t on = (size_t)(1 + dir) * nv, o1 = (dir == 0 ? 2 : 1) * nv, o2 = (dir == 2 ? 2 : 3) * nv;
+            const int b0 = gidx(g, i, j, k);
+            // every load of the stencil before any arithmetic
+            double raw[7][6];
+#pragma unroll
+            for (int s = 0; s < 7; s++) {
+                const int a = b0 + (s - 3) * stride;
+                if constexpr (sizeof(R) == sizeof(double)) {
+                    raw[s][0] = wa[a];
+                    raw[s][1] = wa[on + a];
+                    raw[s][2] = wa[o1 + a];
+                    raw[s][3] = wa[o2 + a];
+                    raw[s][4] = wa[4 * nv + a];
+                    raw[s][5] = wa[5 * nv + a];
+                } else {
+                    // the mixed form stores w_aux in FP32: the FP64 primitives
+                    // of w, periodic neighbours from their images
+                    int pi = i, pj = j, pk = k;
+                    if (dir == 0) pi += s - 3;
+                    else if (dir == 1) pj += s - 3;
+                    else pk += s - 3;
+                    if (P.periodic[0]) pi = pi < 1 ? pi + g.nx : (pi > g.nx ? pi - g.nx : pi);
+                    if (P.periodic[1]) pj = pj < 1 ? pj + g.ny : (pj > g.ny ? pj - g.ny : pj);
+                    if (P.periodic[2]) pk = pk < 1 ? pk + g.nz : (pk > g.nz ? pk - g.nz : pk);
+                    const int src = gidx(g, pi, pj, pk);
+                    raw[s][0] = w[src];
+                    raw[s][1] = w[on + src];
+                    raw[s][2] = w[o1 + src];
+                    raw[s][3] = w[o2 + src];
+                    raw[s][4] = w[4 * nv + src];
+                    raw[s][5] = 0.0;
+                }
+            }
+            const int elo = eoc[c - 1], ehi = eoc[c];
+            const double mt = met[c - 1];
+            Pt q[7];
+#pragma unroll
+            for (int s = 0; s < 7; s++) {
+                if constexpr (sizeof(R) == sizeof(double)) {
+                    q[s] = make_pt(raw[s][0], raw[s][1], raw[s][2], raw[s][3], raw[s][4], raw[s][5], P.rgas0, true);
+                } else {
+                    const double rho = raw[s][0], rhoe = raw[s][4];
+                    const double ri = 1.0 / rho;
+                    const double uu = raw[s][1] * ri, vv = raw[s][2] * ri, ww = raw[s][3] * ri;
+                    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+                    const double tt = temperature_from_e(P, rhoe / rho - qq, 0.0);
+                    const double pp = rho * tt * P.rgas0;
+                    q[s] = make_pt(rho, uu, vv, ww, (rhoe + pp) / rho, tt, P.rgas0, true);
+                }
+            }
+            // WENO face first (the lower one where it has one): the lanes of a
+            // wave then run the WENO branch together
+            const bool alo = lo_hot || !hi_hot;
+            double fa[5], fb[5];
+#pragma unroll 1
+            for (int s2 = 0; s2 < 2; s2++) {
+                const bool lo = (s2 == 0) == alo;
+                Pt qw[6];
+#pragma unroll
+                for (int s = 0; s < 6; s++) qw[s] = lo ? q[s] : q[s + 1];
+                double fh[5];
+                item_face(P, qw, lo ? lo_hot : hi_hot, lo ? c - 1 : c, lo ? elo : ehi, n, dir, fh);
+#pragma unroll
+                for (int m = 0; m < 5; m++) {
+                    if (lo) fa[m] = fh[m];
+                    else fb[m] = fh[m];
+                }
+            }
+            double x[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) x[m] = (fb[m] - fa[m]) * mt;
+            d[0] = x[0];
+            d[4] = x[4];
+            d[1] = dir == 0 ? x[1] : x[2];
+            d[2] = dir == 0 ? x[2] : (dir == 1 ? x[1] : x[3]);
+            d[3] = dir == 2 ? x[1] : x[3];
+        }
+        // the cell's first item adds its other ones (at most two) and stores
+        const int c1 = __shfl_down(cell, 1, 64), c2 = __shfl_down(cell, 2, 64);
+        int cm = __shfl_up(cell, 1, 64);
+        if (lane == 0) {
+            cm = -1;
+            int cd;
+            if (base > 0) item(base - 1, cm, cd);
+        }
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+            const double a = __shfl_down(d[m], 1, 64), b = __shfl_down(d[m], 2, 64);
+            if (c1 == cell) d[m] += a;
+            if (c2 == cell) d[m] += b;
+        }
+        const bool lead = lane < 62 && cell >= 0 && cm != cell;
+        if (lead && (d[0] != 0.0 || d[1] != 0.0 || d[2] != 0.0 || d[3] != 0.0 || d[4] != 0.0)) {
+            R fo[5], fn[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) fo[m] = fl[m * ni + cell];
+#pragma unroll
+            for (int m = 0; m < 5; m++) {
+                fn[m] = R(double(fo[m]) + d[m]);
+                fl[m * ni + cell] = fn[m];
+            }
+            if (A.channel) {
+                const int jj = (cell / g.nx) % g.ny + 1;
+                const double dy = A.yn[jj] - A.yn[jj - 1];
+                red[0] += (double(fn[0]) - double(fo[0])) * dy;
+                red[1] += (double(fn[1]) - double(fo[1])) * dy;
+            }
+        }
+    }
+    if (!A.channel && A.ndt == 0) return;
+    double mx = 0.0;
+    if (A.channel) {
+        const int per = (A.nblk + (int)gridDim.x - 1) / (int)gridDim.x;
+        const int b0 = (int)blockIdx.x * per, b1 = min(b0 + per, A.nblk);
+        for (int b = b0 + t; b < b1; b += 256) {
+#pragma unroll
+            for (int q = 0; q < 5; q++) red[q] += A.partials[(size_t)b * 5 + q];
+        }
+        block_sum<5>(red, lds);
+    }
+    if (A.ndt) {
+        const int per = (A.ndt + (int)gridDim.x - 1) / (int)gridDim.x;
+        const int b0 = (int)blockIdx.x * per, b1 = min(b0 + per, A.ndt);
+        for (int b = b0 + t; b < b1; b += 256) mx = fmax(mx, A.dtpart[b]);
+        mx = wave_max(mx);
+        if (lane == 0) ldm[t >> 6] = mx;
+        __syncthreads();
+        mx = fmax(fmax(ldm[0], ldm[1]), fmax(ldm[2], ldm[3]));
+    }
+    if (t == 0) {
+#pragma unroll
+        for (int q = 0; q < 5; q++) A.stage2[blockIdx.x * 6 + q] = red[q];
+        A.stage2[blockIdx.x * 6 + 5] = mx;
+        __threadfence();
+        last = atomicAdd(A.ticket, 1) == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    // gridDim.x <= 256: one second-level value per thread, past the
+    // non-coherent caches, added by the same fixed tree
+    double v[6];
+#pragma unroll
+    for (int q = 0; q < 6; q++)
+        v[q] = t < (int)gridDim.x
+                   ? __hip_atomic_load(&A.stage2[t * 6 + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                   : 0.0;
+    mx = wave_max(v[5]);
+    if (lane == 0) ldm[t >> 6] = mx;
+    double r5[5] = {v[0], v[1], v[2], v[3], v[4]};
+    block_sum<5>(r5, lds);  // its barrier also covers ldm
+    if (t == 0) {
+        *A.ticket = 0;
+        DevScalars *ds = A.ds;
+        if (A.ndt) {
+            const double dt_min = 1.0 / fmax(fmax(ldm[0], ldm[1]), fmax(ldm[2], ldm[3]));
+            ds->dt = P.cfl * dt_min;
+        }
+        if (A.channel) {
+            const double rhodt = A.rkr * ds->dt, gamdt = A.rkg * ds->dt;
+            double b1 = -gamdt * r5[0], b2 = -gamdt * r5[1];
+            if (A.rkr != 0.0) {
+                b1 -= rhodt * ds->rhs_sum[0];
+                b2 -= rhodt * ds->rhs_sum[1];
+            }
+            b1 = b1 / P.volchan;
+            b2 = b2 / P.volchan;
+            ds->rhs_sum[0] = r5[0];
+            ds->rhs_sum[1] = r5[1];
+            const double b3 = r5[2] / P.volchan, b4 = r5[3] / P.volchan, b5 = r5[4] / P.volchan;
+            ds->dpdx = (A.first ? 0.0 : ds->dpdx) + b2;
+            ds->rhobulk = b3;
+            ds->ubulk = b4 / b3;
+            ds->tbulk = b5 / b3 / ds->ubulk;
+            ds->b1 = b1;
+            ds->b2 = b2;
+        }
+    }
+}
+template <typename R>
+__global__ __launch_bounds__(256) void k_weno_items(Geo g, KPar P, const R *__restrict__ wa,
+                                                    const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
+    k_weno_items_body<R>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, wa, w, fl, A);
+}
+
+// ============================================================ update
+struct UpdArgs {
+    const double *dx1, *dy1, *dz1, *xc, *yc, *zc, *yn;
+    DevScalars *ds;
+    double rkr, rkg;
+    int channel;
+    int chunk;
+    int step_end;      // third stage of st_advance: icyc += 1, time += dt
+    double *partials;  // block sums of rho u T dy (FV)
+};
+
+// visflx_div (kernels_cpu.F90:3484-3532, or its second-order form with O2,
+// :3446-3480) on the completed right-hand side, then update_flux +
+// force_rhs_2 + update_field (:3400-3442, 3092-3116) and the staggered
+// isothermal-wall ghosts; with FV, force_var_1 (:3241-3278) and the block sums
+// of rho*u*T*dy.  The grad(div/3) terms cost two more reads here (mu, div/3:
+// 16 B a cell) where the pass of their own re-read and re-wrote the
+// right-hand side (152 B).  The velocities of the energy term are formed from
+// w as eval_aux forms them.  A workgroup takes 64 x 4 columns of a few planes
+// with the z stencil of div/3 in registers.  Bound by HBM: 197 B a cell, 1.38
+// ms on 512 x 256 x 256 (4.8 TB/s; the update alone took 0.99 ms, the div/3
+// part of the z march about 0.5).  The right-hand sides are read with
+// the non-temporal hint: neither is read again before a full stage of
+// traffic has passed.
+template <typename R, bool FV, bool O2>
+__device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
+                                                  double *__restrict__ w, R *__restrict__ wa,
+                                                  const R *__restrict__ flp, R *__restrict__ fl, UpdArgs U) {
+    __shared__ double lds[4][1];
+    const int i = blockIdx.x * 64 + threadIdx.x + 1;
+    const int j = blockIdx.y * 4 + threadIdx.y + 1;
+    const int k0 = blockIdx.z * U.chunk + 1, k1 = min(k0 + U.chunk - 1, g.nz);
+    constexpr int HW = O2 ? 1 : 3;
+    double acc[1] = {0.0};
+    const double dt = U.ds->dt;
+    if (i <= g.nx && j <= g.ny) {
+        const size_t nv = g.nvol, ni = g.nint;
+        const double rhodt = U.rkr * dt, gamdt = U.rkg * dt;
+        const double b1 = U.channel ? U.ds->b1 : 0.0, b2 = U.channel ? U.ds->b2 : 0.0;
+        const int ng = g.ng;
+        const R *D = wa + 9 * nv;
+        R ax, ay;
+        if (O2) {
+            ax = R(1.0) / R(U.xc[i + ng] - U.xc[i + ng - 2]);
+            ay = R(1.0) / R(U.yc[j + ng] - U.yc[j + ng - 2]);
+        } else {
+            ax = R(U.dx1[i - 1]);
+            ay = R(U.dy1[j - 1]);
+        }
+        const int col = gidx(g, i, j, 0);
+        R dw[2 * HW + 1];
+#pragma unroll
+        for (int q = 0; q < 2 * HW; q++) dw[q + 1] = D[col + (k0 - HW + q) * g.sxy];
+        for (int k = k0; k <= k1; k++) {
+            const int c = col + k * g.sxy, oi = iidx(g, i, j, k);
+#pragma unroll
+            for (int q = 0; q < 2 * HW; q++) dw[q] = dw[q + 1];
+            dw[2 * HW] = D[c + HW * g.sxy];
+            R fo[5], fp[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) fo[m] = __builtin_nontemporal_load(&fl[m * ni + oi]);
+            if (U.rkr != 0.0) {
+#pragma unroll
+                for (int m = 0; m < 5; m++) fp[m] = __builtin_nontemporal_load(&flp[m * ni + oi]);
+            }
+            double wo[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) wo[m] = w[m * nv + c];
+            const R mu = wa[6 * nv + c];
+            R gx = R(0), gy = R(0), gz = R(0);
+#pragma unroll
+            for (int l = 1; l <= HW; l++) {
+                const R cl = O2 ? R(1) : R(P.vd1[l - 1]);
+                gx += cl * (D[c + l] - D[c - l]);
+                gy += cl * (D[c + l * g.sx] - D[c - l * g.sx]);
+                gz += cl * (dw[HW + l] - dw[HW - l]);
+            }
+            const R az = O2 ? R(1.0) / R(U.zc[k + ng] - U.zc[k + ng - 2]) : R(U.dz1[k - 1]);
+            const R sx = mu * (gx * ax), sy = mu * (gy * ay), sz = mu * (gz * az);
+            const double ri = 1.0 / wo[0];
+            const double uo = wo[1] * ri, vo = wo[2] * ri, wwo = wo[3] * ri;
+            fo[1] -= sx;
+            fo[2] -= sy;
+            fo[3] -= sz;
+            fo[4] -= sx * R(uo) + sy * R(vo) + sz * R(wwo);
+#pragma unroll
+            for (int m = 1; m < 5; m++) fl[m * ni + oi] = fo[m];
+            double fln[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) {
+                fln[m] = -gamdt * double(fo[m]);
+                if (U.rkr != 0.0) fln[m] = -rhodt * double(fp[m]) + fln[m];
+            }
+            if (U.channel) {
+                fln[0] = fln[0] - b1;
+                fln[1] = fln[1] - b2;
+                fln[4] = fln[4] - uo * b2;
+            }
+            double wn[5];
+#pragma unroll
+            for (int m = 0; m < 5; m++) {
+                wn[m] = wo[m] + fln[m];
+                w[m * nv + c] = wn[m];
+            }
+            if (FV) {
+                const double dy = U.yn[j] - U.yn[j - 1];
+                const double rn = 1.0 / wn[0];
+                const double uu = wn[1] * rn, vv = wn[2] * rn, ww = wn[3] * rn;
+                const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+                const double ee = wn[4] / wn[0] - qq;
+                const double tt = temperature_from_e(P, ee, 0.0);
+                wa[5 * nv + c] = R(tt);
+                acc[0] += wn[1] * tt * dy;
+            } else {
+                if (P.wall_stag[0] && j <= g.ng) wall_ghost(g, P, w, wa, i, j, 1 - j, k);
+                if (P.wall_stag[1] && j > g.ny - g.ng) wall_ghost(g, P, w, wa, i, j, 2 * g.ny + 1 - j, k);
+            }
+        }
+    }
+    if (FV) {
+        block_sum<1>(acc, lds);
+        if (flat_thread() == 0)
+            U.partials[(int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z))] = acc[0];
+    }
+    // run()'s loop end (singleideal_cpu.F90:1604,1642); nothing else of this
+    // launch reads time or icyc
+    if (U.step_end && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && flat_thread() == 0) {
+        U.ds->icyc = U.ds->icyc + 1;
+        U.ds->time = U.ds->time + dt;
+    }
+}
+template <typename R, bool FV, bool O2>
+__global__ __launch_bounds__(256) void k_update_div(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa,
+                                                    const R *__restrict__ flp, R *__restrict__ fl, UpdArgs U) {
+    k_update_div_body<R, FV, O2>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, w, wa, flp, fl, U);
+}
+
+// ================================================================ launchers
+#define ST_DISPATCH(call)                         \
+    do {                                          \
+        if (s->mixed) {                           \
+            using R = float;                      \
+            call;                                 \
+        } else {                                  \
+            using R = double;                     \
+            call;                                 \
+        }                                         \
+    } while (0)
+
+// The one-pass stage covers the KEEP split of a calorically perfect gas with
+// the Roe split on the fused kernels' three ghost layers.  The span must be
+// periodic (the z stencils sit in registers, where a face of lowered order
+// has no cheap form) and, where force_rhs needs the bulk sums, x periodic
+// and uniform (its grad(div/3) sum is taken by parts along x).
+bool one_pass_stage(const st_solver *s) {
+    const st_params &p = s->p;
+    return p.ng == H && p.nkeep == 0 && p.calorically_perfect == 1 && p.flux_splitting == 0 && s->kp.ndim == 3 &&
+           s->kp.periodic[2] && s->kp.eul_lo[0] <= s->kp.eul_hi[0] && s->kp.eul_lo[1] <= s->kp.eul_hi[1] &&
+           (!p.channel_case || (s->kp.periodic[0] && s->x_uniform));
+}
+
+static const int kFluxTX = 32, kFluxTY = 8;
+
+// Planes per workgroup of k_flux.  The chip holds two (FP64) or three (mixed)
+// workgroups a CU, and a round of them takes about chunk + 1.1 plane times
+// (4.7 us a plane and 5.2 us for the stencil's first planes and the launch, on
+// 512 x 256 x 256 at chunks 4, 8 and 16; with a CU to itself a workgroup takes
+// 3.4 us a plane).  Long chunks spare the start-up, short ones fill the chip
+// and its last round: the chunk with the least rounds x round time.  On
+// 128 x 96 x 64 chunks 2, 4, 8, 16 took 50, 47, 51, 66 us.
+static int flux_chunk(const Geo &g, bool mixed) {
+    const long tiles = (long)((g.nx + kFluxTX - 1) / kFluxTX) * ((g.ny + kFluxTY - 1) / kFluxTY);
+    const int cus = 256, slots = cus * (mixed ? 3 : 2);
+    int best = 1;
+    double least = 0.0;
+    for (int c = 1; c <= kFluxMaxChunk && c <= g.nz; c++) {
+        const long blocks = tiles * ((g.nz + c - 1) / c);
+        const double t = blocks <= cus ? 1.1 + 0.73 * c : (double)((blocks + slots - 1) / slots) * (1.1 + c);
+        if (c == 1 || t < least) {
+            least = t;
+            best = c;
+        }
+    }
+    return best;
+}
+static dim3 flux_grid(const Geo &g, int chunk) {
+    return dim3((g.nx + kFluxTX - 1) / kFluxTX, (g.ny + kFluxTY - 1) / kFluxTY, (g.nz + chunk - 1) / chunk);
+}
+// Planes per workgroup of k_update_div: each reads 6 planes of div/3 beyond its
+// own, and its planes' loads wait for one another's stores; on 512 x 256 x 256
+// chunks 1, 2, 4, 16 took 1371, 1379, 1402, 1438 us, on 256 x 128 x 128 165,
+// 161, 160, 173, on 48 x 40 x 36 chunks 1, 2 took 9.1, 10.0.
+static int update_chunk(const Geo &g) {
+    const long cols = (long)((g.nx + 63) / 64) * ((g.ny + 3) / 4);
+    return cols * ((g.nz + 1) / 2) >= 2048 ? 2 : 1;
+}
+static dim3 update_grid(const Geo &g, int chunk) {
+    return dim3((g.nx + 63) / 64, (g.ny + 3) / 4, (g.nz + chunk - 1) / chunk);
+}
+static int nblocks(const dim3 &d) { return (int)(d.x * d.y * d.z); }
+
+// Doubles of the reduction scratch: [0, flux) the block sums of k_flux (or of
+// k_update_div), [dt, dt + blocks) the CFL maxima of the aux pass, then the
+// second-level values of k_weno_items.
+int one_pass_flux_slots(const Geo &g, bool mixed) { return 5 * nblocks(flux_grid(g, flux_chunk(g, mixed))); }
+int one_pass_update_blocks(const Geo &g) { return nblocks(update_grid(g, update_chunk(g))); }
+
+static int item_segments(const Geo &g, int *wpt) {
+    const long nwords = (long)rec_per_row(g) * g.ny * g.nz;
+    long per = (nwords + 256L * kItemSeg - 1) / (256L * kItemSeg);
+    if (per < 1) per = 1;
+    *wpt = (int)per;
+    return (int)((nwords + 256 * per - 1) / (256 * per));
+}
+
+hipError_t launch_hot_items(st_solver *s) {
+    const Geo &g = s->g;
+    const long words = (long)hot_words(g) * g.sy * g.sz;
+    ST_DISPATCH(ST_GO(k_hot_bits, ST_T(R), 256, 0, dim3((unsigned)((words + 15) / 16)), dim3(256), g, s->kp,
+                      (const R *)s->w_aux, s->hot));
+    int wpt;
+    const int nseg = item_segments(g, &wpt);
+    ST_GO(k_hot_items, , 256, 0, dim3((unsigned)nseg), dim3(256), g, s->kp, (const uint64_t *)s->hot, s->hot_rec, s->hot_dirty, wpt,
+          s->fixlist, s->counters + 8);
+    return hipGetLastError();
+}
+
+hipError_t launch_flux(st_solver *s, void *fl, int stage) {
+    const Geo &g = s->g;
+    const bool sums = s->p.channel_case != 0, cons = s->p.conservative_viscous == 1;
+    // with the bulk sums the chunk is a function of the grid alone: they are
+    // grouped by workgroup, and a tuned chunk must not change results
+    const int chunk = s->visc_chunk > 0 && !sums ? (s->visc_chunk < kFluxMaxChunk ? s->visc_chunk : kFluxMaxChunk)
+                                               : flux_chunk(g, s->mixed);
+    const dim3 grid = flux_grid(g, chunk);
+    FluxArgs F{};
+    F.dx1 = s->dcsidx; F.dxs = s->dcsidxs; F.dx2 = s->dcsidx2;
+    F.dy1 = s->detady; F.dys = s->detadys; F.dy2 = s->detady2;
+    F.dz1 = s->dzitdz; F.dzs = s->dzitdzs; F.dz2 = s->dzitdz2;
+    F.xc = s->x; F.yc = s->y; F.zc = s->z; F.yn = s->yn;
+    F.eocx = s->eoc[0]; F.eocy = s->eoc[1];
+    F.dirty = s->hot_dirty;
+    F.w = s->w;
+    F.wallprop = s->wallprop;
+    F.partials = s->partials;
+    F.chunk = chunk;
+    F.last = stage == 2;
+    if (sums) s->force_nblk = nblocks(grid);
+#define ST_LAUNCH_FX(C_, S_) \
+    ST_DISPATCH(ST_GO(k_flux, ST_T(R, C_, S_), 256, kFluxWaves<R>, grid, dim3(kFluxTX, kFluxTY), g, s->kp, (R *)s->w_aux, (R *)fl, F))
+    if (cons && sums) ST_LAUNCH_FX(true, true);
+    else if (cons) ST_LAUNCH_FX(true, false);
+    else if (sums) ST_LAUNCH_FX(false, true);
+    else ST_LAUNCH_FX(false, false);
+#undef ST_LAUNCH_FX
+    return hipGetLastError();
+}
+
+hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt) {
+    const Geo &g = s->g;
+    ItemArgs A{};
+    for (int d = 0; d < 3; d++) A.eoc[d] = s->eoc[d];
+    A.metric[0] = s->dcsidx;
+    A.metric[1] = s->detady;
+    A.metric[2] = s->dzitdz;
+    A.rec = s->hot_rec;
+    A.list = s->fixlist;
+    A.counts = s->counters + 8;
+    A.nseg = item_segments(g, &A.wpt);
+    A.partials = s->partials;
+    A.nblk = s->force_nblk;
+    A.dtpart = s->dtpart;
+    A.ndt = dt ? aux_dt_blocks(g) : 0;
+    A.stage2 = s->stage2;
+    A.ticket = s->counters + 1;
+    A.ds = s->ds;
+    A.yn = s->yn;
+    A.rkr = s->rhork[stage];
+    A.rkg = s->gamrk[stage];
+    A.channel = s->p.channel_case != 0;
+    A.first = stage == 0;
+    // one workgroup per 8192 cells, at most one per CU (its register budget
+    // holds one wave per SIMD)
+    long nb = (long)((g.nint + 8191) / 8192);
+    nb = nb < 1 ? 1 : (nb > kItemBlocks ? kItemBlocks : nb);
+    ST_DISPATCH(ST_GO(k_weno_items, ST_T(R), 256, 0, dim3((unsigned)nb), dim3(256), g, s->kp, (const R *)s->w_aux, s->w,
+                      (R *)fl, A));
+    return hipGetLastError();
+}
+
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end) {
+    const Geo &g = s->g;
+    const bool fv = s->p.channel_case && s->p.theta_wall >= -1.0, o2 = s->p.conservative_viscous == 1;
+    UpdArgs U{};
+    U.dx1 = s->dcsidx; U.dy1 = s->detady; U.dz1 = s->dzitdz;
+    U.xc = s->x; U.yc = s->y; U.zc = s->z; U.yn = s->yn;
+    U.ds = s->ds;
+    U.rkr = s->rhork[stage];
+    U.rkg = s->gamrk[stage];
+    U.channel = s->p.channel_case;
+    U.chunk = update_chunk(g);
+    U.step_end = step_end ? 1 : 0;
+    U.partials = s->partials;
+    const dim3 grid = update_grid(g, U.chunk);
+#define ST_LAUNCH_UD(F_, O_)                                                                                  \
+    ST_DISPATCH(ST_GO(k_update_div, ST_T(R, F_, O_), 256, 0, grid, dim3(64, 4), g, s->kp, s->w, (R *)s->w_aux, \
+                      (const R *)fl_prev, (R *)fl, U))
+    if (fv && o2) ST_LAUNCH_UD(true, true);
+    else if (fv) ST_LAUNCH_UD(true, false);
+    else if (o2) ST_LAUNCH_UD(false, true);
+    else ST_LAUNCH_UD(false, false);
+#undef ST_LAUNCH_UD
+    return hipGetLastError();
+}
+
+}  // namespace st

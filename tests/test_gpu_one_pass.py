@@ -1,0 +1,102 @@
+"""The one-pass stage (st_stage.hip) at the sizes where it can go wrong,
+against the oracle: extents around its 32 x 8 tiles, 32-cell masks, 64-cell
+records and plane chunks, boundary cells of lowered stencil order on every
+kind of face, and work-item lists from empty over scattered (cells flagged in
+one, two and three directions, sensors in the ghost points included) to full.
+
+Tolerance: the trajectory bar of the parity tests, 1e-10 relative L2 per
+conserved variable over a few steps, which leaves four decades over the
+round-off the two orders of summation differ by; mixed precision 1e-5, its
+bar there.
+"""
+import numpy as np
+import pytest
+
+from helpers import interior, rel_l2
+from oracle import Oracle
+from streams_mi355x import PREC_MIXED, make_channel
+from streams_mi355x.cases import make_bl_box
+from streams_mi355x.params import params_copy
+from streams_mi355x.solver import ChannelSolver
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-10
+MIXED_TOL = 1e-5
+
+
+def _errors(params, grid, w0, steps, sensor_seed=None, precision=None, twin=None):
+    o = Oracle(params, grid)
+    o.w[:] = w0
+    o.init_run()
+    p = params
+    if precision is not None:
+        p = params_copy(params)
+        p.precision = precision
+    with ChannelSolver(p, twin or grid) as g:
+        g.copy_from_field(w0)
+        g.init_run()
+        if sensor_seed is not None:
+            s = np.random.default_rng(sensor_seed).uniform(0.0, 1.0, size=o.w_aux[7].shape)
+            o.w_aux[7][:] = s
+            g.set_aux(8, s)
+        o.advance(steps)
+        g.advance(steps)
+        w = g.copy_to_field()
+        assert np.array_equal(g.count_weno(), o.count_weno())
+    return [rel_l2(interior(w)[m], interior(o.w)[m]) for m in range(5)]
+
+
+@pytest.mark.parametrize("size", [(3, 3, 3), (31, 8, 5), (32, 9, 3), (33, 7, 34), (63, 16, 7), (64, 17, 8), (65, 24, 4),
+                                  (130, 3, 33)])
+@pytest.mark.parametrize("threshold", [1.01, 0.97, 0.5, -1.0])
+def test_channel_sizes_and_item_lists(size, threshold):
+    nx, ny, nz = size
+    c = make_channel(nx=nx, ny=ny, nz=nz, sensor_threshold=threshold, uniform_y=True, seed=nx)
+    if not np.isfinite(c.params.mu0):
+        c.params.mu0 = 1e-3  # three rows: the Re_tau relation has no half channel to integrate
+    seed = None if threshold < 0 else 5
+    errs = _errors(c.params, c.grid, c.w0, 2, sensor_seed=seed)
+    assert max(errs) <= TOL, errs
+
+
+@pytest.mark.parametrize("kw", [{"ep_order": 2}, {"ep_order": 4, "weno_scheme": 2}, {"weno_scheme": 1},
+                                {"correct_bound_ord": 0}, {"weno_version": 1}, {"theta_wall": 1.0},
+                                {"conservative_viscous": 1, "visc_model": 2}])
+def test_channel_schemes(kw):
+    c = make_channel(nx=45, ny=21, nz=10, sensor_threshold=0.9, uniform_y=True, seed=3, **kw)
+    errs = _errors(c.params, c.grid, c.w0, 3, sensor_seed=9)
+    assert max(errs) <= TOL, errs
+
+
+@pytest.mark.parametrize("size", [(40, 24, 16), (33, 9, 5), (67, 19, 6)])
+@pytest.mark.parametrize("conservative", [0, 1])
+@pytest.mark.parametrize("nr", [(0, 1, 0, 1, 0, 0), (0, 0, 0, 0, 0, 0), (2, 1, 6, 3, 0, 0)])
+def test_boundary_layer_faces(size, conservative, nr):
+    nx, ny, nz = size
+    c = make_bl_box(nx=nx, ny=ny, nz=nz, seed=2, conservative_viscous=conservative, bctags_nr=nr,
+                    sensor_threshold=0.95)
+    errs = _errors(c.params, c.grid, c.w0, 2, sensor_seed=4)
+    assert max(errs[:3] + errs[4:]) <= TOL, errs
+    assert errs[3] <= TOL, errs
+
+
+@pytest.mark.parametrize("size", [(31, 8, 5), (65, 17, 12)])
+@pytest.mark.parametrize("conservative", [0, 1])
+def test_mixed_sizes(size, conservative):
+    nx, ny, nz = size
+    c = make_channel(nx=nx, ny=ny, nz=nz, uniform_y=True, seed=1, conservative_viscous=conservative)
+    errs = _errors(c.params, c.grid, c.w0, 3, precision=PREC_MIXED)
+    assert max(errs) <= MIXED_TOL, errs
+
+
+@pytest.mark.parametrize("theta_wall", [-2.0, 1.0])
+def test_non_uniform_x_takes_the_separate_sweeps(theta_wall):
+    """The bulk sums by parts need one x metric; other grids keep the pass of
+    their own."""
+    c = make_channel(nx=36, ny=20, nz=8, seed=6, theta_wall=theta_wall)
+    f = 1.0 + 0.1 * np.sin(2.0 * np.pi * np.arange(36) / 36.0)
+    c.grid.dcsidx[:] *= f
+    c.grid.dcsidxs[:] *= f * f
+    errs = _errors(c.params, c.grid, c.w0, 3)
+    assert max(errs) <= TOL, errs
