@@ -27,6 +27,23 @@ __device__ __forceinline__ double wave_min(double v) {
     return v;
 }
 
+// Sum over the wave in lane 63, by DPP moves (shifts within the rows of 16
+// lanes, then row broadcasts): no LDS round trips.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_total(double v) {
+    v = dpp_add<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
+
 // Block sum of NV values in a fixed order; result valid in thread 0.
 __device__ __forceinline__ int flat_block() { return blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z); }
 __device__ __forceinline__ int flat_thread() { return threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z); }

@@ -220,7 +220,7 @@ size_t hot_rec_bytes(const Geo &g);
 size_t hot_dirty_bytes(const Geo &g);
 int one_pass_flux_slots(const Geo &g, bool mixed);
 int one_pass_update_blocks(const Geo &g);
-constexpr int kStage2Slots = 256 * 6;  // second-level values of k_weno_items
+constexpr int kStage2Slots = 512 * 6;  // second-level values of k_weno_items
 // the step's WENO masks and work items from w_aux(8)
 hipError_t launch_hot_items(st_solver *s);
 // the whole right-hand side but grad(div/3) and the WENO faces

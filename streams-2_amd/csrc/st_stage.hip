@@ -34,7 +34,7 @@ namespace st {
 // sector).
 constexpr int kRecWords = 8;
 constexpr int kItemSeg = 4096;       // list segments at most
-constexpr int kItemBlocks = 256;     // workgroups of the item kernel at most (one per CU)
+constexpr int kItemBlocks = 512;     // workgroups of the item kernel at most (two per CU)
 
 __host__ __device__ __forceinline__ int hot_words(const Geo &g) { return (g.rx + 63) / 64; }
 __host__ __device__ __forceinline__ int rec_per_row(const Geo &g) { return (g.nx + 63) / 64; }
@@ -801,24 +801,177 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFluxWaves<
 }
 
 // ============================================================ WENO items
-// Hybrid flux of one face in direction-aligned velocities (u normal, v and w
-// the tangential ones in the order of the eigenvector routines): the x
-// routines then serve all three directions, with the direction a property of
-// the lane.
-__device__ __forceinline__ void item_face(const KPar &P, const Pt (&q)[6], bool hot, int f, int e, int n, int dir,
-                                          double fh[5]) {
-    if (hot) {
-        weno_flux<0, 3>(P, q, e, fh);
-    } else {
-        Pc c[6];
-#pragma unroll
-        for (int s = 0; s < 6; s++) c[s] = pc_of(q[s]);
-        int lmax = P.lmax_base + e;
-        lmax = lmax < 1 ? 1 : lmax;
-        const int zlo = dir == 0 ? P.fzf[0] : (dir == 1 ? P.fzf[2] : P.fzf[4]);
-        const int zhi = dir == 0 ? P.fzf[1] : (dir == 1 ? P.fzf[3] : P.fzf[5]);
-        central_flux<0, 3, Pc, 0>(P, c, lmax, (f == 0 && zlo == 1) || (f == n && zhi == 1), fh);
+// A stencil point in direction-aligned velocities: n normal, a and b the
+// tangential ones in the order of the eigenvector routines, so that one code
+// serves all directions and the direction is a property of the lane.
+struct IP {
+    double r, n, a, b, t;
+};
+struct ItemConst {
+    double ea, eb, rg, gam;  // e = ea + eb T, gas constant, cp/(cp - R)
+    double ta, tb;           // T = ta + tb (h - |u|^2/2) of the Roe average
+    __device__ __forceinline__ double enthalpy(const IP &q) const {
+        return ea + (eb + rg) * q.t + 0.5 * (q.n * q.n + q.a * q.a + q.b * q.b);
     }
+};
+
+// Reconstruction from five values, v[2] the upwind cell (wenorec_1d,
+// kernels_cpu.F90:2526-2667, one side; orders 3 with Jiang-Shu or Z weights, 2,
+// 1).  The normalized weights alpha_k / sum alpha of alpha_k = d_k / (eps +
+// beta_k)^2 are taken over their common denominator, which leaves one
+// division of the eleven the quotients ask for.
+__device__ __forceinline__ double weno_side(double v0, double v1, double v2, double v3, double v4, int ord,
+                                            int version, double scale) {
+    if (ord >= 3) {
+        const double s0 = v0 - 2.0 * v1 + v2, s1 = v1 - 2.0 * v2 + v3, s2 = v2 - 2.0 * v3 + v4;
+        const double g0 = v0 - 4.0 * v1 + 3.0 * v2, g1 = v1 - v3, g2 = 3.0 * v2 - 4.0 * v3 + v4;
+        const double t = 13.0 / 12.0;
+        const double b0 = scale * (t * s0 * s0 + 0.25 * g0 * g0), b1 = scale * (t * s1 * s1 + 0.25 * g1 * g1),
+                     b2 = scale * (t * s2 * s2 + 0.25 * g2 * g2);
+        double n0, n1, n2;
+        if (version == 0) {
+            const double q0 = 0.000001 + b0, q1 = 0.000001 + b1, q2 = 0.000001 + b2;
+            const double m0 = q1 * q2, m1 = q0 * q2, m2 = q0 * q1;
+            n0 = 0.1 * m0 * m0;
+            n1 = 0.6 * m1 * m1;
+            n2 = 0.3 * m2 * m2;
+        } else {
+            // eps40 is the single-precision literal 1.e-35 of the reference
+            const double eps40 = (double)1.e-35f, tau = fabs(b0 - b2) + eps40;
+            const double q0 = b0 + eps40, q1 = b1 + eps40, q2 = b2 + eps40;
+            n0 = 0.1 * (b0 + tau) * (q1 * q2);
+            n1 = 0.6 * (b1 + tau) * (q0 * q2);
+            n2 = 0.3 * (b2 + tau) * (q0 * q1);
+        }
+        const double c0 = 2.0 * v0 - 7.0 * v1 + 11.0 * v2, c1 = -v1 + 5.0 * v2 + 2.0 * v3, c2 = 2.0 * v2 + 5.0 * v3 - v4;
+        return (n0 * c0 + n1 * c1 + n2 * c2) / (6.0 * (n0 + n1 + n2));
+    }
+    if (ord == 2) {
+        const double d0 = v2 - v1, d1 = v3 - v2;
+        const double q0 = 0.000001 + scale * (d0 * d0), q1 = 0.000001 + scale * (d1 * d1);
+        const double n0 = q1 * q1, n1 = 2.0 * (q0 * q0);
+        return (n0 * (3.0 * v2 - v1) + n1 * (v2 + v3)) / (2.0 * (n0 + n1));
+    }
+    return v2;
+}
+
+// Characteristic WENO flux of the face between q[2] and q[3] (Roe average,
+// eigenvectors and local Lax-Friedrichs split of kernels_cpu.F90:619-682,
+// 2728-2782, 3013-3089).  The projections of a point on the two acoustic
+// fields and the entropy field share K = (b1 - b2 u.u_l + b2 H_l)/2: they are
+// K +- (un - un_l)/(2c) and 1 - 2K; wc = rho s - e p and gc = rho un s + n p then
+// give the conserved and the flux component of any field.
+__device__ __forceinline__ void weno_face(const KPar &P, const ItemConst &C, const IP (&q)[6], int eoc, double fh[5]) {
+    const double hA = C.enthalpy(q[2]), hB = C.enthalpy(q[3]);
+    const double r = sqrt(q[3].r / q[2].r), rp1 = 1.0 / (r + 1.0);
+    const double un = (r * q[3].n + q[2].n) * rp1, ta = (r * q[3].a + q[2].a) * rp1, tb = (r * q[3].b + q[2].b) * rp1;
+    const double h = (r * hB + hA) * rp1;
+    const double qq = 0.5 * (un * un + ta * ta + tb * tb);
+    const double tt = C.ta + C.tb * (h - qq);
+    const double gm1 = C.gam - 1.0, prho = tt * C.rg, cc = C.gam * prho;
+    const double c = sqrt(cc), ci = 1.0 / c;
+    const double etot = h - prho;
+    const double b2 = gm1 * ci * ci, b3 = etot - prho / gm1, b1 = prho * ci * ci - b2 * (etot - 2.0 * qq);
+    double ev0 = -1.0, ev1 = -1.0, ev4 = -1.0;
+    double K[6];
+    const int ws = P.weno_scheme;
+#pragma unroll
+    for (int l = 0; l < 6; l++) {
+        K[l] = 0.5 * (b1 + b2 * (C.enthalpy(q[l]) - (un * q[l].n + ta * q[l].a + tb * q[l].b)));
+        if (l < 3 - ws || l > 2 + ws) continue;
+        const double cl = sqrt(C.gam * C.rg * q[l].t);
+        ev0 = fmax(fabs(q[l].n - cl), ev0);
+        ev1 = fmax(fabs(q[l].n), ev1);
+        ev4 = fmax(fabs(q[l].n + cl), ev4);
+    }
+    int ord = ws + eoc;
+    if (ord < 1) ord = 1;
+    const double u0_2 = P.u0 * P.u0, r2u2 = P.rho0 * P.rho0 * u0_2;
+    const double sc1 = 1.0 / r2u2, sc2 = 1.0 / (r2u2 * u0_2);
+#pragma unroll
+    for (int m = 0; m < 5; m++) fh[m] = 0.0;
+    // one field per iteration, not unrolled (instruction cache): its
+    // projection is al + be K + la un_l + xa a_l + xb b_l
+#pragma unroll 1
+    for (int m = 0; m < 5; m++) {
+        double al, be, la = 0.0, xa = 0.0, xb = 0.0, en, ee, ev = ev1, scale = sc1;
+        double e0 = 1.0, e1 = un, e2 = ta, e3 = tb, e4;  // right eigenvector
+        if (m == 0 || m == 4) {
+            const double sg = m == 0 ? 0.5 : -0.5;
+            al = sg * ci * un;
+            be = 1.0;
+            la = -sg * ci;
+            en = -0.5 * b2 * un - sg * ci;
+            ee = 0.5 * b2;
+            ev = m == 0 ? ev0 : ev4;
+            e1 = un - 2.0 * sg * c;
+            e4 = h - 2.0 * sg * un * c;
+        } else if (m == 1) {
+            al = 1.0;
+            be = -2.0;
+            en = b2 * un;
+            ee = -b2;
+            e4 = b3;
+        } else {
+            al = m == 2 ? -ta : -tb;
+            be = 0.0;
+            en = ee = 0.0;
+            xa = m == 2 ? 1.0 : 0.0;
+            xb = m == 2 ? 0.0 : 1.0;
+            scale = sc2;
+            e0 = e1 = 0.0;
+            e2 = xa;
+            e3 = xb;
+            e4 = m == 2 ? ta : tb;
+        }
+        double gp[6], gn[6];
+#pragma unroll
+        for (int l = 0; l < 6; l++) {
+            const IP &x = q[l];
+            const double s = al + be * K[l] + la * x.n + xa * x.a + xb * x.b;
+            const double pp = x.r * x.t * C.rg;
+            const double wc = x.r * s - ee * pp, gc = x.r * x.n * s + en * pp;
+            gp[l] = 0.5 * (gc + ev * wc);
+            gn[l] = gc - gp[l];
+        }
+        const double fi = weno_side(gp[0], gp[1], gp[2], gp[3], gp[4], ord, P.weno_version, scale) +
+                          weno_side(gn[5], gn[4], gn[3], gn[2], gn[1], ord, P.weno_version, scale);
+        fh[0] += e0 * fi;
+        fh[1] += e1 * fi;
+        fh[2] += e2 * fi;
+        fh[3] += e3 * fi;
+        fh[4] += e4 * fi;
+    }
+}
+
+// Central KEEP flux of the same face with half width lm (kernels_cpu.F90:466-618).
+__device__ __forceinline__ void central_face(const KPar &P, const ItemConst &C, const IP (&q)[6], int lm, bool zero,
+                                             double fh[5]) {
+    double f0 = 0.0, f1 = 0.0, f2 = 0.0, f3 = 0.0, f4 = 0.0, f5 = 0.0;
+#pragma unroll
+    for (int l = 1; l <= 3; l++) {
+        const double v3 = P.cd1tab[2][l - 1], v2 = P.cd1tab[1][l - 1], v1 = P.cd1tab[0][l - 1];
+        const double c = l > lm ? 0.0 : (lm >= 3 ? v3 : (lm == 2 ? v2 : v1));
+#pragma unroll
+        for (int m = 0; m < l; m++) {
+            const IP &A = q[2 - m], &B = q[2 - m + l];
+            const double pA = A.r * A.t * C.rg, pB = B.r * B.t * C.rg;
+            const double uv = c * (A.n + B.n) * (A.r + B.r);
+            f0 += uv;
+            f1 += uv * (A.n + B.n);
+            f2 += uv * (A.a + B.a);
+            f3 += uv * (A.b + B.b);
+            f4 += uv * (2.0 * C.ea + C.eb * (A.t + B.t) + A.n * B.n + A.a * B.a + A.b * B.b) +
+                  4.0 * c * (A.n * pB + B.n * pA);
+            f5 += c * (pA + pB);
+        }
+    }
+    const double w = zero ? 0.0 : 0.25;
+    fh[0] = 2.0 * w * f0;
+    fh[1] = w * f1 + f5;
+    fh[2] = w * f2;
+    fh[3] = w * f3;
+    fh[4] = w * f4;
 }
 
 struct ItemArgs {
@@ -847,7 +1000,11 @@ struct ItemArgs {
 // order and stores, so a cell is written once and the result does not depend
 // on the schedule.  A wave takes 64 items and owns the cells that start in
 // the first 62.  All directions share one launch, and every face is hybrid
-// per lane; bound by the latency of the scattered stencil loads.
+// per lane; bound by the latency of the scattered stencil loads and, where
+// WENO cells are many, by the arithmetic of the faces.  On 384 x 128 x 96 with
+// a shock (1.6 % WENO faces) 69 us a stage, with the general characteristic
+// routines of st_flux.h at one wave per SIMD 125; on 512 x 256 x 256 after 25
+// steps 0.32 ms for 0.43.
 //
 // The workgroups then finish the reductions of the stage (two levels, fixed
 // order): the bulk sums of k_flux with the items' changes, giving b1, b2,
@@ -860,8 +1017,7 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
                                                   R *__restrict__ fl, ItemArgs A) {
     __shared__ int pre[kItemSeg + 1];
     __shared__ int wsum[4];
-    __shared__ double lds[4][5];
-    __shared__ double ldm[4];
+    __shared__ double lds[4][6];
     __shared__ bool last;
     const int t = threadIdx.x, lane = t & 63;
     double red[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -907,6 +1063,13 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
             code = d << 24 | (int)((rc[0] >> (i0 & 63)) & 1ull) << 26 | (int)((rc[1] >> (i0 & 63)) & 1ull) << 27;
         }
     };
+    ItemConst C;
+    C.eb = cvc(P, 0);
+    C.ea = P.t0 * (cvc(P, P.indx_cp_r + 1) - C.eb);
+    C.rg = P.rgas0;
+    C.gam = cpc(P, 0) / (cpc(P, 0) - P.rgas0);
+    C.tb = 1.0 / cpc(P, 0);
+    C.ta = P.t0 - cpc(P, P.indx_cp_r + 1) * P.t0 * C.tb;
     const int wave = (blockIdx.x * blockDim.x + t) >> 6;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     for (int base = wave * 62; base < total; base += nwaves * 62) {
@@ -916,12 +1079,10 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
         const bool lo_hot = (code >> 26) & 1, hi_hot = (code >> 27) & 1;
         const bool work = cell >= 0 && (lo_hot || hi_hot);
         double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        int j = 1;
         if (work) {
             const int dir = (code >> 24) & 3;
             const int i = cell % g.nx + 1, jk = cell / g.nx;
-            j = jk % g.ny + 1;
-            const int k = jk / g.ny + 1;
+            const int j = jk % g.ny + 1, k = jk / g.ny + 1;
             const int c = dir == 0 ? i : (dir == 1 ? j : k);
             const int n = dir == 0 ? g.nx : (dir == 1 ? g.ny : g.nz);
             const int stride = dir == 0 ? 1 : (dir == 1 ? g.sx : g.sxy);
@@ -929,21 +1090,24 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
             const double *met = dir == 0 ? A.metric[0] : (dir == 1 ? A.metric[1] : A.metric[2]);
             const size_t on = (size_t)(1 + dir) * nv, o1 = (dir == 0 ? 2 : 1) * nv, o2 = (dir == 2 ? 2 : 3) * nv;
             const int b0 = gidx(g, i, j, k);
+            IP q[7];
             // every load of the stencil before any arithmetic
-            double raw[7][6];
+            if constexpr (sizeof(R) == sizeof(double)) {
 #pragma unroll
-            for (int s = 0; s < 7; s++) {
-                const int a = b0 + (s - 3) * stride;
-                if constexpr (sizeof(R) == sizeof(double)) {
-                    raw[s][0] = wa[a];
-                    raw[s][1] = wa[on + a];
-                    raw[s][2] = wa[o1 + a];
-                    raw[s][3] = wa[o2 + a];
-                    raw[s][4] = wa[4 * nv + a];
-                    raw[s][5] = wa[5 * nv + a];
-                } else {
-                    // the mixed form stores w_aux in FP32: the FP64 primitives
-                    // of w, periodic neighbours from their images
+                for (int s = 0; s < 7; s++) {
+                    const int a = b0 + (s - 3) * stride;
+                    q[s].r = wa[a];
+                    q[s].n = wa[on + a];
+                    q[s].a = wa[o1 + a];
+                    q[s].b = wa[o2 + a];
+                    q[s].t = wa[5 * nv + a];
+                }
+            } else {
+                // the mixed form stores w_aux in FP32: the FP64 primitives of
+                // w, periodic neighbours from their images
+                double re[7];
+#pragma unroll
+                for (int s = 0; s < 7; s++) {
                     int pi = i, pj = j, pk = k;
                     if (dir == 0) pi += s - 3;
                     else if (dir == 1) pj += s - 3;
@@ -952,52 +1116,55 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
                     if (P.periodic[1]) pj = pj < 1 ? pj + g.ny : (pj > g.ny ? pj - g.ny : pj);
                     if (P.periodic[2]) pk = pk < 1 ? pk + g.nz : (pk > g.nz ? pk - g.nz : pk);
                     const int src = gidx(g, pi, pj, pk);
-                    raw[s][0] = w[src];
-                    raw[s][1] = w[on + src];
-                    raw[s][2] = w[o1 + src];
-                    raw[s][3] = w[o2 + src];
-                    raw[s][4] = w[4 * nv + src];
-                    raw[s][5] = 0.0;
+                    q[s].r = w[src];
+                    q[s].n = w[on + src];
+                    q[s].a = w[o1 + src];
+                    q[s].b = w[o2 + src];
+                    re[s] = w[4 * nv + src];
+                }
+#pragma unroll
+                for (int s = 0; s < 7; s++) {
+                    const double ri = 1.0 / q[s].r;
+                    q[s].n *= ri;
+                    q[s].a *= ri;
+                    q[s].b *= ri;
+                    const double qq = 0.5 * (q[s].n * q[s].n + q[s].a * q[s].a + q[s].b * q[s].b);
+                    q[s].t = temperature_from_e(P, re[s] / q[s].r - qq, 0.0);
                 }
             }
             const int elo = eoc[c - 1], ehi = eoc[c];
             const double mt = met[c - 1];
-            Pt q[7];
-#pragma unroll
-            for (int s = 0; s < 7; s++) {
-                if constexpr (sizeof(R) == sizeof(double)) {
-                    q[s] = make_pt(raw[s][0], raw[s][1], raw[s][2], raw[s][3], raw[s][4], raw[s][5], P.rgas0, true);
-                } else {
-                    const double rho = raw[s][0], rhoe = raw[s][4];
-                    const double ri = 1.0 / rho;
-                    const double uu = raw[s][1] * ri, vv = raw[s][2] * ri, ww = raw[s][3] * ri;
-                    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-                    const double tt = temperature_from_e(P, rhoe / rho - qq, 0.0);
-                    const double pp = rho * tt * P.rgas0;
-                    q[s] = make_pt(rho, uu, vv, ww, (rhoe + pp) / rho, tt, P.rgas0, true);
-                }
-            }
+            const int zlo = dir == 0 ? P.fzf[0] : (dir == 1 ? P.fzf[2] : P.fzf[4]);
+            const int zhi = dir == 0 ? P.fzf[1] : (dir == 1 ? P.fzf[3] : P.fzf[5]);
             // WENO face first (the lower one where it has one): the lanes of a
             // wave then run the WENO branch together
             const bool alo = lo_hot || !hi_hot;
-            double fa[5], fb[5];
+            auto sel = [](bool c, const IP &x, const IP &y) {
+                return IP{c ? x.r : y.r, c ? x.n : y.n, c ? x.a : y.a, c ? x.b : y.b, c ? x.t : y.t};
+            };
+            // the window of the first face and the point the other one adds
+            IP qw[6], ex = sel(alo, q[6], q[0]);
+#pragma unroll
+            for (int s = 0; s < 6; s++) qw[s] = sel(alo, q[s], q[s + 1]);
+            double x[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll 1
             for (int s2 = 0; s2 < 2; s2++) {
                 const bool lo = (s2 == 0) == alo;
-                Pt qw[6];
-#pragma unroll
-                for (int s = 0; s < 6; s++) qw[s] = lo ? q[s] : q[s + 1];
                 double fh[5];
-                item_face(P, qw, lo ? lo_hot : hi_hot, lo ? c - 1 : c, lo ? elo : ehi, n, dir, fh);
+                const int eo = lo ? elo : ehi;
+                if (lo ? lo_hot : hi_hot) weno_face(P, C, qw, eo, fh);
+                else
+                    central_face(P, C, qw, max(P.lmax_base + eo, 1),
+                                 lo ? c == 1 && zlo == 1 : c == n && zhi == 1, fh);
+                const double sg = lo ? -mt : mt;
 #pragma unroll
-                for (int m = 0; m < 5; m++) {
-                    if (lo) fa[m] = fh[m];
-                    else fb[m] = fh[m];
-                }
+                for (int m = 0; m < 5; m++) x[m] += sg * fh[m];
+                IP nw[6];
+#pragma unroll
+                for (int s = 0; s < 6; s++) nw[s] = sel(alo, s < 5 ? qw[s + 1] : ex, s > 0 ? qw[s - 1] : ex);
+#pragma unroll
+                for (int s = 0; s < 6; s++) qw[s] = nw[s];
             }
-            double x[5];
-#pragma unroll
-            for (int m = 0; m < 5; m++) x[m] = (fb[m] - fa[m]) * mt;
             d[0] = x[0];
             d[4] = x[4];
             d[1] = dir == 0 ? x[1] : x[2];
@@ -1037,6 +1204,7 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
         }
     }
     if (!A.channel && A.ndt == 0) return;
+    // this workgroup's slices of the block sums and of the CFL maxima
     double mx = 0.0;
     if (A.channel) {
         const int per = (A.nblk + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -1045,58 +1213,69 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
 #pragma unroll
             for (int q = 0; q < 5; q++) red[q] += A.partials[(size_t)b * 5 + q];
         }
-        block_sum<5>(red, lds);
     }
     if (A.ndt) {
         const int per = (A.ndt + (int)gridDim.x - 1) / (int)gridDim.x;
         const int b0 = (int)blockIdx.x * per, b1 = min(b0 + per, A.ndt);
         for (int b = b0 + t; b < b1; b += 256) mx = fmax(mx, A.dtpart[b]);
+    }
+    auto block_reduce = [&]() {  // totals in every thread
+#pragma unroll
+        for (int q = 0; q < 5; q++) red[q] = wave_total(red[q]);
         mx = wave_max(mx);
-        if (lane == 0) ldm[t >> 6] = mx;
+        if (lane == 63) {
+#pragma unroll
+            for (int q = 0; q < 5; q++) lds[t >> 6][q] = red[q];
+        }
+        if (lane == 0) lds[t >> 6][5] = mx;
         __syncthreads();
-        mx = fmax(fmax(ldm[0], ldm[1]), fmax(ldm[2], ldm[3]));
-    }
-    if (t == 0) {
 #pragma unroll
-        for (int q = 0; q < 5; q++) A.stage2[blockIdx.x * 6 + q] = red[q];
-        A.stage2[blockIdx.x * 6 + 5] = mx;
+        for (int q = 0; q < 5; q++) red[q] = (lds[0][q] + lds[1][q]) + (lds[2][q] + lds[3][q]);
+        mx = fmax(fmax(lds[0][5], lds[1][5]), fmax(lds[2][5], lds[3][5]));
+    };
+    block_reduce();
+    if (gridDim.x > 1) {
+        if (t == 0) {
+#pragma unroll
+            for (int q = 0; q < 5; q++) A.stage2[blockIdx.x * 6 + q] = red[q];
+            A.stage2[blockIdx.x * 6 + 5] = mx;
+            __threadfence();
+            last = atomicAdd(A.ticket, 1) == (int)gridDim.x - 1;
+        }
+        __syncthreads();
+        if (!last) return;
         __threadfence();
-        last = atomicAdd(A.ticket, 1) == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    // gridDim.x <= 256: one second-level value per thread, past the
-    // non-coherent caches, added by the same fixed tree
-    double v[6];
+        // the second-level values, past the non-coherent caches, by the same tree
+        mx = 0.0;
 #pragma unroll
-    for (int q = 0; q < 6; q++)
-        v[q] = t < (int)gridDim.x
-                   ? __hip_atomic_load(&A.stage2[t * 6 + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                   : 0.0;
-    mx = wave_max(v[5]);
-    if (lane == 0) ldm[t >> 6] = mx;
-    double r5[5] = {v[0], v[1], v[2], v[3], v[4]};
-    block_sum<5>(r5, lds);  // its barrier also covers ldm
+        for (int q = 0; q < 5; q++) red[q] = 0.0;
+        for (int b = t; b < (int)gridDim.x; b += 256) {
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+                red[q] += __hip_atomic_load(&A.stage2[b * 6 + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            mx = fmax(mx, __hip_atomic_load(&A.stage2[b * 6 + 5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        }
+        block_reduce();  // (the barrier after the ticket separates the two uses of lds)
+        if (t == 0) *A.ticket = 0;
+    }
     if (t == 0) {
-        *A.ticket = 0;
         DevScalars *ds = A.ds;
         if (A.ndt) {
-            const double dt_min = 1.0 / fmax(fmax(ldm[0], ldm[1]), fmax(ldm[2], ldm[3]));
+            const double dt_min = 1.0 / mx;
             ds->dt = P.cfl * dt_min;
         }
         if (A.channel) {
             const double rhodt = A.rkr * ds->dt, gamdt = A.rkg * ds->dt;
-            double b1 = -gamdt * r5[0], b2 = -gamdt * r5[1];
+            double b1 = -gamdt * red[0], b2 = -gamdt * red[1];
             if (A.rkr != 0.0) {
                 b1 -= rhodt * ds->rhs_sum[0];
                 b2 -= rhodt * ds->rhs_sum[1];
             }
             b1 = b1 / P.volchan;
             b2 = b2 / P.volchan;
-            ds->rhs_sum[0] = r5[0];
-            ds->rhs_sum[1] = r5[1];
-            const double b3 = r5[2] / P.volchan, b4 = r5[3] / P.volchan, b5 = r5[4] / P.volchan;
+            ds->rhs_sum[0] = red[0];
+            ds->rhs_sum[1] = red[1];
+            const double b3 = red[2] / P.volchan, b4 = red[3] / P.volchan, b5 = red[4] / P.volchan;
             ds->dpdx = (A.first ? 0.0 : ds->dpdx) + b2;
             ds->rhobulk = b3;
             ds->ubulk = b4 / b3;
@@ -1106,9 +1285,10 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
         }
     }
 }
+// two waves per SIMD: the scattered loads of one batch overlap the other's work
 template <typename R>
-__global__ __launch_bounds__(256) void k_weno_items(Geo g, KPar P, const R *__restrict__ wa,
-                                                    const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_weno_items(
+    Geo g, KPar P, const R *__restrict__ wa, const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
     k_weno_items_body<R>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, wa, w, fl, A);
 }
 
@@ -1393,11 +1573,10 @@ hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt) {
     A.rkg = s->gamrk[stage];
     A.channel = s->p.channel_case != 0;
     A.first = stage == 0;
-    // one workgroup per 8192 cells, at most one per CU (its register budget
-    // holds one wave per SIMD)
+    // one workgroup per 8192 cells, at most what the chip holds at once
     long nb = (long)((g.nint + 8191) / 8192);
     nb = nb < 1 ? 1 : (nb > kItemBlocks ? kItemBlocks : nb);
-    ST_DISPATCH(ST_GO(k_weno_items, ST_T(R), 256, 0, dim3((unsigned)nb), dim3(256), g, s->kp, (const R *)s->w_aux, s->w,
+    ST_DISPATCH(ST_GO(k_weno_items, ST_T(R), 256, 2, dim3((unsigned)nb), dim3(256), g, s->kp, (const R *)s->w_aux, s->w,
                       (R *)fl, A));
     return hipGetLastError();
 }
