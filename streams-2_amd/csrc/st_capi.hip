@@ -291,20 +291,23 @@ struct TimeScope {
 bool fp64_sensor(const st_solver *s) { return s->mixed && s->p.conservative_viscous != 1; }
 
 // one RK stage of rk_sync in four launches (st_stage.hip), plus the step's
-// WENO masks at its first stage; end: the last stage of a st_advance step
-int stage_one_pass(st_solver *s, int istep, bool end) {
+// WENO masks at its first stage; end: the last stage of a st_advance step;
+// last: no step of the same call follows, so what its third stage leaves is
+// the caller's to read
+int stage_one_pass(st_solver *s, int istep, bool end, bool last) {
     using namespace st;
     void *fprev = s->F[s->cur], *fcur = s->F[s->cur ^ 1];
     const Geo &g = s->g;
     const bool dt = istep == 0 && s->dt_in_stage && s->p.cfl > 0;
     if (istep == 0) TIMED(ST_K_WENO_FIX, launch_hot_items(s));
-    TIMED(ST_K_AUX, launch_aux(s, 1 - g.ng, g.nx + g.ng, 1 - g.ng, g.ny + g.ng, 1 - g.ng, g.nz + g.ng, true, dt, true));
+    TIMED(ST_K_AUX, launch_aux(s, 1 - g.ng, g.nx + g.ng, 1 - g.ng, g.ny + g.ng, 1 - g.ng, g.nz + g.ng, true, dt, true,
+                               s->has_nr || (last && istep == 2)));
     if (istep == 0) s->dt_in_stage = false;
     TIMED(ST_K_EULER_XY, launch_flux(s, fcur, istep));
     if (istep == 2 && fp64_sensor(s)) TIMED(ST_K_SENSOR, launch_sensor_refine(s, false, true));
     TIMED(ST_K_WENO_FIX, launch_weno_items(s, fcur, istep, dt));
     if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur));
-    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end));
+    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end, last));
     if (s->p.channel_case && s->p.theta_wall >= -1.0)
         TIMED(ST_K_FORCE_VAR, launch_force_var(s, one_pass_update_blocks(g)));
     if (s->recyc) TIMED(ST_K_BC, launch_inflow_draws(s));
@@ -378,11 +381,12 @@ int stage(st_solver *s, int istep) {
     return ST_OK;
 }
 
-// end: the step of st_advance, which also moves time and the step counter
-int do_rk_sync(st_solver *s, bool end) {
+// end: the step of st_advance, which also moves time and the step counter;
+// last: no step of the same call follows
+int do_rk_sync(st_solver *s, bool end, bool last) {
     const bool one = st::one_pass_stage(s);
     for (int istep = 0; istep < 3; istep++) {
-        int rc = one ? stage_one_pass(s, istep, end && istep == 2) : stage(s, istep);
+        int rc = one ? stage_one_pass(s, istep, end && istep == 2, last) : stage(s, istep);
         if (rc) return rc;
     }
     if (end && !one) TIMED(ST_K_STEP_END, st::launch_step_end(s));
@@ -1187,7 +1191,7 @@ int st_rk_sync(st_solver *s) {
         if (rc) return rc;
         return rk_sync_pieces(s, s->hs->dt);
     }
-    return do_rk_sync(s, false);
+    return do_rk_sync(s, false, true);
 }
 
 int st_advance(st_solver *s, int32_t nsteps) {
@@ -1215,7 +1219,7 @@ int st_advance(st_solver *s, int32_t nsteps) {
             // therefore takes the reduction
             s->dt_in_stage = true;
         }
-        int rc = do_rk_sync(s, true);
+        int rc = do_rk_sync(s, true, n + 1 == nsteps);
         if (rc) return rc;
     }
     return ST_OK;

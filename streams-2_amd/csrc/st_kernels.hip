@@ -548,6 +548,10 @@ __global__ void k_rng_reset(Win31 seeded, uint32_t *__restrict__ win2, int *__re
 // one block maximum per workgroup: the first stage of a step that recomputes
 // dt evaluates the same primitives of the same w as compute_dt's own
 // compute_aux(central=1) at the start of the step.
+// Bound by HBM: 40 B read and 56 B written a point.  image & 2 leaves the
+// enthalpy out (8 B of 96): the one-pass stage forms it from the other
+// primitives, so only the last stage of a call (whose w_aux the caller can
+// read) and bc_nr want it.
 template <typename R, bool DT = false>
 __device__ __forceinline__ void k_aux_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P, const double *__restrict__ w, R *__restrict__ wa,
                                              int i0, int ni, int j0, int nj, int k0, int nk, int image,
@@ -581,7 +585,7 @@ __device__ __forceinline__ void k_aux_body(const dim3 blockIdx, const dim3 gridD
     }
     if (act) {
         int is = i, js = j, ks = k;
-        if (image) {
+        if (image & 1) {
             if (P.periodic[0]) is = i < 1 ? i + g.nx : (i > g.nx ? i - g.nx : i);
             if (P.periodic[1]) js = j < 1 ? j + g.ny : (j > g.ny ? j - g.ny : j);
             if (P.periodic[2]) ks = k < 1 ? k + g.nz : (k > g.nz ? k - g.nz : k);
@@ -600,7 +604,7 @@ __device__ __forceinline__ void k_aux_body(const dim3 blockIdx, const dim3 gridD
         wa[nv + d] = R(uu);
         wa[2 * nv + d] = R(vv);
         wa[3 * nv + d] = R(ww);
-        wa[4 * nv + d] = R((rhoe + pp) / rho);
+        if (!(image & 2)) wa[4 * nv + d] = R((rhoe + pp) / rho);
         wa[5 * nv + d] = R(tt);
         wa[6 * nv + d] = R(mu);
         if constexpr (sizeof(R) != sizeof(double)) wa[10 * nv + d] = R(pp - P.p_ref);
@@ -629,7 +633,8 @@ __device__ __forceinline__ void k_aux_body(const dim3 blockIdx, const dim3 gridD
         const int d = gidx(g, i, j, k);
         const size_t nv = g.nvol;
 #pragma unroll
-        for (int m = 0; m < 7; m++) wa[m * nv + d] = R(0.0);
+        for (int m = 0; m < 7; m++)
+            if (m != 4 || !(image & 2)) wa[m * nv + d] = R(0.0);
         if constexpr (sizeof(R) != sizeof(double)) wa[10 * nv + d] = R(0.0);
     }
     if constexpr (DT) {
@@ -3324,7 +3329,7 @@ int aux_dt_blocks(const Geo &g) { return (int)((aux_lanes(g) + 255) / 256); }
 int update_blocks(const Geo &g) { return cell_blocks(g); }
 
 hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image, bool dt,
-                      bool defer_dt) {
+                      bool defer_dt, bool enthalpy) {
     const int ni = i1 - i0 + 1, nj = j1 - j0 + 1, nk = k1 - k0 + 1;
     if (ni <= 0 || nj <= 0 || nk <= 0) return hipSuccess;
     const size_t tot = aux_whole_box(s->g, i0, ni, j0, nj, k0, nk) ? aux_lanes(s->g)
@@ -3332,7 +3337,7 @@ hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int 
     const unsigned nblk = (unsigned)((tot + 255) / 256);
 #define ST_LAUNCH_AUX(D_)                                                                                          \
     ST_DISPATCH(ST_GO(k_aux, ST_T(R, D_), 256, 0, dim3(nblk), dim3(256), s->g, s->kp, s->w, (R *)s->w_aux, i0, ni,  \
-                      j0, nj, k0, nk, image ? 1 : 0, s->dcsidx, s->detady, s->dzitdz, s->dcsidxs, s->detadys,        \
+                      j0, nj, k0, nk, (image ? 1 : 0) | (enthalpy ? 0 : 2), s->dcsidx, s->detady, s->dzitdz, s->dcsidxs, s->detadys,        \
                       s->dzitdzs, defer_dt ? s->dtpart : s->partials))
     if (dt && s->p.cfl > 0) ST_LAUNCH_AUX(true);
     else ST_LAUNCH_AUX(false);

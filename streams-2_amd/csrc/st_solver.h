@@ -165,9 +165,10 @@ hipError_t launch_fill_periodic(st_solver *s, double *arr, int nv);
 hipError_t launch_fill_periodic_aux(st_solver *s, int var);
 hipError_t launch_extrapolate_aux(st_solver *s, int var);
 // dt also takes the CFL reduction: its block maxima to dt itself, or with
-// defer_dt to dtpart, for launch_weno_items to finish
+// defer_dt to dtpart, for launch_weno_items to finish; enthalpy: w_aux(5) has
+// a reader before it is formed again
 hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image,
-                      bool dt = false, bool defer_dt = false);
+                      bool dt = false, bool defer_dt = false, bool enthalpy = true);
 int aux_dt_blocks(const Geo &g);  // block maxima of an aux pass over the ghosted box
 hipError_t launch_wall_ghosts(st_solver *s);
 // physical ghosts of every non-periodic face in the order xmin..zmax
@@ -228,7 +229,7 @@ hipError_t launch_flux(st_solver *s, void *fl, int stage);
 // WENO faces; bulk sums of force_rhs and, with dt, the CFL step finished
 hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt);
 // grad(div/3), update_flux, update_field, wall ghosts; the end of the step
-hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end);
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last);
 hipError_t launch_dt(st_solver *s);
 hipError_t launch_step_end(st_solver *s);
 hipError_t launch_residual(st_solver *s);

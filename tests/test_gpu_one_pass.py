@@ -100,3 +100,24 @@ def test_non_uniform_x_takes_the_separate_sweeps(theta_wall):
     c.grid.dcsidxs[:] *= f * f
     errs = _errors(c.params, c.grid, c.w0, 3)
     assert max(errs) <= TOL, errs
+
+
+@pytest.mark.parametrize("make", [lambda: make_channel(nx=34, ny=11, nz=7, seed=8),
+                                  lambda: make_channel(nx=34, ny=11, nz=7, seed=8, theta_wall=1.0),
+                                  lambda: make_bl_box(nx=40, ny=17, nz=6, seed=2)])
+@pytest.mark.parametrize("precision", [0, PREC_MIXED])
+def test_one_call_leaves_what_single_steps_leave(make, precision):
+    """Within a call, what no later stage reads is not stored; the arrays a
+    caller can read afterwards are those of step-by-step calls, bit for bit."""
+    c = make()
+    c.params.precision = precision
+    got = []
+    for calls in ([3], [1, 1, 1]):
+        with ChannelSolver(c.params, c.grid) as g:
+            g.copy_from_field(c.w0)
+            g.init_run()
+            for n in calls:
+                g.advance(n)
+            got.append([g.copy_to_field(), g.get_fl()] + [g.get_aux(v) for v in range(1, 11)])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b, equal_nan=True)
