@@ -255,6 +255,7 @@ void free_all(st_solver *s) {
         (void)hipFree(p);
     }
     if (s->hs && !s->borrowed_hs) (void)hipHostFree(s->hs);
+    st::stage_destroy(s->own_stage);
     if (s->own_stream && s->stream) (void)hipStreamDestroy(s->stream);
 }
 
@@ -510,6 +511,7 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
         s->arena_hi = mem->arena + off;
         s->hs = mem->hs;
         s->borrowed_hs = true;
+        s->stage = mem->stage;
     } else {
         for (int q = 0; q < kNArrays && ea == hipSuccess; q++) ea = hipMalloc(dst[q], n[q] > 0 ? n[q] : 8);
         if (ea == hipSuccess) ea = hipHostMalloc((void **)&s->hs, sizeof(st::DevScalars), hipHostMallocDefault);
@@ -518,6 +520,8 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
             delete s;
             return fail(ST_ERR_NOMEM, std::string("device allocation failed: ") + hipGetErrorString(ea));
         }
+        st::stage_create(s->own_stage, 5 * sizeof(double) * (size_t)g.nvol);
+        s->stage = &s->own_stage;
     }
     s->dtpart = s->partials + partial_head(g, s->mixed);
     s->stage2 = s->dtpart + st::aux_dt_blocks(g);
@@ -575,39 +579,6 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
     }
     *out = s;
     return ST_OK;
-}
-
-// nvars ghosted variables of es-byte values between the solver's pitched
-// layout (device) and the reference layout (host): each variable's rows are
-// re-spaced in a host buffer of one variable and move in one copy on the
-// solver's stream.  Returns once the copies have completed.
-hipError_t copy_rows(st_solver *s, void *dst, const void *src, size_t es, int nvars, hipMemcpyKind kind) {
-    const st::Geo &g = s->g;
-    const size_t dpitch = (size_t)g.sx * es, hpitch = (size_t)g.rx * es;
-    const size_t rows = (size_t)g.sy * g.sz;  // of one variable
-    const size_t dvar = (size_t)g.nvol * es, hvar = (size_t)g.nref * es;
-    std::vector<char> tmp;
-    try {
-        tmp.assign(rows * dpitch, 0);
-    } catch (const std::bad_alloc &) {
-        return hipErrorOutOfMemory;
-    }
-    hipError_t e = hipSuccess;
-    for (int m = 0; m < nvars && e == hipSuccess; m++) {
-        if (kind == hipMemcpyHostToDevice) {
-            const char *h = (const char *)src + m * hvar;
-            for (size_t r = 0; r < rows; r++) std::memcpy(tmp.data() + r * dpitch, h + r * hpitch, hpitch);
-            e = hipMemcpyAsync((char *)dst + m * dvar, tmp.data(), dvar, kind, s->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-        } else {
-            e = hipMemcpyAsync(tmp.data(), (const char *)src + m * dvar, dvar, kind, s->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
-            char *h = (char *)dst + m * hvar;
-            if (e == hipSuccess)
-                for (size_t r = 0; r < rows; r++) std::memcpy(h + r * hpitch, tmp.data() + r * dpitch, hpitch);
-        }
-    }
-    return e;
 }
 
 }  // namespace
@@ -668,7 +639,7 @@ int st_set_grid(st_solver *s, const double *x, const double *y, const double *z,
 int st_copy_from_field(st_solver *s, const double *w_host) {
     NEED(s);
     if (!w_host) return fail(ST_ERR_ARG, "null host array");
-    HIPCHK(copy_rows(s, s->w, w_host, sizeof(double), 5, hipMemcpyHostToDevice));
+    HIPCHK(st::copy_rows(s, s->w, w_host, sizeof(double), 5, hipMemcpyHostToDevice));
     HIPCHK(hipStreamSynchronize(s->stream));
     return ST_OK;
 }
@@ -676,7 +647,7 @@ int st_copy_from_field(st_solver *s, const double *w_host) {
 int st_copy_to_field(st_solver *s, double *w_host) {
     NEED(s);
     if (!w_host) return fail(ST_ERR_ARG, "null host array");
-    HIPCHK(copy_rows(s, w_host, s->w, sizeof(double), 5, hipMemcpyDeviceToHost));
+    HIPCHK(st::copy_rows(s, w_host, s->w, sizeof(double), 5, hipMemcpyDeviceToHost));
     HIPCHK(hipStreamSynchronize(s->stream));
     return ST_OK;
 }
@@ -701,12 +672,12 @@ static int to_host(st_solver *s, double *host, const void *dev, size_t n) {
 static int ghost_to_host(st_solver *s, double *host, const void *dev) {
     const size_t n = (size_t)s->g.nref;
     if (!s->mixed) {
-        HIPCHK(copy_rows(s, host, dev, sizeof(double), 1, hipMemcpyDeviceToHost));
+        HIPCHK(st::copy_rows(s, host, dev, sizeof(double), 1, hipMemcpyDeviceToHost));
         HIPCHK(hipStreamSynchronize(s->stream));
         return ST_OK;
     }
     std::vector<float> tmp(n);
-    HIPCHK(copy_rows(s, tmp.data(), dev, sizeof(float), 1, hipMemcpyDeviceToHost));
+    HIPCHK(st::copy_rows(s, tmp.data(), dev, sizeof(float), 1, hipMemcpyDeviceToHost));
     HIPCHK(hipStreamSynchronize(s->stream));
     for (size_t t = 0; t < n; t++) host[t] = tmp[t];
     return ST_OK;
@@ -715,12 +686,12 @@ static int ghost_to_host(st_solver *s, double *host, const void *dev) {
 static int ghost_from_host(st_solver *s, void *dev, const double *host) {
     const size_t n = (size_t)s->g.nref;
     if (!s->mixed) {
-        HIPCHK(copy_rows(s, dev, host, sizeof(double), 1, hipMemcpyHostToDevice));
+        HIPCHK(st::copy_rows(s, dev, host, sizeof(double), 1, hipMemcpyHostToDevice));
         HIPCHK(hipStreamSynchronize(s->stream));
         return ST_OK;
     }
     std::vector<float> tmp(host, host + n);
-    HIPCHK(copy_rows(s, dev, tmp.data(), sizeof(float), 1, hipMemcpyHostToDevice));
+    HIPCHK(st::copy_rows(s, dev, tmp.data(), sizeof(float), 1, hipMemcpyHostToDevice));
     HIPCHK(hipStreamSynchronize(s->stream));
     return ST_OK;
 }

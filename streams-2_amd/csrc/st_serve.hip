@@ -250,6 +250,7 @@ struct st_server {
     Pool pool;
     int64_t used = 0;
     std::thread th, worker;
+    st::CopyStage stage;       // the worker's: it alone copies fields
     std::mutex mu;
     std::condition_variable cv_work, cv_done, cv_job;
     std::deque<ServeReq *> pending;
@@ -312,7 +313,7 @@ int capture(st_server *sv, Slot &sl) {
 // block this thread only).
 int setup(st_server *sv, Slot &sl) {
     ServeReq *r = sl.r;
-    st::SlotMem m{sv->pool.base + sl.off, (size_t)r->bytes, sl.stream, sl.hs, sl.tabs, r->time0, r->icyc0};
+    st::SlotMem m{sv->pool.base + sl.off, (size_t)r->bytes, sl.stream, sl.hs, sl.tabs, &sv->stage, r->time0, r->icyc0};
     int rc = st::solver_create_in(&r->p, m, &sl.s);
     if (rc) return rc;
     const std::vector<double> *gd = r->grid;
@@ -1086,6 +1087,7 @@ void destroy_slots(st_server *sv) {
         if (sl.stream) (void)hipStreamDestroy(sl.stream);
         sl = Slot();
     }
+    st::stage_destroy(sv->stage);
     if (sv->pool.base) (void)hipFree(sv->pool.base);
     sv->pool.base = nullptr;
 }
@@ -1131,6 +1133,7 @@ int st_server_create(int64_t hbm_capacity_bytes, int32_t max_slots, int32_t step
         delete sv;
         return sfail(ST_ERR_NOMEM, std::string("server memory: ") + hipGetErrorString(e));
     }
+    st::stage_create(sv->stage, st::kStagePerThread * st::kStageThreads);
     sv->t0 = Clock::now();
     sv->th = std::thread(serve_loop, sv);
     sv->worker = std::thread(worker_loop, sv);

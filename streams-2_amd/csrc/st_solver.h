@@ -6,6 +6,25 @@
 #include "st_batch.h"
 #include "st_internal.h"
 
+namespace st {
+// Pinned staging of field copies (st_copy.hip): a pair of buffers and their
+// events for each host thread of a copy.  Used by one copy at a time.
+constexpr int kStageThreads = 8;
+constexpr size_t kStagePerThread = 4 << 20;  // field bytes that are worth a thread
+constexpr size_t kStageBuffer = 2 << 20;
+struct CopyStage {
+    char *mem = nullptr;  // 2 * threads buffers of bytes each; null: none
+    size_t bytes = 0;
+    int threads = 0;
+    hipEvent_t ev[2 * kStageThreads] = {};
+};
+void stage_create(CopyStage &cs, size_t nbytes);
+void stage_destroy(CopyStage &cs);
+// nvars ghosted variables of es-byte values between the solver's pitched
+// layout (device) and the reference layout (host); returns once they are there
+hipError_t copy_rows(st_solver *s, void *dst, const void *src, size_t es, int nvars, hipMemcpyKind kind);
+}  // namespace st
+
 struct st_solver {
     st_params p;
     st::Geo g;
@@ -83,6 +102,8 @@ struct st_solver {
     // the solver's arrays, hs is the lender's; neither is freed with the solver
     char *arena_lo, *arena_hi;
     bool borrowed_hs;
+    st::CopyStage *stage;     // pinned staging of field copies: own_stage, or lent (null: none)
+    st::CopyStage own_stage;
 };
 
 // HIP events around each kernel family while st_kernel_times runs
@@ -109,6 +130,7 @@ struct SlotMem {
     hipStream_t stream;
     DevScalars *hs;
     int *tabs;
+    CopyStage *stage;  // pinned staging of field copies, one thread at a time
     double time0;   // start time and step counter of the run (st_set_time without its synchronisation)
     int64_t icyc0;
 };
