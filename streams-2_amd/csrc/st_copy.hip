@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
@@ -136,6 +137,7 @@ hipError_t copy_rows(st_solver *s, void *dst, const void *src, size_t es, int nv
     CopyStage *cs = s->stage;
     const size_t total = j.rows * j.dpitch;
     std::vector<char> tmp;
+    std::unique_lock<std::mutex> lk;
     int threads = 1;
     if (cs && cs->mem && cs->bytes >= j.dpitch) {
         threads = (int)(total / kStagePerThread);
@@ -143,6 +145,7 @@ hipError_t copy_rows(st_solver *s, void *dst, const void *src, size_t es, int nv
         j.mem = cs->mem;
         j.bytes = cs->bytes;
         j.ev = cs->ev;
+        lk = std::unique_lock<std::mutex>(cs->mu);
     } else {
         j.bytes = j.dpitch > kStageBuffer ? j.dpitch : kStageBuffer;
         j.ev = nullptr;

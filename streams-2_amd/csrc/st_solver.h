@@ -1,6 +1,7 @@
 // st_solver.h -- host-side solver state shared by the C ABI and the launchers.
 #pragma once
 
+#include <mutex>
 #include <string>
 
 #include "st_batch.h"
@@ -8,11 +9,13 @@
 
 namespace st {
 // Pinned staging of field copies (st_copy.hip): a pair of buffers and their
-// events for each host thread of a copy.  Used by one copy at a time.
+// events for each host thread of a copy.  One copy at a time holds mu: calls
+// on one handle from several threads queue there.
 constexpr int kStageThreads = 8;
 constexpr size_t kStagePerThread = 4 << 20;  // field bytes that are worth a thread
 constexpr size_t kStageBuffer = 2 << 20;
 struct CopyStage {
+    std::mutex mu;
     char *mem = nullptr;  // 2 * threads buffers of bytes each; null: none
     size_t bytes = 0;
     int threads = 0;
@@ -130,7 +133,7 @@ struct SlotMem {
     hipStream_t stream;
     DevScalars *hs;
     int *tabs;
-    CopyStage *stage;  // pinned staging of field copies, one thread at a time
+    CopyStage *stage;  // pinned staging of field copies
     double time0;   // start time and step counter of the run (st_set_time without its synchronisation)
     int64_t icyc0;
 };

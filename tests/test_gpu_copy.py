@@ -50,3 +50,13 @@ def test_two_solvers_copy_at_once():
     with ThreadPoolExecutor(2) as ex:
         for f in [ex.submit(_round_trip, (96, 80, 70), s) for s in (3, 4)]:
             f.result()
+
+
+def test_one_handle_read_by_two_threads():
+    c = _case((96, 80, 70))
+    with ChannelSolver(c.params, c.grid) as g:
+        w = np.random.default_rng(5).standard_normal((5,) + g.shape_g)
+        g.copy_from_field(w)
+        with ThreadPoolExecutor(2) as ex:
+            for f in [ex.submit(g.copy_to_field) for _ in range(4)]:
+                assert np.array_equal(f.result(), w)
