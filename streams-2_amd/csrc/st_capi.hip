@@ -311,8 +311,7 @@ int stage_one_pass(st_solver *s, int istep, bool end, bool last) {
     TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end, last));
     if (s->p.channel_case && s->p.theta_wall >= -1.0)
         TIMED(ST_K_FORCE_VAR, launch_force_var(s, one_pass_update_blocks(g)));
-    if (s->recyc) TIMED(ST_K_BC, launch_inflow_draws(s));
-    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s));
+    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s, true));
     s->cur ^= 1;
     s->last_stage = istep;
     s->fln_current = false;
@@ -373,9 +372,9 @@ int stage(st_solver *s, int istep) {
     if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur));  // bc_nr
     TIMED(ST_K_UPDATE, launch_update(s, fprev, fcur, istep));
     if (s->p.channel_case && s->p.theta_wall >= -1.0) TIMED(ST_K_FORCE_VAR, launch_force_var(s, update_blocks(g)));
-    // get_crandom_f of euler_z: the random inflow plane of this stage
-    if (s->recyc) TIMED(ST_K_BC, launch_inflow_draws(s));
-    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s));  // update_ghost(do_swap=0)
+    // get_crandom_f of euler_z (the random inflow plane of this stage), then
+    // update_ghost(do_swap=0)
+    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s, true));
     s->cur ^= 1;
     s->last_stage = istep;
     s->fln_current = false;
@@ -870,7 +869,7 @@ int st_set_recycling(st_solver *s, int32_t i_recyc, double betarecyc, double glu
 int st_update_ghost(st_solver *s, int32_t do_swap) {
     NEED(s);
     if (s->recyc && !s->recyc_set) return fail(ST_ERR_STATE, "st_set_recycling not called");
-    if (s->general_bc) HIPCHK(st::launch_physical_ghosts(s));
+    if (s->general_bc) HIPCHK(st::launch_physical_ghosts(s, false));
     else HIPCHK(st::launch_wall_ghosts(s));
     if (do_swap) HIPCHK(st::launch_fill_periodic(s, s->w, 5));
     return ST_OK;

@@ -135,21 +135,17 @@ __device__ __forceinline__ int face_boundary(const Geo &g, int ilat, int a, int 
     }
 }
 
-// One face of update_ghost (singleideal_cpu.F90:1064-1138), one thread per
-// tangential point: free stream (bcfree_subroutine, kernels_cpu.F90:
+// One point of a face of update_ghost (singleideal_cpu.F90:1064-1138): free
+// stream (bcfree_subroutine, kernels_cpu.F90:
 // 5989-6056), extrapolation (bcextr_subroutine, :6323-6390), symmetry on
 // ymin (bcsym_subroutine, :6394-6418), staggered or node isothermal wall
 // on ymin (bcwall_staggered_subroutine :6612-6678, bcwall_subroutine
 // :6478-6525), oblique shock on ymax (bcshock_subroutine, :6159-6196).
 template <typename R>
-__global__ void k_bc_face(Geo g, KPar P, double *__restrict__ w, const R *__restrict__ wa,
-                          const double *__restrict__ xc, const double *__restrict__ yc, int ilat, int tag,
-                          int staggered, const double *__restrict__ wmean) {
-    const int na = ilat <= 2 ? g.ny : g.nx;
-    const int nb = ilat <= 4 ? g.nz : g.ny;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= na * nb) return;
-    const int a = t % na + 1, b = t / na + 1;
+__device__ __forceinline__ void bc_point(const Geo &g, const KPar &P, double *__restrict__ w,
+                                         const R *__restrict__ wa, const double *__restrict__ xc,
+                                         const double *__restrict__ yc, int ilat, int tag, int staggered,
+                                         const double *__restrict__ wmean, int a, int b) {
     const size_t nv = g.nvol;
     const int ng = g.ng;
     if (tag == 1) {
@@ -384,38 +380,60 @@ __device__ __forceinline__ size_t wrc(const Geo &g, int i, int j, int k, int m) 
     return (size_t)(i - 1) + (size_t)g.ng * ((size_t)(j - 1) + (size_t)g.ny * ((size_t)(k - 1) + (size_t)g.nz * m));
 }
 
+// recyc_exchange (singleideal_cpu.F90:935-999) for one block in x and z:
+// wrecyc(i, j, k, m) = w(i_recyc+1-i, j, k shifted by nz/2, m)
+__device__ __forceinline__ void recyc_copy(const Geo &g, const double *__restrict__ w, int i_recyc,
+                                           double *__restrict__ wrecyc, long long t) {
+    const long long n = (long long)g.ng * g.ny * g.nz;
+    if (t >= n) return;
+    const int i = (int)(t % g.ng) + 1, j = (int)((t / g.ng) % g.ny) + 1, k = (int)(t / ((long long)g.ng * g.ny)) + 1;
+    const int src = gidx(g, i_recyc + 1 - i, j, recyc_k(k, g.nz));
+    for (int m = 0; m < 5; m++) wrecyc[(size_t)m * n + t] = w[(size_t)m * g.nvol + src];
+}
+__global__ void k_recyc_exchange(Geo g, const double *__restrict__ w, int i_recyc, double *__restrict__ wrecyc) {
+    recyc_copy(g, w, i_recyc, wrecyc, (long long)blockIdx.x * blockDim.x + threadIdx.x);
+}
+
 // bcrecyc_subroutine_1 (kernels_cpu.F90:5810-5828): spanwise sums of the
-// recycled planes, one thread per (i, j), k summed in order.
-__global__ void k_recyc_avg(Geo g, const double *__restrict__ wrecyc, double *__restrict__ av) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+// recycled planes, one thread per (i, j, m), k summed in order; read where
+// the planes come from, so that the copies need not be there yet.
+__device__ __forceinline__ void recyc_sum(const Geo &g, const double *__restrict__ w, int i_recyc,
+                                          double *__restrict__ av, int t) {
     if (t >= g.ng * g.ny * 5) return;
     const int i = t % g.ng + 1, j = (t / g.ng) % g.ny + 1, m = t / (g.ng * g.ny);
-    // one (i, j, m) per thread; the sum runs over k in order, its loads
-    // issued eight at a time ahead of the additions
+    const double *wm = w + (size_t)m * g.nvol;
+    auto at = [&](int k) { return wm[gidx(g, i_recyc + 1 - i, j, recyc_k(k, g.nz))]; };
+    // the loads are issued sixteen at a time ahead of the additions
     double a = 0.0;
     int k = 1;
-    for (; k + 7 <= g.nz; k += 8) {
-        double v[8];
+    for (; k + 15 <= g.nz; k += 16) {
+        double v[16];
 #pragma unroll
-        for (int q = 0; q < 8; q++) v[q] = wrecyc[wrc(g, i, j, k + q, m)];
+        for (int q = 0; q < 16; q++) v[q] = at(k + q);
 #pragma unroll
-        for (int q = 0; q < 8; q++) a = a + v[q];
+        for (int q = 0; q < 16; q++) a = a + v[q];
     }
-    for (; k <= g.nz; k++) a = a + wrecyc[wrc(g, i, j, k, m)];
+    for (; k <= g.nz; k++) a = a + at(k);
     av[(i - 1) + g.ng * ((j - 1) + g.ny * m)] = a;
 }
 
-// bcrecyc_subroutine_2/3 (kernels_cpu.F90:5832-5947): one thread per
-// (j, k) of the inflow; the Favre fluctuations of the recycled planes are
+// bcrecyc_subroutine_2/3 (kernels_cpu.F90:5832-5947) for point t = (j, k) of
+// inflow plane 1-i; the Favre fluctuations of the recycled planes are
 // formed where they are interpolated.  wmean(1-ng:0, j, m) sits at
 // [(ng-i) + ng*((j-1) + ny*m)] for plane 1-i.  With u0_02 != 0 (rand_type
 // != 0) each velocity fluctuation gains u0_02*(r - 0.5)*min(eta, 1) from
 // the random plane r(j, k, c) (Fortran order (1:ny, 1:nz, 1:3)).
-__global__ void k_recyc_inflow(Geo g, KPar P, double *__restrict__ w, const double *__restrict__ rc,
-                               const int *__restrict__ maps, const double *__restrict__ wrecyc, double betarecyc,
-                               const double *__restrict__ rplane, double u0_02) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= g.ny * g.nz) return;
+struct Inflow {
+    const double *rc;
+    const int *maps;
+    const double *wrecyc, *rplane;
+    double betarecyc, u0_02;
+};
+__device__ __forceinline__ void recyc_inflow(const Geo &g, const KPar &P, double *__restrict__ w, const Inflow &I, int i,
+                                             int t) {
+    const double *rc = I.rc, *wrecyc = I.wrecyc, *rplane = I.rplane;
+    const int *maps = I.maps;
+    const double betarecyc = I.betarecyc, u0_02 = I.u0_02;
     const int j = t % g.ny + 1, k = t / g.ny + 1;
     const int ng = g.ng, ny = g.ny, nz = g.nz, ny2 = ny + 2 * ng;
     const size_t nv = g.nvol;
@@ -435,54 +453,52 @@ __global__ void k_recyc_inflow(Geo g, KPar P, double *__restrict__ w, const doub
         disty_out = (eta - etr[j_out + ng - 1]) / (etr[j_out + 1 + ng - 1] - etr[j_out + ng - 1]);
     }
     const double p0 = P.rho0 * P.rgas0 * P.t0;
-    for (int i = 1; i <= ng; i++) {
-        const double rhomean = wmean[(ng - i) + ng * ((j - 1) + ny * 0)];
-        const double uumean = wmean[(ng - i) + ng * ((j - 1) + ny * 1)] / rhomean;
-        const double vvmean = wmean[(ng - i) + ng * ((j - 1) + ny * 2)] / rhomean;
-        const double wwmean = wmean[(ng - i) + ng * ((j - 1) + ny * 3)] / rhomean;
-        double rhofluc = 0.0, ufluc = 0.0, vfluc = 0.0, wfluc = 0.0;
-        if (!zero) {
-            // fluctuation of variable m (0 rho, 1..3 velocity) of plane i at row jx
-            auto fluc = [&](int jx, int m) {
-                const double *a = av + (i - 1) + ng * (jx - 1);
-                const double rho = wrecyc[wrc(g, i, jx, k, 0)];
-                if (m == 0) return rho - a[0] / nz;
-                return wrecyc[wrc(g, i, jx, k, m)] / rho - a[(size_t)ng * ny * m] / a[0];
-            };
-            double f_in[4], f_out[4];
-            for (int m = 0; m < 4; m++) {
-                f_in[m] = fluc(j_inn, m) * (1.0 - disty_inn) + fluc(j_inn + 1, m) * disty_inn;
-                f_out[m] = fluc(j_out, m) * (1.0 - disty_out) + fluc(j_out + 1, m) * disty_out;
-            }
-            rhofluc = f_in[0] * weta1 + f_out[0] * weta;
-            ufluc = f_in[1] * weta1 + f_out[1] * weta;
-            vfluc = f_in[2] * weta1 + f_out[2] * weta;
-            wfluc = f_in[3] * weta1 + f_out[3] * weta;
-            rhofluc = rhofluc * bdamp;
-            ufluc = ufluc * bdamp * betarecyc;
-            vfluc = vfluc * bdamp * betarecyc;
-            wfluc = wfluc * bdamp * betarecyc;
-            if (u0_02 != 0.0) {
-                const size_t pl = (size_t)(j - 1) + (size_t)ny * (k - 1), pn = (size_t)ny * nz;
-                ufluc = ufluc + u0_02 * (rplane[pl] - 0.5) * etamin;
-                vfluc = vfluc + u0_02 * (rplane[pl + pn] - 0.5) * etamin;
-                wfluc = wfluc + u0_02 * (rplane[pl + 2 * pn] - 0.5) * etamin;
-            }
+    const double rhomean = wmean[(ng - i) + ng * ((j - 1) + ny * 0)];
+    const double uumean = wmean[(ng - i) + ng * ((j - 1) + ny * 1)] / rhomean;
+    const double vvmean = wmean[(ng - i) + ng * ((j - 1) + ny * 2)] / rhomean;
+    const double wwmean = wmean[(ng - i) + ng * ((j - 1) + ny * 3)] / rhomean;
+    double rhofluc = 0.0, ufluc = 0.0, vfluc = 0.0, wfluc = 0.0;
+    if (!zero) {
+        // fluctuation of variable m (0 rho, 1..3 velocity) of plane i at row jx
+        auto fluc = [&](int jx, int m) {
+            const double *a = av + (i - 1) + ng * (jx - 1);
+            const double rho = wrecyc[wrc(g, i, jx, k, 0)];
+            if (m == 0) return rho - a[0] / nz;
+            return wrecyc[wrc(g, i, jx, k, m)] / rho - a[(size_t)ng * ny * m] / a[0];
+        };
+        double f_in[4], f_out[4];
+        for (int m = 0; m < 4; m++) {
+            f_in[m] = fluc(j_inn, m) * (1.0 - disty_inn) + fluc(j_inn + 1, m) * disty_inn;
+            f_out[m] = fluc(j_out, m) * (1.0 - disty_out) + fluc(j_out + 1, m) * disty_out;
         }
-        rhofluc = fmax(-0.75 * rhomean, rhofluc);
-        rhofluc = fmin(4.0 * rhomean, rhofluc);
-        const double rho = rhomean + rhofluc;
-        const double tt = p0 / rho / P.rgas0;
-        const double uu = uumean + ufluc, vv = vvmean + vfluc, ww = wwmean + wfluc;
-        const double rhou = rho * uu, rhov = rho * vv, rhow = rho * ww;
-        const double ee = e_from_temperature(P, tt);
-        const int d = gidx(g, 1 - i, j, k);
-        w[d] = rho;
-        w[nv + d] = rhou;
-        w[2 * nv + d] = rhov;
-        w[3 * nv + d] = rhow;
-        w[4 * nv + d] = rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho;
+        rhofluc = f_in[0] * weta1 + f_out[0] * weta;
+        ufluc = f_in[1] * weta1 + f_out[1] * weta;
+        vfluc = f_in[2] * weta1 + f_out[2] * weta;
+        wfluc = f_in[3] * weta1 + f_out[3] * weta;
+        rhofluc = rhofluc * bdamp;
+        ufluc = ufluc * bdamp * betarecyc;
+        vfluc = vfluc * bdamp * betarecyc;
+        wfluc = wfluc * bdamp * betarecyc;
+        if (u0_02 != 0.0) {
+            const size_t pl = (size_t)(j - 1) + (size_t)ny * (k - 1), pn = (size_t)ny * nz;
+            ufluc = ufluc + u0_02 * (rplane[pl] - 0.5) * etamin;
+            vfluc = vfluc + u0_02 * (rplane[pl + pn] - 0.5) * etamin;
+            wfluc = wfluc + u0_02 * (rplane[pl + 2 * pn] - 0.5) * etamin;
+        }
     }
+    rhofluc = fmax(-0.75 * rhomean, rhofluc);
+    rhofluc = fmin(4.0 * rhomean, rhofluc);
+    const double rho = rhomean + rhofluc;
+    const double tt = p0 / rho / P.rgas0;
+    const double uu = uumean + ufluc, vv = vvmean + vfluc, ww = wwmean + wfluc;
+    const double rhou = rho * uu, rhov = rho * vv, rhow = rho * ww;
+    const double ee = e_from_temperature(P, tt);
+    const int d = gidx(g, 1 - i, j, k);
+    w[d] = rho;
+    w[nv + d] = rhou;
+    w[2 * nv + d] = rhov;
+    w[3 * nv + d] = rhow;
+    w[4 * nv + d] = rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho;
 }
 
 // ------------------------------------------------------ random inflow plane
@@ -495,9 +511,9 @@ __global__ void k_recyc_inflow(Geo g, KPar P, double *__restrict__ w, const doub
 // win[q] = r[n0-31+q] before the sweep, so every draw is independent.  The
 // window of the next sweep is written to the other buffer; the last
 // workgroup to finish flips the buffer index and clears the ticket.
-__global__ __launch_bounds__(256) void k_inflow_draws(Geo g, const uint32_t *__restrict__ coef, int n,
-                                                      uint32_t *__restrict__ win2, int *__restrict__ ctl,
-                                                      double *__restrict__ plane) {
+__device__ __forceinline__ void inflow_draws(const Geo &g, const uint32_t *__restrict__ coef, int n,
+                                             uint32_t *__restrict__ win2, int *__restrict__ ctl,
+                                             double *__restrict__ plane, int blk, int nblk) {
     __shared__ uint32_t wl[31];
     __shared__ bool last;
     const int par = __hip_atomic_load(&ctl[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -505,7 +521,7 @@ __global__ __launch_bounds__(256) void k_inflow_draws(Geo g, const uint32_t *__r
     uint32_t *wout = win2 + 31 * (par ^ 1);
     if (threadIdx.x < 31) wl[threadIdx.x] = win[threadIdx.x];
     __syncthreads();
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blk * 256 + threadIdx.x;
     if (t < n) {
         uint32_t r = 0u;
         for (int q = 0; q < 31; q++) r += coef[(size_t)q * n + t] * wl[q];
@@ -516,11 +532,74 @@ __global__ __launch_bounds__(256) void k_inflow_draws(Geo g, const uint32_t *__r
     if (t < 31 && n - 31 + t < 0) wout[t] = wl[n + t];  // fewer than 31 draws: the window slides
     __threadfence();
     __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(&ctl[1], 1) == (int)gridDim.x - 1;
+    if (threadIdx.x == 0) last = atomicAdd(&ctl[1], 1) == nblk - 1;
     __syncthreads();
     if (last && threadIdx.x == 0) {
         ctl[0] = par ^ 1;
         ctl[1] = 0;
+    }
+}
+__global__ __launch_bounds__(256) void k_inflow_draws(Geo g, const uint32_t *__restrict__ coef, int n,
+                                                      uint32_t *__restrict__ win2, int *__restrict__ ctl,
+                                                      double *__restrict__ plane) {
+    inflow_draws(g, coef, n, win2, ctl, plane, blockIdx.x, gridDim.x);
+}
+
+// What the recycled inflow wants before its planes are formed, in one launch:
+// the copies (nc workgroups), their spanwise sums (ns) and, where a stage asks
+// for them, the draws of its random plane (the rest).  None reads what another
+// writes.
+__global__ __launch_bounds__(256) void k_recyc_gather(Geo g, const double *__restrict__ w, int i_recyc,
+                                                      double *__restrict__ wrecyc, double *__restrict__ av, int nc,
+                                                      int ns, const uint32_t *__restrict__ coef, int n,
+                                                      uint32_t *__restrict__ win2, int *__restrict__ ctl,
+                                                      double *__restrict__ plane) {
+    int blk = blockIdx.x;
+    if (blk < nc) return recyc_copy(g, w, i_recyc, wrecyc, (long long)blk * 256 + threadIdx.x);
+    blk -= nc;
+    if (blk < ns) return recyc_sum(g, w, i_recyc, av, blk * 256 + threadIdx.x);
+    inflow_draws(g, coef, n, win2, ctl, plane, blk - ns, (int)gridDim.x - nc - ns);
+}
+
+// The physical faces in one launch, 128 points a workgroup: face q of the set
+// has the workgroups first[q] .. first[q+1]-1; face 0 is the recycled inflow,
+// its ng planes one after the other.  A launch of its own for every face cost
+// 5.8 us each on 256x96x64, and the inflow with its planes in one thread 22 us,
+// of serial divisions in 24 waves.  The faces write ghost points of their own
+// and read interior cells, but the node wall and the impinging shock also
+// change the row of cells they stand on.  After the x faces, in the order of
+// the reference: there the thread of the row's first or last cell first does
+// the x face's point of that cell (take), and the x face leaves it out.
+struct FaceSet {
+    int n;
+    int first[7], ilat[7], tag[7];
+    bool take[2];  // ymin, ymax
+};
+template <typename R>
+__global__ __launch_bounds__(128) void k_bc_faces(Geo g, KPar P, double *__restrict__ w, const R *__restrict__ wa,
+                                                  const double *__restrict__ xc, const double *__restrict__ yc,
+                                                  int staggered, FaceSet F, Inflow I) {
+    int q = 0, blk = blockIdx.x;
+    while (q + 1 < F.n && blk >= F.first[q + 1]) q++;
+    const int t = (blk - F.first[q]) * 128 + threadIdx.x;
+    const int ilat = F.ilat[q];
+    if (ilat == 0) {
+        const int np = g.ny * g.nz;
+        if (t < np * g.ng) recyc_inflow(g, P, w, I, t / np + 1, t % np);
+        return;
+    }
+    const int na = ilat <= 2 ? g.ny : g.nx;
+    const int nb = ilat <= 4 ? g.nz : g.ny;
+    if (t >= na * nb) return;
+    const int a = t % na + 1, b = t / na + 1;
+    if (ilat <= 2 && ((a == 1 && F.take[0]) || (a == g.ny && F.take[1]))) return;
+    const bool takes = (ilat == 3 && F.take[0]) || (ilat == 4 && F.take[1]);
+#pragma unroll 1
+    for (int o = takes && (a == 1 || a == g.nx) ? 0 : q; o <= q; o++) {
+        const int lat = F.ilat[o];
+        const bool own = o == q;
+        if (!own && !((lat == 1 && a == 1) || (lat == 2 && a == g.nx))) continue;
+        bc_point(g, P, w, wa, xc, yc, lat, F.tag[o], staggered, I.rc, own ? a : (ilat == 3 ? 1 : g.ny), b);
     }
 }
 
@@ -3252,17 +3331,6 @@ __global__ __launch_bounds__(256) void k_force_var_sums(Geo g, KPar P, const dou
     if (flat_thread() == 0) partials[flat_block()] = acc[0];
 }
 
-// recyc_exchange (singleideal_cpu.F90:935-999) for one block in x and z:
-// wrecyc(i, j, k, m) = w(i_recyc+1-i, j, k shifted by nz/2, m)
-__global__ void k_recyc_exchange(Geo g, const double *__restrict__ w, int i_recyc, double *__restrict__ wrecyc) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long n = (long long)g.ng * g.ny * g.nz;
-    if (t >= n) return;
-    const int i = (int)(t % g.ng) + 1, j = (int)((t / g.ng) % g.ny) + 1, k = (int)(t / ((long long)g.ng * g.ny)) + 1;
-    const int src = gidx(g, i_recyc + 1 - i, j, recyc_k(k, g.nz));
-    for (int m = 0; m < 5; m++) wrecyc[(size_t)m * n + t] = w[(size_t)m * g.nvol + src];
-}
-
 // ================================================================ launchers
 static inline dim3 cell_grid(const Geo &g) { return dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz); }
 static inline int cell_blocks(const Geo &g) { return ((g.nx + 63) / 64) * ((g.ny + 3) / 4) * g.nz; }
@@ -3653,20 +3721,6 @@ hipError_t launch_update(st_solver *s, const void *fl_prev, const void *fl, int 
     return hipGetLastError();
 }
 
-hipError_t launch_recycling(st_solver *s) {
-    ST_NOREC();
-    const Geo &g = s->g;
-    double *av = s->rc_real + (size_t)g.ng * g.ny * 4 + g.ny + 4 * (size_t)(g.ny + 2 * g.ng);
-    const int n1 = g.ng * g.ny, n2 = g.ny * g.nz;
-    hipError_t e = launch_recyc_exchange(s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_recyc_avg, dim3((5 * n1 + 127) / 128), dim3(128), 0, s->stream, g, s->wrecyc, av);
-    const double u0_02 = s->p.rand_type != 0 && s->rplane ? 0.02 * s->p.u0 : 0.0;
-    hipLaunchKernelGGL(k_recyc_inflow, dim3((n2 + 127) / 128), dim3(128), 0, s->stream, g, s->kp, s->w, s->rc_real,
-                       s->rc_maps, s->wrecyc, s->betarecyc, s->rplane, u0_02);
-    return hipGetLastError();
-}
-
 hipError_t launch_inflow_draws(st_solver *s) {
     ST_NOREC();
     const int n = s->rng_n;
@@ -3686,25 +3740,57 @@ hipError_t launch_rng_reset(st_solver *s) {
     return hipGetLastError();
 }
 
-hipError_t launch_physical_ghosts(st_solver *s) {
+hipError_t launch_physical_ghosts(st_solver *s, bool draws) {
     ST_NOREC();
     const Geo &g = s->g;
-    if (s->recyc) {
-        hipError_t e = launch_recycling(s);  // recyc_exchange, then face xmin
+    Inflow I{};
+    I.rc = s->rc_real;
+    FaceSet F{};
+    int blocks = 0;
+    auto add = [&](int ilat, int tag, int points) {
+        F.first[F.n] = blocks;
+        F.ilat[F.n] = ilat;
+        F.tag[F.n] = tag;
+        F.n++;
+        blocks += (points + 127) / 128;
+    };
+    auto launch = [&]() {
+        ST_DISPATCH(hipLaunchKernelGGL(k_bc_faces<R>, dim3(blocks), dim3(128), 0, s->stream, g, s->kp, s->w,
+                                       (const R *)s->w_aux, s->x, s->y, s->p.is_y_staggered, F, I));
+        F = FaceSet{};
+        blocks = 0;
+        return hipGetLastError();
+    };
+    if (s->recyc) {  // recyc_exchange, then face xmin
+        double *av = s->rc_real + (size_t)g.ng * g.ny * 4 + g.ny + 4 * (size_t)(g.ny + 2 * g.ng);
+        const int nc = (int)(((long long)g.ng * g.ny * g.nz + 255) / 256), ns = (5 * g.ng * g.ny + 255) / 256;
+        const int n = draws && s->rplane && s->rng_n > 0 ? s->rng_n : 0, nt = n > 31 ? n : 31;
+        hipLaunchKernelGGL(k_recyc_gather, dim3(nc + ns + (n ? (nt + 255) / 256 : 0)), dim3(256), 0, s->stream, g, s->w,
+                           s->i_recyc, s->wrecyc, av, nc, ns, s->rng_coef, n, s->rng_win, s->rng_ctl, s->rplane);
+        hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
+        I.maps = s->rc_maps;
+        I.wrecyc = s->wrecyc;
+        I.rplane = s->rplane;
+        I.betarecyc = s->betarecyc;
+        I.u0_02 = s->p.rand_type != 0 && s->rplane ? 0.02 * s->p.u0 : 0.0;
+        add(0, 10, g.ng * g.ny * g.nz);
     }
     for (int ilat = 1; ilat <= 2 * s->kp.ndim; ilat++) {
         const int tag = s->kp.bctag[ilat - 1];
         if (tag == 0 || tag == 8 || tag == 10) continue;
         if (tag == 9 && !s->wmean_set) continue;
-        const int n = (ilat <= 2 ? g.ny : g.nx) * (ilat <= 4 ? g.nz : g.ny);
-        ST_DISPATCH(hipLaunchKernelGGL(k_bc_face<R>, dim3((n + 127) / 128), dim3(128), 0, s->stream, g, s->kp, s->w,
-                                       (const R *)s->w_aux, s->x, s->y, ilat, tag, s->p.is_y_staggered,
-                                       (const double *)s->rc_real));
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        // z faces read the rows that a y face changes; below eight rows the y
+        // faces read each other's
+        if (F.n && (g.ny < 8 || (ilat >= 5 && (F.take[0] || F.take[1])))) {
+            hipError_t e = launch();
+            if (e != hipSuccess) return e;
+        }
+        add(ilat, tag, (ilat <= 2 ? g.ny : g.nx) * (ilat <= 4 ? g.nz : g.ny));
+        if (ilat == 3) F.take[0] = tag == 6 && !s->p.is_y_staggered;
+        if (ilat == 4) F.take[1] = tag == 7;
     }
-    return hipSuccess;
+    return F.n ? launch() : hipSuccess;
 }
 
 hipError_t launch_bc_nr(st_solver *s, void *fl) {

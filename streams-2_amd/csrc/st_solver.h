@@ -197,12 +197,11 @@ hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int 
 int aux_dt_blocks(const Geo &g);  // block maxima of an aux pass over the ghosted box
 hipError_t launch_wall_ghosts(st_solver *s);
 // physical ghosts of every non-periodic face in the order xmin..zmax
-// (update_ghost without the periodic swap)
-hipError_t launch_physical_ghosts(st_solver *s);
+// (update_ghost without the periodic swap), recyc_exchange and the recycled
+// inflow included; draws: first redraw the random inflow plane
+hipError_t launch_physical_ghosts(st_solver *s, bool draws);
 // characteristic boundary treatment added to fl (bc_nr)
 hipError_t launch_bc_nr(st_solver *s, void *fl);
-// recyc_exchange + bcrecyc of face xmin
-hipError_t launch_recycling(st_solver *s);
 // the random inflow plane: redraw rows 2..jbl (after a z sweep), and the
 // generator window reset to its seeded state
 hipError_t launch_inflow_draws(st_solver *s);

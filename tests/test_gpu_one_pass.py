@@ -121,3 +121,29 @@ def test_one_call_leaves_what_single_steps_leave(make, precision):
             got.append([g.copy_to_field(), g.get_fl()] + [g.get_aux(v) for v in range(1, 11)])
     for a, b in zip(*got):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("size", [(20, 7, 6), (20, 8, 6), (131, 9, 5)])
+@pytest.mark.parametrize("tags", [(2, 2, 6, 7, 0, 0), (4, 2, 6, 2, 2, 2), (1, 4, 5, 7, 2, 2), (3, 4, 6, 4, 0, 0)])
+def test_faces_of_one_launch(size, tags):
+    """All faces at once, where a node wall or a shock changes the row an x
+    face or a z face reads, down to rows that the y faces read from each other
+    (they then launch one by one).  The bar of the face tests, 1e-14."""
+    nx, ny, nz = size
+    c = make_bl_box(nx=nx, ny=ny, nz=nz, seed=4, bctags=tags, bctags_nr=(0,) * 6, mach=0.5 if 3 in tags else 2.0,
+                    **(dict(shock_angle_deg=35.0, xshock_imp=5.0, tanhfacs=0.5) if 7 in tags else {}))
+    rng = np.random.default_rng(nx + ny)
+    w0 = c.w0 * (1.0 + 0.01 * rng.standard_normal(c.w0.shape))
+    o = Oracle(c.params, c.grid)
+    o.w[:] = w0
+    with ChannelSolver(c.params, c.grid) as g:
+        g.copy_from_field(w0)
+        o.update_ghost(0)
+        g.update_ghost(0)
+        w = g.copy_to_field()
+    n = 3
+    for m in range(5):
+        a, b = w[m], o.w[m]
+        assert rel_l2(a[n:-n, n:-n, :], b[n:-n, n:-n, :]) <= 1e-14, m
+        assert rel_l2(a[n:-n, :, n:-n], b[n:-n, :, n:-n]) <= 1e-14, m
+        assert rel_l2(a[:, n:-n, n:-n], b[:, n:-n, n:-n]) <= 1e-14, m
