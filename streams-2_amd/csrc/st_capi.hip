@@ -291,27 +291,29 @@ struct TimeScope {
 // near the threshold in FP64 from w (its fluxes and stresses stay FP32).
 bool fp64_sensor(const st_solver *s) { return s->mixed && s->p.conservative_viscous != 1; }
 
-// one RK stage of rk_sync in four launches (st_stage.hip), plus the step's
-// WENO masks at its first stage; end: the last stage of a st_advance step;
-// last: no step of the same call follows, so what its third stage leaves is
-// the caller's to read
-int stage_one_pass(st_solver *s, int istep, bool end, bool last) {
+// one RK stage of rk_sync in three launches (st_stage.hip), plus the step's
+// WENO masks at its first stage; first, last: the first and last stage of a
+// call, where w_aux comes from and goes to the caller; end: the last stage of
+// a st_advance step; stay: no step of the call follows
+int stage_one_pass(st_solver *s, int istep, bool end, bool first, bool stay) {
     using namespace st;
     void *fprev = s->F[s->cur], *fcur = s->F[s->cur ^ 1];
     const Geo &g = s->g;
-    const bool dt = istep == 0 && s->dt_in_stage && s->p.cfl > 0;
+    const bool dt = istep == 0 && s->dt_in_stage && s->p.cfl > 0, last = stay && istep == 2;
     if (istep == 0) TIMED(ST_K_WENO_FIX, launch_hot_items(s));
-    TIMED(ST_K_AUX, launch_aux(s, 1 - g.ng, g.nx + g.ng, 1 - g.ng, g.ny + g.ng, 1 - g.ng, g.nz + g.ng, true, dt, true,
-                               s->has_nr || (last && istep == 2)));
+    const bool aux_dt = dt && s->mixed;  // (k_flux takes the radii in FP64)
+    if ((first && istep == 0) || last || aux_dt)
+        TIMED(ST_K_AUX, launch_aux(s, 1 - g.ng, g.nx + g.ng, 1 - g.ng, g.ny + g.ng, 1 - g.ng, g.nz + g.ng, true, aux_dt,
+                                   true, last));
     if (istep == 0) s->dt_in_stage = false;
-    TIMED(ST_K_EULER_XY, launch_flux(s, fcur, istep));
+    TIMED(ST_K_EULER_XY, launch_flux(s, fcur, istep, dt));
     if (istep == 2 && fp64_sensor(s)) TIMED(ST_K_SENSOR, launch_sensor_refine(s, false, true));
     TIMED(ST_K_WENO_FIX, launch_weno_items(s, fcur, istep, dt));
-    if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur));
-    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end, last));
+    if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur, true));
+    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end, stay, !last));
     if (s->p.channel_case && s->p.theta_wall >= -1.0)
-        TIMED(ST_K_FORCE_VAR, launch_force_var(s, one_pass_update_blocks(g)));
-    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s, true));
+        TIMED(ST_K_FORCE_VAR, launch_force_var(s, one_pass_update_blocks(g), !last));
+    if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s, true, !last));
     s->cur ^= 1;
     s->last_stage = istep;
     s->fln_current = false;
@@ -382,11 +384,11 @@ int stage(st_solver *s, int istep) {
 }
 
 // end: the step of st_advance, which also moves time and the step counter;
-// last: no step of the same call follows
-int do_rk_sync(st_solver *s, bool end, bool last) {
+// first, last: no step of the same call before it, after it
+int do_rk_sync(st_solver *s, bool end, bool first, bool last) {
     const bool one = st::one_pass_stage(s);
     for (int istep = 0; istep < 3; istep++) {
-        int rc = one ? stage_one_pass(s, istep, end && istep == 2, last) : stage(s, istep);
+        int rc = one ? stage_one_pass(s, istep, end && istep == 2, first, last) : stage(s, istep);
         if (rc) return rc;
     }
     if (end && !one) TIMED(ST_K_STEP_END, st::launch_step_end(s));
@@ -415,7 +417,7 @@ int partial_head(const st::Geo &g, bool mixed) {
     return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 int partial_total(const st::Geo &g, bool mixed) {
-    return partial_head(g, mixed) + st::aux_dt_blocks(g) + st::kStage2Slots + 128 * 8;
+    return partial_head(g, mixed) + st::one_pass_dt_slots(g) + st::kStage2Slots + 128 * 8;
 }
 
 void array_sizes(const st_params &p, size_t n[kNArrays]) {
@@ -523,7 +525,7 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
         s->stage = &s->own_stage;
     }
     s->dtpart = s->partials + partial_head(g, s->mixed);
-    s->stage2 = s->dtpart + st::aux_dt_blocks(g);
+    s->stage2 = s->dtpart + st::one_pass_dt_slots(g);
     // the first points of w and w_aux sit lead_bytes into their allocations
     s->w_alloc = s->w;
     s->w_aux_alloc = s->w_aux;
@@ -1161,7 +1163,7 @@ int st_rk_sync(st_solver *s) {
         if (rc) return rc;
         return rk_sync_pieces(s, s->hs->dt);
     }
-    return do_rk_sync(s, false, true);
+    return do_rk_sync(s, false, true, true);
 }
 
 int st_advance(st_solver *s, int32_t nsteps) {
@@ -1189,7 +1191,7 @@ int st_advance(st_solver *s, int32_t nsteps) {
             // therefore takes the reduction
             s->dt_in_stage = true;
         }
-        int rc = do_rk_sync(s, true, n + 1 == nsteps);
+        int rc = do_rk_sync(s, true, n == 0, n + 1 == nsteps);
         if (rc) return rc;
     }
     return ST_OK;

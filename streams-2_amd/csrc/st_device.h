@@ -71,30 +71,49 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double (*lds)[NV]) {
     }
 }
 
-// bcwall_staggered_subroutine (kernels_cpu.F90:6612-6678) for one ghost
-// point: the mirror of interior point js, written at jg.
-template <typename R>
-__device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *__restrict__ w,
-                                           const R *__restrict__ wa, int i, int js, int jg, int k) {
-    const int s = gidx(g, i, js, k), d = gidx(g, i, jg, k);
-    const size_t nv = g.nvol;
-    double rho = w[s];
-    const double uu = w[nv + s] / rho;
-    const double vv = w[2 * nv + s] / rho;
-    const double ww = w[3 * nv + s] / rho;
-    const double rhoe = w[4 * nv + s];
+// The viscosity of a conserved state, by the operations of k_aux: whether the
+// aux pass or the kernel that last wrote w formed it must not show in a result.
+__device__ __forceinline__ double mu_of(const KPar &P, const double (&c)[5]) {
+    const double ri = 1.0 / c[0];
+    const double uu = c[1] * ri, vv = c[2] * ri, ww = c[3] * ri;
     const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-    double ee = rhoe / rho - qq;
-    double tt = temperature_from_e(P, ee, double(wa[5 * nv + s]));
+    const double ee = c[4] / c[0] - qq;
+    return viscosity_of(P, temperature_from_e(P, ee, P.t0));
+}
+
+// bcwall_staggered_subroutine (kernels_cpu.F90:6612-6678): the ghost state d
+// that mirrors the state c about an isothermal wall (t_start as in
+// temperature_from_e).
+__device__ __forceinline__ void wall_ghost_of(const KPar &P, const double (&c)[5], double t_start, double (&d)[5]) {
+    double rho = c[0];
+    const double uu = c[1] / rho, vv = c[2] / rho, ww = c[3] / rho;
+    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+    double ee = c[4] / rho - qq;
+    double tt = temperature_from_e(P, ee, t_start);
     const double pp = rho * tt * P.rgas0;
     tt = 2.0 * P.t_wall - tt;
     ee = e_from_temperature(P, tt);
     rho = pp / tt / P.rgas0;
-    w[d] = rho;
-    w[nv + d] = -rho * uu;
-    w[2 * nv + d] = -rho * vv;
-    w[3 * nv + d] = -rho * ww;
-    w[4 * nv + d] = rho * (ee + qq);
+    d[0] = rho;
+    d[1] = -rho * uu;
+    d[2] = -rho * vv;
+    d[3] = -rho * ww;
+    d[4] = rho * (ee + qq);
+}
+// for one ghost point: the mirror of interior point js, written at jg; with mu
+// its viscosity too
+template <typename R>
+__device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *__restrict__ w, R *__restrict__ wa, int i,
+                                           int js, int jg, int k, bool mu) {
+    const int s = gidx(g, i, js, k), d = gidx(g, i, jg, k);
+    const size_t nv = g.nvol;
+    double c[5], x[5];
+#pragma unroll
+    for (int m = 0; m < 5; m++) c[m] = w[m * nv + s];
+    wall_ghost_of(P, c, double(wa[5 * nv + s]), x);
+#pragma unroll
+    for (int m = 0; m < 5; m++) w[m * nv + d] = x[m];
+    if (mu) wa[6 * nv + d] = R(mu_of(P, x));
 }
 
 // exclusive prefix over the block's 256 threads of v; *total receives the sum

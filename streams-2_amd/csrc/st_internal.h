@@ -190,11 +190,11 @@ __device__ __forceinline__ double e_from_temperature(const KPar &P, double tt) {
 
 // viscosity law of eval_aux_subroutine, kernels_cpu.F90:6998-7005
 __device__ __forceinline__ double viscosity_of(const KPar &P, double tt) {
-    if (P.visc_model == 1) return P.mu0 * pow(tt / P.t0, P.vtexp);
-    if (P.visc_model == 2)
-        return P.mu0 * pow(tt / P.t0, 1.5) * (1.0 + P.sutherland_s / P.t_ref_dim) /
-               (tt / P.t0 + P.sutherland_s / P.t_ref_dim);
-    return 0.0;
+    if (P.visc_model != 1 && P.visc_model != 2) return 0.0;
+    // (one pow for both laws: it is most of a kernel's code)
+    const double x = tt / P.t0, m = P.mu0 * pow(x, P.visc_model == 1 ? P.vtexp : 1.5);
+    if (P.visc_model == 1) return m;
+    return m * (1.0 + P.sutherland_s / P.t_ref_dim) / (x + P.sutherland_s / P.t_ref_dim);
 }
 
 }  // namespace st

@@ -95,7 +95,7 @@ __global__ void k_extrapolate_var(Geo g, T *__restrict__ a) {
 }
 
 template <typename R>
-__global__ void k_wall_ghosts(Geo g, KPar P, double *__restrict__ w, const R *__restrict__ wa) {
+__global__ void k_wall_ghosts(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa, int mu) {
     const int tot = 2 * g.ng * g.nx * g.nz;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
         const int i = t % g.nx + 1;
@@ -103,10 +103,10 @@ __global__ void k_wall_ghosts(Geo g, KPar P, double *__restrict__ w, const R *__
         const int l = r % (2 * g.ng);
         const int k = r / (2 * g.ng) + 1;
         if (l < g.ng) {
-            if (P.wall_stag[0]) wall_ghost(g, P, w, wa, i, l + 1, -l, k);
+            if (P.wall_stag[0]) wall_ghost(g, P, w, wa, i, l + 1, -l, k, mu != 0);
         } else {
             const int ll = l - g.ng + 1;
-            if (P.wall_stag[1]) wall_ghost(g, P, w, wa, i, g.ny + 1 - ll, g.ny + ll, k);
+            if (P.wall_stag[1]) wall_ghost(g, P, w, wa, i, g.ny + 1 - ll, g.ny + ll, k, mu != 0);
         }
     }
 }
@@ -143,7 +143,7 @@ __device__ __forceinline__ int face_boundary(const Geo &g, int ilat, int a, int 
 // :6478-6525), oblique shock on ymax (bcshock_subroutine, :6159-6196).
 template <typename R>
 __device__ __forceinline__ void bc_point(const Geo &g, const KPar &P, double *__restrict__ w,
-                                         const R *__restrict__ wa, const double *__restrict__ xc,
+                                         R *__restrict__ wa, const double *__restrict__ xc,
                                          const double *__restrict__ yc, int ilat, int tag, int staggered,
                                          const double *__restrict__ wmean, int a, int b) {
     const size_t nv = g.nvol;
@@ -219,60 +219,67 @@ __device__ __forceinline__ void bc_point(const Geo &g, const KPar &P, double *__
         }
     } else if (tag == 2) {
         const int s0 = face_boundary(g, ilat, a, b);
+        double c[5];
+        for (int m = 0; m < 5; m++) c[m] = w[m * nv + s0];
         for (int l = 1; l <= ng; l++) {
             const int d = face_ghost(g, ilat, a, b, l);
-            for (int m = 0; m < 5; m++) w[m * nv + d] = w[m * nv + s0];
+            for (int m = 0; m < 5; m++) w[m * nv + d] = c[m];
         }
     } else if (tag == 5 && ilat == 3) {
         for (int l = 1; l <= ng; l++) {
             const int d = gidx(g, a, 1 - l, b), s0 = gidx(g, a, 1 + l, b);
-            for (int m = 0; m < 5; m++) w[m * nv + d] = w[m * nv + s0];
+            double c[5];
+            for (int m = 0; m < 5; m++) c[m] = w[m * nv + s0];
+            for (int m = 0; m < 5; m++) w[m * nv + d] = c[m];
         }
     } else if (tag == 6 && staggered) {
         for (int l = 1; l <= ng; l++) {
-            if (ilat == 3) wall_ghost(g, P, w, wa, a, l, 1 - l, b);
-            else if (ilat == 4) wall_ghost(g, P, w, wa, a, g.ny + 1 - l, g.ny + l, b);
+            if (ilat == 3) wall_ghost(g, P, w, wa, a, l, 1 - l, b, false);
+            else if (ilat == 4) wall_ghost(g, P, w, wa, a, g.ny + 1 - l, g.ny + l, b, false);
         }
     } else if (tag == 6 && ilat == 3) {
         const int c1 = gidx(g, a, 1, b);
+        const double r1 = w[c1];
+        // all loads of three ghost layers before the stores (ng is 3 or 4)
+        double c[3][5], t0[3];
+#pragma unroll
+        for (int l = 0; l < 3; l++) {
+            const int s0 = gidx(g, a, 2 + l, b);
+#pragma unroll
+            for (int m = 0; m < 5; m++) c[l][m] = w[m * nv + s0];
+            t0[l] = double(wa[5 * nv + s0]);
+        }
         w[nv + c1] = 0.0;
         w[2 * nv + c1] = 0.0;
         w[3 * nv + c1] = 0.0;
-        double ee = e_from_temperature(P, P.t_wall);
-        w[4 * nv + c1] = w[c1] * ee;
-        for (int l = 1; l <= ng; l++) {
-            const int s0 = gidx(g, a, 1 + l, b), d = gidx(g, a, 1 - l, b);
-            double rho = w[s0];
-            const double uu = w[nv + s0] / rho, vv = w[2 * nv + s0] / rho, ww = w[3 * nv + s0] / rho;
-            const double rhoe = w[4 * nv + s0];
-            const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-            ee = rhoe / rho - qq;
-            double tt = temperature_from_e(P, ee, double(wa[5 * nv + s0]));
-            const double pp = rho * tt * P.rgas0;
-            tt = 2.0 * P.t_wall - tt;
-            ee = e_from_temperature(P, tt);
-            rho = pp / tt / P.rgas0;
-            w[d] = rho;
-            w[nv + d] = -rho * uu;
-            w[2 * nv + d] = -rho * vv;
-            w[3 * nv + d] = -rho * ww;
-            w[4 * nv + d] = rho * (ee + qq);
+        w[4 * nv + c1] = r1 * e_from_temperature(P, P.t_wall);
+#pragma unroll
+        for (int l = 0; l < 3; l++) {
+            double x[5];
+            wall_ghost_of(P, c[l], t0[l], x);
+#pragma unroll
+            for (int m = 0; m < 5; m++) w[m * nv + gidx(g, a, -l, b)] = x[m];
         }
+        for (int l = 4; l <= ng; l++) wall_ghost(g, P, w, wa, a, 1 + l, 1 - l, b, false);
     } else if (tag == 7 && ilat == 4) {
         const double tanhlen = 8.0 * P.tanhfacs;
         const int i = a, k = b;
         const int cn = gidx(g, i, g.ny, k);
+        double c[5];  // the cell, as the face leaves it
+        for (int m = 0; m < 5; m++) c[m] = w[m * nv + cn];
         for (int l = 0; l <= ng; l++) {
             const double xsh = P.xshock_imp - yc[g.ny + l + ng - 1] / tan(P.shock_angle);
             const double xx = xc[i + ng - 1] - xsh;
             const int d = gidx(g, i, g.ny + l, k);
             if (fabs(xx) > tanhlen) {
-                for (int m = 0; m < 5; m++) w[m * nv + d] = w[m * nv + cn];
+                for (int m = 0; m < 5; m++) w[m * nv + d] = c[m];
             } else {
                 const double tanhf = 0.5 * (1.0 + tanh(xx / P.tanhfacs));
                 for (int m = 0; m < 5; m++) {
                     const double dwinf = P.winf_ps[m] - P.winf[m];
-                    w[m * nv + d] = P.winf[m] + dwinf * tanhf;
+                    const double x = P.winf[m] + dwinf * tanhf;
+                    w[m * nv + d] = x;
+                    if (l == 0) c[m] = x;
                 }
             }
         }
@@ -284,7 +291,8 @@ __device__ __forceinline__ void bc_point(const Geo &g, const KPar &P, double *__
 // one-sided derivative of w along the normal in characteristic variables
 // at the boundary state, scaled by the (clipped) eigenvalues, back through
 // the right eigenvectors into fl.
-template <typename R, int DIR>
+// The boundary state from w_aux, or with FROMW from w (the one-pass stage).
+template <typename R, int DIR, bool FROMW>
 __global__ void k_bc_nr(Geo g, KPar P, const double *__restrict__ w, const R *__restrict__ wa, R *__restrict__ fl,
                         const double *__restrict__ metric, int start, int nr_type) {
     const int na = DIR == 0 ? g.ny : g.nx;
@@ -312,8 +320,23 @@ __global__ void k_bc_nr(Geo g, KPar P, const double *__restrict__ w, const R *__
         else if (nr_type == 3) w_target = P.winf[m];
         dw_dn_outer[m] = sgn * (wm[c] - w_target);
     }
-    const double rho = wa[c], uu = wa[nv + c], vv = wa[2 * nv + c], ww = wa[3 * nv + c];
-    const double h = wa[4 * nv + c], tt = wa[5 * nv + c];
+    double rho, uu, vv, ww, h, tt;
+    if (FROMW) {
+        rho = w[c];
+        const double ri = 1.0 / rho, rhoe = w[4 * nv + c];
+        uu = w[nv + c] * ri;
+        vv = w[2 * nv + c] * ri;
+        ww = w[3 * nv + c] * ri;
+        tt = temperature_from_e(P, rhoe / rho - 0.5 * (uu * uu + vv * vv + ww * ww), P.t0);
+        h = (rhoe + rho * tt * P.rgas0) / rho;
+    } else {
+        rho = wa[c];
+        uu = wa[nv + c];
+        vv = wa[2 * nv + c];
+        ww = wa[3 * nv + c];
+        h = wa[4 * nv + c];
+        tt = wa[5 * nv + c];
+    }
     const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
     const double gamloc = gamloc_of(P, tt);
     const double cc = gamloc * tt * P.rgas0;
@@ -403,15 +426,22 @@ __device__ __forceinline__ void recyc_sum(const Geo &g, const double *__restrict
     const int i = t % g.ng + 1, j = (t / g.ng) % g.ny + 1, m = t / (g.ng * g.ny);
     const double *wm = w + (size_t)m * g.nvol;
     auto at = [&](int k) { return wm[gidx(g, i_recyc + 1 - i, j, recyc_k(k, g.nz))]; };
-    // the loads are issued sixteen at a time ahead of the additions
+    // the loads are issued many at a time ahead of the additions
     double a = 0.0;
     int k = 1;
-    for (; k + 15 <= g.nz; k += 16) {
-        double v[16];
+    for (; k + 31 <= g.nz; k += 32) {
+        double v[32];
 #pragma unroll
-        for (int q = 0; q < 16; q++) v[q] = at(k + q);
+        for (int q = 0; q < 32; q++) v[q] = at(k + q);
 #pragma unroll
-        for (int q = 0; q < 16; q++) a = a + v[q];
+        for (int q = 0; q < 32; q++) a = a + v[q];
+    }
+    for (; k + 7 <= g.nz; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = at(k + q);
+#pragma unroll
+        for (int q = 0; q < 8; q++) a = a + v[q];
     }
     for (; k <= g.nz; k++) a = a + at(k);
     av[(i - 1) + g.ng * ((j - 1) + g.ny * m)] = a;
@@ -429,8 +459,9 @@ struct Inflow {
     const double *wrecyc, *rplane;
     double betarecyc, u0_02;
 };
-__device__ __forceinline__ void recyc_inflow(const Geo &g, const KPar &P, double *__restrict__ w, const Inflow &I, int i,
-                                             int t) {
+template <typename R>
+__device__ __forceinline__ void recyc_inflow(const Geo &g, const KPar &P, double *__restrict__ w, R *__restrict__ wa,
+                                             const Inflow &I, int i, int t, bool mu) {
     const double *rc = I.rc, *wrecyc = I.wrecyc, *rplane = I.rplane;
     const int *maps = I.maps;
     const double betarecyc = I.betarecyc, u0_02 = I.u0_02;
@@ -494,11 +525,9 @@ __device__ __forceinline__ void recyc_inflow(const Geo &g, const KPar &P, double
     const double rhou = rho * uu, rhov = rho * vv, rhow = rho * ww;
     const double ee = e_from_temperature(P, tt);
     const int d = gidx(g, 1 - i, j, k);
-    w[d] = rho;
-    w[nv + d] = rhou;
-    w[2 * nv + d] = rhov;
-    w[3 * nv + d] = rhow;
-    w[4 * nv + d] = rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho;
+    const double x[5] = {rho, rhou, rhov, rhow, rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho};
+    for (int m = 0; m < 5; m++) w[m * nv + d] = x[m];
+    if (mu) wa[6 * nv + d] = R(mu_of(P, x));
 }
 
 // ------------------------------------------------------ random inflow plane
@@ -569,23 +598,24 @@ __global__ __launch_bounds__(256) void k_recyc_gather(Geo g, const double *__res
 // and read interior cells, but the node wall and the impinging shock also
 // change the row of cells they stand on.  After the x faces, in the order of
 // the reference: there the thread of the row's first or last cell first does
-// the x face's point of that cell (take), and the x face leaves it out.
+// the x face's point of that cell (take), and the x face leaves it out.  With
+// mu the viscosity of every point that was written follows.
 struct FaceSet {
     int n;
     int first[7], ilat[7], tag[7];
     bool take[2];  // ymin, ymax
 };
 template <typename R>
-__global__ __launch_bounds__(128) void k_bc_faces(Geo g, KPar P, double *__restrict__ w, const R *__restrict__ wa,
+__global__ __launch_bounds__(128) void k_bc_faces(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa,
                                                   const double *__restrict__ xc, const double *__restrict__ yc,
-                                                  int staggered, FaceSet F, Inflow I) {
+                                                  int staggered, int mu, FaceSet F, Inflow I) {
     int q = 0, blk = blockIdx.x;
     while (q + 1 < F.n && blk >= F.first[q + 1]) q++;
     const int t = (blk - F.first[q]) * 128 + threadIdx.x;
     const int ilat = F.ilat[q];
     if (ilat == 0) {
         const int np = g.ny * g.nz;
-        if (t < np * g.ng) recyc_inflow(g, P, w, I, t / np + 1, t % np);
+        if (t < np * g.ng) recyc_inflow(g, P, w, wa, I, t / np + 1, t % np, mu != 0);
         return;
     }
     const int na = ilat <= 2 ? g.ny : g.nx;
@@ -599,7 +629,22 @@ __global__ __launch_bounds__(128) void k_bc_faces(Geo g, KPar P, double *__restr
         const int lat = F.ilat[o];
         const bool own = o == q;
         if (!own && !((lat == 1 && a == 1) || (lat == 2 && a == g.nx))) continue;
-        bc_point(g, P, w, wa, xc, yc, lat, F.tag[o], staggered, I.rc, own ? a : (ilat == 3 ? 1 : g.ny), b);
+        const int at = own ? a : (ilat == 3 ? 1 : g.ny);
+        bc_point(g, P, w, wa, xc, yc, lat, F.tag[o], staggered, I.rc, at, b);
+        if (!mu) continue;
+        // the boundary cell, if it was changed, and its three ghosts at once
+        double x[4][5];
+        int at_[4];
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            at_[l] = l == 0 ? face_boundary(g, lat, at, b) : face_ghost(g, lat, at, b, l);
+#pragma unroll
+            for (int m = 0; m < 5; m++) x[l][m] = w[(size_t)m * g.nvol + at_[l]];
+        }
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            if (l > 0 || (own && takes)) wa[6 * (size_t)g.nvol + at_[l]] = R(mu_of(P, x[l]));
+        }
     }
 }
 
@@ -2776,8 +2821,8 @@ __device__ __forceinline__ void k_update_body(const dim3 blockIdx, const dim3 gr
             wa[5 * nv + c] = R(tt);
             acc[0] = wn[1] * tt * dy;
         } else {
-            if (P.wall_stag[0] && j <= g.ng) wall_ghost(g, P, w, wa, i, j, 1 - j, k);
-            if (P.wall_stag[1] && j > g.ny - g.ng) wall_ghost(g, P, w, wa, i, j, 2 * g.ny + 1 - j, k);
+            if (P.wall_stag[0] && j <= g.ng) wall_ghost(g, P, w, wa, i, j, 1 - j, k, false);
+            if (P.wall_stag[1] && j > g.ny - g.ng) wall_ghost(g, P, w, wa, i, j, 2 * g.ny + 1 - j, k, false);
         }
     }
     if (FORCE_VAR) {
@@ -2809,8 +2854,8 @@ __global__ __launch_bounds__(RED_THREADS) void k_force_var_finish(KPar P, const 
 
 // force_var_2_subroutine (kernels_cpu.F90:3282-3314) + wall ghosts
 template <typename R>
-__global__ __launch_bounds__(256) void k_force_var2(Geo g, KPar P, double *__restrict__ w, const R *__restrict__ wa,
-                                                    const DevScalars *__restrict__ ds) {
+__global__ __launch_bounds__(256) void k_force_var2(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa,
+                                                    const DevScalars *__restrict__ ds, int mu) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
@@ -2820,7 +2865,9 @@ __global__ __launch_bounds__(256) void k_force_var2(Geo g, KPar P, double *__res
     const double rho = w[c], rhou = w[nv + c], rhov = w[2 * nv + c], rhow = w[3 * nv + c];
     const double ttnew = double(wa[5 * nv + c]) + ds->bulkt;
     const double ee = e_from_temperature(P, ttnew);
-    w[4 * nv + c] = rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho;
+    const double x[5] = {rho, rhou, rhov, rhow, rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho};
+    w[4 * nv + c] = x[4];
+    if (mu) wa[6 * nv + c] = R(mu_of(P, x));
 }
 
 // ------------------------------------------------------------ statistics
@@ -3417,13 +3464,13 @@ hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int 
     return hipGetLastError();
 }
 
-hipError_t launch_wall_ghosts(st_solver *s) {
+hipError_t launch_wall_ghosts(st_solver *s, bool mu) {
     ST_NOREC();
     const Geo &g = s->g;
     if (!s->kp.wall_stag[0] && !s->kp.wall_stag[1]) return hipSuccess;
     size_t tot = (size_t)2 * g.ng * g.nx * g.nz;
     ST_DISPATCH(hipLaunchKernelGGL(k_wall_ghosts<R>, dim3(grid1d(tot, 256)), dim3(256), 0, s->stream, g, s->kp, s->w,
-                                   (const R *)s->w_aux));
+                                   (R *)s->w_aux, mu ? 1 : 0));
     return hipGetLastError();
 }
 
@@ -3740,7 +3787,7 @@ hipError_t launch_rng_reset(st_solver *s) {
     return hipGetLastError();
 }
 
-hipError_t launch_physical_ghosts(st_solver *s, bool draws) {
+hipError_t launch_physical_ghosts(st_solver *s, bool draws, bool mu) {
     ST_NOREC();
     const Geo &g = s->g;
     Inflow I{};
@@ -3756,7 +3803,7 @@ hipError_t launch_physical_ghosts(st_solver *s, bool draws) {
     };
     auto launch = [&]() {
         ST_DISPATCH(hipLaunchKernelGGL(k_bc_faces<R>, dim3(blocks), dim3(128), 0, s->stream, g, s->kp, s->w,
-                                       (const R *)s->w_aux, s->x, s->y, s->p.is_y_staggered, F, I));
+                                       (R *)s->w_aux, s->x, s->y, s->p.is_y_staggered, mu ? 1 : 0, F, I));
         F = FaceSet{};
         blocks = 0;
         return hipGetLastError();
@@ -3793,38 +3840,39 @@ hipError_t launch_physical_ghosts(st_solver *s, bool draws) {
     return F.n ? launch() : hipSuccess;
 }
 
-hipError_t launch_bc_nr(st_solver *s, void *fl) {
+hipError_t launch_bc_nr(st_solver *s, void *fl, bool from_w) {
     ST_NOREC();
     const Geo &g = s->g;
+    const double *met[3] = {s->dcsidx, s->detady, s->dzitdz};
     for (int ilat = 1; ilat <= 2 * s->kp.ndim; ilat++) {
         const int nr = s->kp.nrtag[ilat - 1];
         if (nr == 0) continue;
         const int dir = (ilat - 1) / 2, start = (ilat - 1) % 2 == 0 ? 1 : 0;
         const int n = (dir == 0 ? g.ny : g.nx) * (dir == 2 ? g.ny : g.nz);
-        const dim3 grid((n + 127) / 128), block(128);
-        if (dir == 0)
-            ST_DISPATCH(hipLaunchKernelGGL((k_bc_nr<R, 0>), grid, block, 0, s->stream, g, s->kp, s->w,
-                                           (const R *)s->w_aux, (R *)fl, s->dcsidx, start, nr));
-        else if (dir == 1)
-            ST_DISPATCH(hipLaunchKernelGGL((k_bc_nr<R, 1>), grid, block, 0, s->stream, g, s->kp, s->w,
-                                           (const R *)s->w_aux, (R *)fl, s->detady, start, nr));
-        else
-            ST_DISPATCH(hipLaunchKernelGGL((k_bc_nr<R, 2>), grid, block, 0, s->stream, g, s->kp, s->w,
-                                           (const R *)s->w_aux, (R *)fl, s->dzitdz, start, nr));
+#define ST_LAUNCH_NR(D_, W_)                                                                                      \
+    ST_DISPATCH(hipLaunchKernelGGL((k_bc_nr<R, D_, W_>), dim3((n + 127) / 128), dim3(128), 0, s->stream, g, s->kp, \
+                                   s->w, (const R *)s->w_aux, (R *)fl, met[D_], start, nr))
+        if (dir == 0 && from_w) ST_LAUNCH_NR(0, true);
+        else if (dir == 0) ST_LAUNCH_NR(0, false);
+        else if (dir == 1 && from_w) ST_LAUNCH_NR(1, true);
+        else if (dir == 1) ST_LAUNCH_NR(1, false);
+        else if (from_w) ST_LAUNCH_NR(2, true);
+        else ST_LAUNCH_NR(2, false);
+#undef ST_LAUNCH_NR
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
-hipError_t launch_force_var(st_solver *s, int nblk) {
+hipError_t launch_force_var(st_solver *s, int nblk, bool mu) {
     ST_NOREC();
     const Geo &g = s->g;
     hipLaunchKernelGGL(k_force_var_finish, dim3(red_blocks(nblk)), dim3(RED_THREADS), 0, s->stream, s->kp,
                        s->partials, nblk, s->partials + s->npart - RB * 8, s->counters + 1, s->ds);
     ST_DISPATCH(hipLaunchKernelGGL(k_force_var2<R>, cell_grid(g), kCellBlock, 0, s->stream, g, s->kp, s->w,
-                                   (const R *)s->w_aux, s->ds));
-    return launch_wall_ghosts(s);
+                                   (R *)s->w_aux, s->ds, mu ? 1 : 0));
+    return launch_wall_ghosts(s, mu);
 }
 
 int dt_blocks_per_plane(const Geo &g) { return ((g.nx + 63) / 64) * ((g.ny + 3) / 4); }
@@ -3992,7 +4040,7 @@ hipError_t launch_force_var_piece(st_solver *s) {
     hipLaunchKernelGGL(k_force_var_finish, dim3(red_blocks(cell_blocks(g))), dim3(RED_THREADS), 0, s->stream, s->kp,
                        s->partials, cell_blocks(g), s->partials + s->npart - RB * 8, s->counters + 1, s->ds);
     ST_DISPATCH(hipLaunchKernelGGL(k_force_var2<R>, cell_grid(g), kCellBlock, 0, s->stream, g, s->kp, s->w,
-                                   (const R *)s->w_aux, s->ds));
+                                   (R *)s->w_aux, s->ds, 0));
     return hipGetLastError();
 }
 

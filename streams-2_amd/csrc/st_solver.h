@@ -68,6 +68,7 @@ struct st_solver {
     bool dt_in_stage;   // the CFL reduction of this step rides on the first stage's aux
     int visc_chunk;     // planes per tile of the z-marching viscous kernel (0: automatic)
     int march_chunk;    // points per thread of the y/z flux marches (0: automatic)
+    int dt_nblk;        // CFL block maxima of the last launch_flux that took them
     bool x_uniform;     // dcsidx is one value (set by st_set_grid)
     bool fuse_xy;       // x and y Euler fluxes in one pass
     bool fuse_zv;       // viscous divergence terms folded into the z march (Laplacian form)
@@ -195,13 +196,14 @@ hipError_t launch_extrapolate_aux(st_solver *s, int var);
 hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image,
                       bool dt = false, bool defer_dt = false, bool enthalpy = true);
 int aux_dt_blocks(const Geo &g);  // block maxima of an aux pass over the ghosted box
-hipError_t launch_wall_ghosts(st_solver *s);
+hipError_t launch_wall_ghosts(st_solver *s, bool mu = false);
 // physical ghosts of every non-periodic face in the order xmin..zmax
 // (update_ghost without the periodic swap), recyc_exchange and the recycled
-// inflow included; draws: first redraw the random inflow plane
-hipError_t launch_physical_ghosts(st_solver *s, bool draws);
+// inflow included; draws: first redraw the random inflow plane; mu: also
+// w_aux(7) of the points written (as in the wall ghosts and force_var)
+hipError_t launch_physical_ghosts(st_solver *s, bool draws, bool mu = false);
 // characteristic boundary treatment added to fl (bc_nr)
-hipError_t launch_bc_nr(st_solver *s, void *fl);
+hipError_t launch_bc_nr(st_solver *s, void *fl, bool from_w = false);
 // the random inflow plane: redraw rows 2..jbl (after a z sweep), and the
 // generator window reset to its seeded state
 hipError_t launch_inflow_draws(st_solver *s);
@@ -236,7 +238,7 @@ hipError_t launch_visc_div(st_solver *s, void *fl, const void *fl_prev, int stag
 hipError_t launch_force_finish(st_solver *s, int stage);
 hipError_t launch_update(st_solver *s, const void *fl_prev, const void *fl, int stage);
 // nblk block sums of rho*u*T*dy from the update
-hipError_t launch_force_var(st_solver *s, int nblk);
+hipError_t launch_force_var(st_solver *s, int nblk, bool mu = false);
 int update_blocks(const Geo &g);
 // ---- one-pass stage (st_stage.hip)
 bool one_pass_stage(const st_solver *s);
@@ -245,15 +247,16 @@ size_t hot_rec_bytes(const Geo &g);
 size_t hot_dirty_bytes(const Geo &g);
 int one_pass_flux_slots(const Geo &g, bool mixed);
 int one_pass_update_blocks(const Geo &g);
+int one_pass_dt_slots(const Geo &g);
 constexpr int kStage2Slots = 512 * 6;  // second-level values of k_weno_items
 // the step's WENO masks and work items from w_aux(8)
 hipError_t launch_hot_items(st_solver *s);
 // the whole right-hand side but grad(div/3) and the WENO faces
-hipError_t launch_flux(st_solver *s, void *fl, int stage);
+hipError_t launch_flux(st_solver *s, void *fl, int stage, bool dt);
 // WENO faces; bulk sums of force_rhs and, with dt, the CFL step finished
 hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt);
 // grad(div/3), update_flux, update_field, wall ghosts; the end of the step
-hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last);
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last, bool mu);
 hipError_t launch_dt(st_solver *s);
 hipError_t launch_step_end(st_solver *s);
 hipError_t launch_residual(st_solver *s);

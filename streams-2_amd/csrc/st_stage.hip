@@ -4,16 +4,22 @@
 // every other solve runs the separate sweeps of st_kernels.hip.
 //
 // One stage is
-//   aux      w -> w_aux(1:7) over the ghosted box (st_kernels.hip)
 //   flux     x, y and z central fluxes and the viscous terms of every cell in
-//            one march along z, the bulk sums of force_rhs, and at the third
-//            stage the Ducros sensor
+//            one march along z, the bulk sums of force_rhs, the CFL radii where
+//            the step recomputes dt, and at the third stage the Ducros sensor
 //   items    WENO faces of the flagged cells; the last workgroup finishes the
 //            bulk sums (dpdx) and, at the first stage, the CFL step
-//   update   grad(div/3) terms, w += fln with the forcing, wall ghosts
+//   update   grad(div/3) terms, w += fln with the forcing, wall ghosts, and
+//            the viscosity of the new state
 // and at the first stage of a step two kernels turn the sensor into bit masks
 // and into the list of WENO work items, which the three stages share (the
-// reference switches on the sensor of the previous step's last stage).
+// reference switches on the sensor of the previous step's last stage).  All of
+// them form the primitives from w; of w_aux they read the viscosity (its power
+// law is the one costly primitive, and whoever changes w stores it), the sensor
+// and div/3.  The aux pass (w -> w_aux(1:7) over the ghosted box,
+// st_kernels.hip) runs at the last stage of a call alone, whose w_aux the
+// caller can read, and at the first, for the viscosity of a w that anyone may
+// have set.
 #include "st_device.h"
 #include "st_flux.h"
 #include "st_solver.h"
@@ -184,6 +190,14 @@ __device__ __forceinline__ int opaque(int v) {
     return v;
 }
 
+// A value that is the same in every lane, held in scalar registers: what FP64
+// arithmetic makes of kernel arguments would otherwise fill vector ones.
+__device__ __forceinline__ double uniform(double v) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+
 // A point's stencil values: rho, u, v, w, T, mu, and in the mixed form the
 // stored deviation p - p_ref (in FP64 the pressure is rho*T*R).
 constexpr int VR = 0, VU = 1, VT = 4, VM = 5, VP_ = 6;
@@ -223,7 +237,11 @@ struct FluxConst {
     R c[H], c2[H + 1];  // first- and second-derivative weights (the viscous terms; Euler along z)
     R rg, pref;         // pressure = rg * sp_press + pref
     R ea, eb;           // internal energy = ea + eb T
+    R rg4, ea2, eb4;    // 4 rg, 2 ea, eb / 4
     R cpr;              // cp / Pr
+    R gamr, prm1;       // c^2 = gamr T, 1 / Pr
+    double ta, tb;      // T = ta + tb e
+    double rgas, p0;    // stored p - p_ref of the mixed form = rgas rho T - p0
 };
 
 // The central flux difference of the cell along direction D, and its viscous
@@ -284,8 +302,8 @@ __device__ __forceinline__ R flux_dir(const FluxConst<R> &K, const SP<R> &o, con
         lt += c2 * p.a[VT];
     });
     const R mu4 = R(-4) * o.a[VM];
-    (D == 0 ? mu_ : (D == 1 ? mv : mw)) += (R(4) * K.rg) * ps;
-    A.e += am * (R(0.25) * K.eb * mt + pr * (D == 2 ? gw : gn));
+    (D == 0 ? mu_ : (D == 1 ? mv : mw)) += K.rg4 * ps;
+    A.e += am * (K.eb4 * mt + pr * (D == 2 ? gw : gn));
     gu *= a1; gv *= a1; gw *= a1; gt *= a1; gm *= a1;
     A.m += am * m;
     A.mk[0] += am * mu_ + mu4 * (lu * s1 + gu * q1);
@@ -334,8 +352,8 @@ __device__ __forceinline__ R flux_dir_cons(const FluxConst<R> &K, const SP<R> &o
             A.e -= f * ((p.a[VT] - o.a[VT]) * K.cpr + R(0.5) * k2);
         }
     });
-    (D == 0 ? mu_ : (D == 1 ? mv : mw)) += (R(4) * K.rg) * ps;
-    A.e += am * (R(0.25) * K.eb * mt + pr * gn);
+    (D == 0 ? mu_ : (D == 1 ? mv : mw)) += K.rg4 * ps;
+    A.e += am * (K.eb4 * mt + pr * gn);
     A.m += am * m;
     A.mk[0] += am * mu_;
     A.mk[1] += am * mv;
@@ -377,7 +395,7 @@ __device__ __forceinline__ void edge_cell(const Get &at, const SP<R> &o, unsigne
 #pragma unroll
         for (int x = 0; x < 3; x++) f[1 + x] += uv * (A.a[VU + x] + B.a[VU + x]);
         f[1 + D] += W.p[l - 1] * (pA + pB);
-        f[4] += uv * (R(2) * K.ea + K.eb * (A.a[VT] + B.a[VT]) + A.a[VU] * B.a[VU] + A.a[VU + 1] * B.a[VU + 1] +
+        f[4] += uv * (K.ea2 + K.eb * (A.a[VT] + B.a[VT]) + A.a[VU] * B.a[VU] + A.a[VU + 1] * B.a[VU + 1] +
                       A.a[VU + 2] * B.a[VU + 2]) +
                 W.e[l - 1] * (una * (pB + K.pref) + unb * (pA + K.pref));
     };
@@ -405,6 +423,10 @@ template <typename R>
 constexpr int kFluxWaves = sizeof(R) == sizeof(double) ? 2 : 3;
 
 constexpr int kFluxMaxChunk = 32;
+// FP64 also takes the CFL radii, from the point it holds; the mixed form's
+// points are rounded, and its radii are those of an aux pass in FP64
+template <typename R>
+constexpr bool kFluxDt = sizeof(R) == sizeof(double);
 
 struct FluxArgs {
     const double *dx1, *dxs, *dx2, *dy1, *dys, *dy2, *dz1, *dzs, *dz2;  // metrics
@@ -413,6 +435,7 @@ struct FluxArgs {
     const uint3 *dirty;   // cells with a WENO face (k_hot_items)
     const double *w;
     double *wallprop;
+    double *dtpart;       // block maxima of the CFL radii (null: no new dt)
     double *partials;     // 5 block sums of force_rhs (SUMS)
     int chunk;
     int last;             // third stage: |omega| and the sensor are written
@@ -422,17 +445,21 @@ struct FluxArgs {
 // each lane keeps its 7-plane z stencil in registers, the x and y stencils
 // come from an LDS copy of the current plane with a 3-point halo (two
 // buffers, one barrier a plane).  All three directions read the same six
-// values of a point, so w_aux is read once a stage and the right-hand side is
-// written once; the separate passes (x + y sweep, viscous march, z march)
-// moved 96 + 120 + 152 B a cell, this one 48 + 48.  Two waves per SIMD: the z
+// values of a point, so the state is read once a stage and the right-hand side
+// is written once; the separate passes (aux, x + y sweep, viscous march, z
+// march) moved 96 + 96 + 120 + 152 B a cell, this one 48 + 48.  Two waves per SIMD: the z
 // window, the look-ahead and the accumulators fill 256 registers, so what a
-// lane can re-read (offsets, metrics, running sums) stays in LDS; a spilled
-// look-ahead load (waited for at once to be stored) cost 2x.
-// Bound by FP64 issue: ~830 vector instructions a wave and plane, 4.4 cycles
+// lane can re-read (offsets, metrics, running sums) stays in LDS, and what is
+// uniform in scalar registers; a spilled look-ahead load (waited for at once to
+// be stored) cost 2x.
+// The primitives are formed from w as a point enters the window or the halo,
+// about 20 operations each for two points a lane and plane: 512 x 256 x 256
+// 1.25 -> 1.36 ms, for the aux pass of 0.60 ms and half of the reads.
+// Bound by FP64 issue: ~870 vector instructions a wave and plane, 4.4 cycles
 // each at the ~2.0 GHz of a loaded chip (59 TFLOP/s of FMAs measured), 77 % of
-// the kernel's time.  512 x 256 x 256, with the bulk sums: 1.29 ms, where the
-// passes it replaces took 0.85 + 0.99 + 1.37; 128 x 96 x 64: 49 us for 38 + 35
-// + 41.  Mixed, 256 x 192 x 128: 189 us for 124 + 115 + 175.
+// the kernel's time.  512 x 256 x 256, with the bulk sums: 1.36 ms, where the
+// passes it replaces took 0.64 + 0.85 + 0.99 + 1.37; 128 x 96 x 64: 52 us for
+// 20 + 38 + 35 + 41.  Mixed, 256 x 192 x 128: 203 us for 131 + 124 + 115 + 175.
 template <typename T>
 __device__ __forceinline__ T at_off(const T *__restrict__ base, unsigned bytes) {
     return *(const T *)((const char *)base + bytes);
@@ -441,19 +468,36 @@ template <typename T>
 __device__ __forceinline__ void put_off(T *__restrict__ base, unsigned bytes, T v) {
     *(T *)((char *)base + bytes) = v;
 }
-// a point of one plane: `plane` its (uniform) start, `off` the lane's byte
-// offset in it (a plane is far below 4 GiB)
+// a point of one plane of w and of the viscosity: `plane` and `mu` their
+// (uniform) starts, `off` the lane's byte offset in w's (a plane is far below
+// 4 GiB)
 template <typename R>
-__device__ __forceinline__ SP<R> load_sp(const R *__restrict__ plane, size_t nv, unsigned off) {
+struct Raw {
+    double c[5];
+    R mu;
+};
+template <typename R>
+__device__ __forceinline__ Raw<R> load_raw(const double *__restrict__ plane, const R *__restrict__ mu, size_t nv,
+                                           unsigned off) {
+    Raw<R> p;
+#pragma unroll
+    for (int m = 0; m < 5; m++) p.c[m] = at_off(plane + m * nv, off);
+    p.mu = at_off(mu, sizeof(R) == sizeof(double) ? off : off >> 1);
+    return p;
+}
+// eval_aux (kernels_cpu.F90:6960-7011) for a calorically perfect gas
+template <typename R>
+__device__ __forceinline__ SP<R> primitives(const FluxConst<R> &K, const Raw<R> &x) {
     SP<R> p;
-
-    p.a[VR] = at_off(plane, off);
-    p.a[VU] = at_off(plane + nv, off);
-    p.a[VU + 1] = at_off(plane + 2 * nv, off);
-    p.a[VU + 2] = at_off(plane + 3 * nv, off);
-    p.a[VT] = at_off(plane + 5 * nv, off);
-    p.a[VM] = at_off(plane + 6 * nv, off);
-    if constexpr (sizeof(R) != sizeof(double)) p.a[VP_] = at_off(plane + 10 * nv, off);
+    const double ri = 1.0 / x.c[0], u = x.c[1] * ri, v = x.c[2] * ri, w = x.c[3] * ri;
+    const double t = K.ta + K.tb * (x.c[4] * ri - 0.5 * (u * u + v * v + w * w));
+    p.a[VR] = R(x.c[0]);
+    p.a[VU] = R(u);
+    p.a[VU + 1] = R(v);
+    p.a[VU + 2] = R(w);
+    p.a[VT] = R(t);
+    p.a[VM] = x.mu;
+    if constexpr (sizeof(R) != sizeof(double)) p.a[VP_] = R(x.c[0] * t * K.rgas - K.p0);
     return p;
 }
 
@@ -476,6 +520,7 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
     __shared__ unsigned sedge[2][TX * TY];  // edge_cell's face orders along x and y
     __shared__ R scd[H][H];
     __shared__ R swx[H][TX], swy[H][TY];    // Euler weights of the tile's columns and rows
+    __shared__ double sdt[kFluxDt<R> ? TX * TY : 1];  // running CFL maximum of each lane
     const int tx = threadIdx.x, ty = threadIdx.y;
     // band of whole tile rows per XCD (workgroups are dealt round-robin to the
     // 8 XCDs): the halo points then mostly come from the XCD's own L2
@@ -499,7 +544,16 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
     // offsets in a plane: this lane's point, its halo point (lanes 0 ..
     // 2H*TX-1 the y halo rows, the next 2H*TY lanes the x halo columns, the
     // rest none) and its cell of the right-hand side
-    soff[0][tid] = (unsigned)sizeof(R) * (unsigned)((min(i, g.nx + H) + ng - 1) + g.sx * (min(j, g.ny + H) + ng - 1));
+    // (ghost points of periodic directions at their images, which are what
+    // bcswap would have copied there)
+    auto source = [&](int x, int y) {
+        x = min(x, g.nx + H);
+        y = min(y, g.ny + H);
+        if (P.periodic[0]) x = x < 1 ? x + g.nx : (x > g.nx ? x - g.nx : x);
+        if (P.periodic[1]) y = y < 1 ? y + g.ny : (y > g.ny ? y - g.ny : y);
+        return (unsigned)sizeof(double) * (unsigned)((x + ng - 1) + g.sx * (y + ng - 1));
+    };
+    soff[0][tid] = source(i, j);
     soff[2][tid] = (unsigned)sizeof(R) * (unsigned)((ic - 1) + g.nx * (jc - 1));
     const bool hl = tid < 2 * H * (TX + TY);
     int hlx = tx + H, hly = ty + H;
@@ -512,13 +566,16 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
         hly = q / (2 * H) + H;
         hlx = c6 < H ? c6 : c6 + TX;
     }
-    soff[1][tid] = (unsigned)sizeof(R) *
-        (unsigned)((min(bx * TX + 1 - H + hlx, g.nx + H) + ng - 1) + g.sx * (min(by * TY + 1 - H + hly, g.ny + H) + ng - 1));
+    soff[1][tid] = source(bx * TX + 1 - H + hlx, by * TY + 1 - H + hly);
     const int hslot = hly * (TX + 2 * H) + hlx;
     // (indices for the rare branches, formed there)
     auto li = [&]() { return bx * TX + opaque(tx) + 1; };
     auto lj = [&]() { return by * TY + opaque(ty) + 1; };
     auto plane = [&](int k) { return wa + (ptrdiff_t)(k + ng - 1) * g.sxy; };
+    auto load = [&](int k, unsigned off) {  // z is periodic
+        const ptrdiff_t z = (ptrdiff_t)((k < 1 ? k + g.nz : (k > g.nz ? k - g.nz : k)) + ng - 1) * g.sxy;
+        return load_raw(F.w + z, (const R *)(wa + 6 * nv + z), nv, off);
+    };
     // cells beside a non-periodic boundary: faces of lowered order or zero flux
     const int lb = P.lmax_base;
     const bool inx = i >= P.eul_lo[0] && i <= P.eul_hi[0], iny = j >= P.eul_lo[1] && j <= P.eul_hi[1];
@@ -555,8 +612,17 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
     K.pref = R(sizeof(R) == sizeof(double) ? 0.0 : P.p_ref);
     // e_from_temperature of a calorically perfect gas
     K.eb = R(cvc(P, 0));
-    K.ea = R(P.t0 * (cvc(P, P.indx_cp_r + 1) - cvc(P, 0)));
-    K.cpr = R(cpc(P, 0) / P.prandtl);
+    K.ea = uniform(R(P.t0 * (cvc(P, P.indx_cp_r + 1) - cvc(P, 0))));
+    K.ea2 = uniform(R(2) * K.ea);
+    K.eb4 = uniform(R(0.25) * K.eb);
+    K.rg4 = uniform(R(4) * K.rg);
+    K.cpr = uniform(R(cpc(P, 0) / P.prandtl));
+    K.tb = uniform(1.0 / cvc(P, 0));
+    K.ta = uniform(P.t0 - cvc(P, P.indx_cp_r + 1) * P.t0 * K.tb);
+    K.gamr = uniform(R(cpc(P, 0) / (cpc(P, 0) - P.rgas0) * P.rgas0));
+    K.prm1 = uniform(R(1.0 / P.prandtl));
+    K.rgas = P.rgas0;
+    K.p0 = P.p_ref;
     if (tid < TX) {
         const int q = min(bx * TX + tid + 1, g.nx);
         smx[0][tid] = R(F.dx1[q - 1]);
@@ -612,16 +678,17 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
             if (hl) (&tiles[b][q][0][0])[hslot] = halo.a[q];
         }
     };
-    SP<R> win[2 * H + 1], nxt, hv;  // planes k-3 .. k+3; the look-ahead
+    SP<R> win[2 * H + 1], hv;  // planes k-3 .. k+3; the halo
+    Raw<R> nxt, hnx;           // the look-ahead
+    if (kFluxDt<R>) sdt[tid] = 0.0;
     uint3 mk;
     unsigned wm;
 #pragma unroll
-    for (int q = 0; q < 2 * H + 1; q++) win[q] = load_sp(plane(min(k0 - H + q, g.nz + H)), nv, soff[0][tid]);
-    hv = load_sp(plane(k0), nv, soff[1][tid]);
+    for (int q = 0; q < 2 * H + 1; q++) win[q] = primitives(K, load(min(k0 - H + q, g.nz + H), soff[0][tid]));
+    hv = primitives(K, load(k0, soff[1][tid]));
     mk = load_masks(k0);
     wm = masks_of(mk);
     fill(0, win[H], hv);
-    nxt = win[2 * H];
     int buf = 0;
     for (int k = k0; k <= k1; k++, buf ^= 1) {
         const SP<R> &o = win[H];
@@ -657,8 +724,8 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
             // (clamped, not skipped, behind the last plane: a load left in
             // flight by one iteration only would make every iteration wait
             // for its stores)
-            nxt = load_sp(plane(min(k + 1 + H, g.nz + H)), nv, soff[0][tid]);
-            hv = load_sp(plane(k + 1), nv, soff[1][tid]);
+            nxt = load(min(k + 1 + H, g.nz + H), soff[0][tid]);
+            hnx = load(k + 1, soff[1][tid]);
             mk = load_masks(min(k + 1, g.nz));
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -726,7 +793,7 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
         f[1] = R(0.25) * (u * A.m + A.mk[0]);
         f[2] = R(0.25) * (v * A.m + A.mk[1]);
         f[3] = R(0.25) * (w * A.m + A.mk[2]);
-        f[4] = R(0.25) * ((R(2) * K.ea + K.eb * t) * A.m + u * A.mk[0] + v * A.mk[1] + w * A.mk[2]) + A.e;
+        f[4] = R(0.25) * ((K.ea2 + K.eb * t) * A.m + u * A.mk[0] + v * A.mk[1] + w * A.mk[2]) + A.e;
         if (edx && !(wm & 1u)) edge_cell<R, 0>(at_x, o, sedge[0][tid], scd, K, ax, f);
         if (edy && !(wm & 2u)) edge_cell<R, 1>(at_y, o, sedge[1][tid], scd, K, ay, f);
         if (SUMS && act) {
@@ -747,14 +814,26 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
             sred[3][tid] += w2;
             sred[4][tid] += w2 * double(t);
         }
+        if constexpr (kFluxDt<R>) {
+            if (F.dtpart && act) {
+                // the spectral radii of compute_dt (kernels_cpu.F90:6814-6880)
+                const int ii = li() - 1, jj = lj() - 1;
+                const R nu = o.a[VM] / o.a[VR], cs = sqrt(K.gamr * t);
+                const R sm = fmax(fmax(F.dxs[ii], F.dys[jj]), F.dzs[k - 1]);
+                R mx = fmax((fabs(u) + cs) * ax, (fabs(v) + cs) * ay);
+                mx = fmax(mx, (fabs(w) + cs) * az);
+                sdt[tid] = fmax(sdt[tid], fmax(mx, fmax(nu, nu * K.prm1) * sm));
+            }
+        }
+        hv = primitives(K, hnx);
         fill(buf ^ 1, win[H + 1], hv);
         wm = masks_of(mk);
 #pragma unroll
         for (int q = 0; q < 2 * H; q++) win[q] = win[q + 1];
-        win[2 * H] = nxt;
+        win[2 * H] = primitives(K, nxt);
         __builtin_amdgcn_sched_barrier(0);
         if (act) {
-            const unsigned oc = soff[0][tid], of = soff[2][tid];
+            const unsigned oc = sizeof(R) == sizeof(double) ? soff[0][tid] : soff[0][tid] >> 1, of = soff[2][tid];
             R *fk = fl + (size_t)(k - 1) * g.nx * g.ny;
 #pragma unroll
             for (int q = 0; q < 5; q++) put_off(fk + q * ni, of, f[q]);
@@ -781,6 +860,13 @@ __device__ __forceinline__ void k_flux_body(const dim3 blockIdx, const dim3 grid
                 F.wallprop[2 * wsz + wp] = double(mu * gty * K.cpr);
             }
         }
+    }
+    if (kFluxDt<R> && F.dtpart) {
+        const double mx = wave_max(sdt[tid]);
+        if ((tid & 63) == 0) lds[tid >> 6][0] = mx;
+        __syncthreads();
+        if (tid == 0) F.dtpart[flat] = fmax(fmax(lds[0][0], lds[1][0]), fmax(lds[2][0], lds[3][0]));
+        __syncthreads();
     }
     if (SUMS) {
         const int jy = min(lj(), g.ny);
@@ -1013,8 +1099,7 @@ struct ItemArgs {
 // side are those it finished with (DevScalars::rhs_sum).
 template <typename R>
 __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
-                                                  const R *__restrict__ wa, const double *__restrict__ w,
-                                                  R *__restrict__ fl, ItemArgs A) {
+                                                  const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
     __shared__ int pre[kItemSeg + 1];
     __shared__ int wsum[4];
     __shared__ double lds[4][6];
@@ -1085,52 +1170,37 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
             const int j = jk % g.ny + 1, k = jk / g.ny + 1;
             const int c = dir == 0 ? i : (dir == 1 ? j : k);
             const int n = dir == 0 ? g.nx : (dir == 1 ? g.ny : g.nz);
-            const int stride = dir == 0 ? 1 : (dir == 1 ? g.sx : g.sxy);
             const int *eoc = dir == 0 ? A.eoc[0] : (dir == 1 ? A.eoc[1] : A.eoc[2]);
             const double *met = dir == 0 ? A.metric[0] : (dir == 1 ? A.metric[1] : A.metric[2]);
             const size_t on = (size_t)(1 + dir) * nv, o1 = (dir == 0 ? 2 : 1) * nv, o2 = (dir == 2 ? 2 : 3) * nv;
-            const int b0 = gidx(g, i, j, k);
+            // every load of the stencil before any arithmetic; periodic
+            // neighbours at their images
             IP q[7];
-            // every load of the stencil before any arithmetic
-            if constexpr (sizeof(R) == sizeof(double)) {
+            double re[7];
 #pragma unroll
-                for (int s = 0; s < 7; s++) {
-                    const int a = b0 + (s - 3) * stride;
-                    q[s].r = wa[a];
-                    q[s].n = wa[on + a];
-                    q[s].a = wa[o1 + a];
-                    q[s].b = wa[o2 + a];
-                    q[s].t = wa[5 * nv + a];
-                }
-            } else {
-                // the mixed form stores w_aux in FP32: the FP64 primitives of
-                // w, periodic neighbours from their images
-                double re[7];
+            for (int s = 0; s < 7; s++) {
+                int pi = i, pj = j, pk = k;
+                if (dir == 0) pi += s - 3;
+                else if (dir == 1) pj += s - 3;
+                else pk += s - 3;
+                if (P.periodic[0]) pi = pi < 1 ? pi + g.nx : (pi > g.nx ? pi - g.nx : pi);
+                if (P.periodic[1]) pj = pj < 1 ? pj + g.ny : (pj > g.ny ? pj - g.ny : pj);
+                if (P.periodic[2]) pk = pk < 1 ? pk + g.nz : (pk > g.nz ? pk - g.nz : pk);
+                const int src = gidx(g, pi, pj, pk);
+                q[s].r = w[src];
+                q[s].n = w[on + src];
+                q[s].a = w[o1 + src];
+                q[s].b = w[o2 + src];
+                re[s] = w[4 * nv + src];
+            }
 #pragma unroll
-                for (int s = 0; s < 7; s++) {
-                    int pi = i, pj = j, pk = k;
-                    if (dir == 0) pi += s - 3;
-                    else if (dir == 1) pj += s - 3;
-                    else pk += s - 3;
-                    if (P.periodic[0]) pi = pi < 1 ? pi + g.nx : (pi > g.nx ? pi - g.nx : pi);
-                    if (P.periodic[1]) pj = pj < 1 ? pj + g.ny : (pj > g.ny ? pj - g.ny : pj);
-                    if (P.periodic[2]) pk = pk < 1 ? pk + g.nz : (pk > g.nz ? pk - g.nz : pk);
-                    const int src = gidx(g, pi, pj, pk);
-                    q[s].r = w[src];
-                    q[s].n = w[on + src];
-                    q[s].a = w[o1 + src];
-                    q[s].b = w[o2 + src];
-                    re[s] = w[4 * nv + src];
-                }
-#pragma unroll
-                for (int s = 0; s < 7; s++) {
-                    const double ri = 1.0 / q[s].r;
-                    q[s].n *= ri;
-                    q[s].a *= ri;
-                    q[s].b *= ri;
-                    const double qq = 0.5 * (q[s].n * q[s].n + q[s].a * q[s].a + q[s].b * q[s].b);
-                    q[s].t = temperature_from_e(P, re[s] / q[s].r - qq, 0.0);
-                }
+            for (int s = 0; s < 7; s++) {
+                const double ri = 1.0 / q[s].r;
+                q[s].n *= ri;
+                q[s].a *= ri;
+                q[s].b *= ri;
+                const double qq = 0.5 * (q[s].n * q[s].n + q[s].a * q[s].a + q[s].b * q[s].b);
+                q[s].t = temperature_from_e(P, re[s] / q[s].r - qq, 0.0);
             }
             const int elo = eoc[c - 1], ehi = eoc[c];
             const double mt = met[c - 1];
@@ -1288,8 +1358,8 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
 // two waves per SIMD: the scattered loads of one batch overlap the other's work
 template <typename R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_weno_items(
-    Geo g, KPar P, const R *__restrict__ wa, const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
-    k_weno_items_body<R>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, wa, w, fl, A);
+    Geo g, KPar P, const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
+    k_weno_items_body<R>(dim3(blockIdx.x, blockIdx.y, blockIdx.z), dim3(gridDim.x, gridDim.y, gridDim.z), g, P, w, fl, A);
 }
 
 // ============================================================ update
@@ -1298,8 +1368,8 @@ struct UpdArgs {
     DevScalars *ds;
     double rkr, rkg;
     int channel;
-    int chunk;
     int keep;          // something reads the finished right-hand side again: store it
+    int mu;            // the next stage reads the viscosity of the new state: store it
     int step_end;      // third stage of st_advance: icyc += 1, time += dt
     double *partials;  // block sums of rho u T dy (FV)
 };
@@ -1311,11 +1381,15 @@ struct UpdArgs {
 // of rho*u*T*dy.  The grad(div/3) terms cost two more reads here (mu, div/3:
 // 16 B a cell) where the pass of their own re-read and re-wrote the
 // right-hand side (152 B).  The velocities of the energy term are formed from
-// w as eval_aux forms them.  A workgroup takes 64 x 4 columns of a few planes
-// with the z stencil of div/3 in registers.  Bound by HBM: 197 B a cell, 1.38
-// ms on 512 x 256 x 256 (4.8 TB/s; the update alone took 0.99 ms, the div/3
-// part of the z march about 0.5).  The right-hand sides are read with
-// the non-temporal hint: neither is read again before a full stage of
+// w as eval_aux forms them.  With U.mu the viscosity of the new state follows:
+// here its power law hides behind the memory, in k_flux, which evaluates every
+// point about twice, it would not.  One cell a lane: with a few planes to a
+// lane the constants of that power law were kept in registers across them, one
+// wave per SIMD less and 4 % slower (and without it no faster, 1379 against
+// 1371 us).  Bound by HBM: 40 + 40 + 40 + 8 + 8 B read and 32 + 40 + 8 B
+// written a cell (the third stage mostly without the 32), 1.33 ms a stage on
+// 512 x 256 x 256 (5.2 TB/s), 34 us on 128 x 96 x 64.  The right-hand sides are
+// read with the non-temporal hint: neither is read again before a full stage of
 // traffic has passed.
 template <typename R, bool FV, bool O2>
 __device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
@@ -1324,7 +1398,7 @@ __device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim
     __shared__ double lds[4][1];
     const int i = blockIdx.x * 64 + threadIdx.x + 1;
     const int j = blockIdx.y * 4 + threadIdx.y + 1;
-    const int k0 = blockIdx.z * U.chunk + 1, k1 = min(k0 + U.chunk - 1, g.nz);
+    const int k = blockIdx.z + 1;
     constexpr int HW = O2 ? 1 : 3;
     double acc[1] = {0.0};
     const double dt = U.ds->dt;
@@ -1342,75 +1416,82 @@ __device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim
             ax = R(U.dx1[i - 1]);
             ay = R(U.dy1[j - 1]);
         }
-        const int col = gidx(g, i, j, 0);
-        R dw[2 * HW + 1];
+        const int c = gidx(g, i, j, k), oi = iidx(g, i, j, k);
+        R fo[5], fp[5];
 #pragma unroll
-        for (int q = 0; q < 2 * HW; q++) dw[q + 1] = D[col + (k0 - HW + q) * g.sxy];
-        for (int k = k0; k <= k1; k++) {
-            const int c = col + k * g.sxy, oi = iidx(g, i, j, k);
+        for (int m = 0; m < 5; m++) fo[m] = __builtin_nontemporal_load(&fl[m * ni + oi]);
+        if (U.rkr != 0.0) {
 #pragma unroll
-            for (int q = 0; q < 2 * HW; q++) dw[q] = dw[q + 1];
-            dw[2 * HW] = D[c + HW * g.sxy];
-            R fo[5], fp[5];
+            for (int m = 0; m < 5; m++) fp[m] = __builtin_nontemporal_load(&flp[m * ni + oi]);
+        }
+        double wo[5];
 #pragma unroll
-            for (int m = 0; m < 5; m++) fo[m] = __builtin_nontemporal_load(&fl[m * ni + oi]);
-            if (U.rkr != 0.0) {
+        for (int m = 0; m < 5; m++) wo[m] = w[m * nv + c];
+        const R mu = wa[6 * nv + c];
+        R gx = R(0), gy = R(0), gz = R(0);
 #pragma unroll
-                for (int m = 0; m < 5; m++) fp[m] = __builtin_nontemporal_load(&flp[m * ni + oi]);
-            }
-            double wo[5];
+        for (int l = 1; l <= HW; l++) {
+            const R cl = O2 ? R(1) : R(P.vd1[l - 1]);
+            gx += cl * (D[c + l] - D[c - l]);
+            gy += cl * (D[c + l * g.sx] - D[c - l * g.sx]);
+            gz += cl * (D[c + l * g.sxy] - D[c - l * g.sxy]);
+        }
+        const R az = O2 ? R(1.0) / R(U.zc[k + ng] - U.zc[k + ng - 2]) : R(U.dz1[k - 1]);
+        const R sx = mu * (gx * ax), sy = mu * (gy * ay), sz = mu * (gz * az);
+        const double ri = 1.0 / wo[0];
+        const double uo = wo[1] * ri, vo = wo[2] * ri, wwo = wo[3] * ri;
+        fo[1] -= sx;
+        fo[2] -= sy;
+        fo[3] -= sz;
+        fo[4] -= sx * R(uo) + sy * R(vo) + sz * R(wwo);
+        if (U.keep) {
 #pragma unroll
-            for (int m = 0; m < 5; m++) wo[m] = w[m * nv + c];
-            const R mu = wa[6 * nv + c];
-            R gx = R(0), gy = R(0), gz = R(0);
+            for (int m = 1; m < 5; m++) fl[m * ni + oi] = fo[m];
+        }
+        double fln[5];
 #pragma unroll
-            for (int l = 1; l <= HW; l++) {
-                const R cl = O2 ? R(1) : R(P.vd1[l - 1]);
-                gx += cl * (D[c + l] - D[c - l]);
-                gy += cl * (D[c + l * g.sx] - D[c - l * g.sx]);
-                gz += cl * (dw[HW + l] - dw[HW - l]);
-            }
-            const R az = O2 ? R(1.0) / R(U.zc[k + ng] - U.zc[k + ng - 2]) : R(U.dz1[k - 1]);
-            const R sx = mu * (gx * ax), sy = mu * (gy * ay), sz = mu * (gz * az);
-            const double ri = 1.0 / wo[0];
-            const double uo = wo[1] * ri, vo = wo[2] * ri, wwo = wo[3] * ri;
-            fo[1] -= sx;
-            fo[2] -= sy;
-            fo[3] -= sz;
-            fo[4] -= sx * R(uo) + sy * R(vo) + sz * R(wwo);
-            if (U.keep) {
+        for (int m = 0; m < 5; m++) {
+            fln[m] = -gamdt * double(fo[m]);
+            if (U.rkr != 0.0) fln[m] = -rhodt * double(fp[m]) + fln[m];
+        }
+        if (U.channel) {
+            fln[0] = fln[0] - b1;
+            fln[1] = fln[1] - b2;
+            fln[4] = fln[4] - uo * b2;
+        }
+        double wn[5];
 #pragma unroll
-                for (int m = 1; m < 5; m++) fl[m * ni + oi] = fo[m];
-            }
-            double fln[5];
+        for (int m = 0; m < 5; m++) {
+            wn[m] = wo[m] + fln[m];
+            w[m * nv + c] = wn[m];
+        }
+        if (FV) {
+            const double dy = U.yn[j] - U.yn[j - 1];
+            const double rn = 1.0 / wn[0];
+            const double uu = wn[1] * rn, vv = wn[2] * rn, ww = wn[3] * rn;
+            const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+            const double ee = wn[4] / wn[0] - qq;
+            const double tt = temperature_from_e(P, ee, 0.0);
+            wa[5 * nv + c] = R(tt);
+            acc[0] += wn[1] * tt * dy;
+        } else {
+            // the cell's viscosity, and bcwall_staggered (kernels_cpu.F90:
+            // 6612-6678) with the ghosts' at either wall
+#pragma unroll 1
+            for (int o = U.mu ? 0 : 1; o < 3; o++) {
+                double x[5];
+                int d = c;
+                if (o == 0) {
 #pragma unroll
-            for (int m = 0; m < 5; m++) {
-                fln[m] = -gamdt * double(fo[m]);
-                if (U.rkr != 0.0) fln[m] = -rhodt * double(fp[m]) + fln[m];
-            }
-            if (U.channel) {
-                fln[0] = fln[0] - b1;
-                fln[1] = fln[1] - b2;
-                fln[4] = fln[4] - uo * b2;
-            }
-            double wn[5];
+                    for (int m = 0; m < 5; m++) x[m] = wn[m];
+                } else {
+                    if (!P.wall_stag[o - 1] || (o == 1 ? j > g.ng : j <= g.ny - g.ng)) continue;
+                    wall_ghost_of(P, wn, 0.0, x);
+                    d = gidx(g, i, o == 1 ? 1 - j : 2 * g.ny + 1 - j, k);
 #pragma unroll
-            for (int m = 0; m < 5; m++) {
-                wn[m] = wo[m] + fln[m];
-                w[m * nv + c] = wn[m];
-            }
-            if (FV) {
-                const double dy = U.yn[j] - U.yn[j - 1];
-                const double rn = 1.0 / wn[0];
-                const double uu = wn[1] * rn, vv = wn[2] * rn, ww = wn[3] * rn;
-                const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
-                const double ee = wn[4] / wn[0] - qq;
-                const double tt = temperature_from_e(P, ee, 0.0);
-                wa[5 * nv + c] = R(tt);
-                acc[0] += wn[1] * tt * dy;
-            } else {
-                if (P.wall_stag[0] && j <= g.ng) wall_ghost(g, P, w, wa, i, j, 1 - j, k);
-                if (P.wall_stag[1] && j > g.ny - g.ng) wall_ghost(g, P, w, wa, i, j, 2 * g.ny + 1 - j, k);
+                    for (int m = 0; m < 5; m++) w[m * nv + d] = x[m];
+                }
+                if (U.mu) wa[6 * nv + d] = R(mu_of(P, x));
             }
         }
     }
@@ -1483,24 +1564,18 @@ static int flux_chunk(const Geo &g, bool mixed) {
 static dim3 flux_grid(const Geo &g, int chunk) {
     return dim3((g.nx + kFluxTX - 1) / kFluxTX, (g.ny + kFluxTY - 1) / kFluxTY, (g.nz + chunk - 1) / chunk);
 }
-// Planes per workgroup of k_update_div: each reads 6 planes of div/3 beyond its
-// own, and its planes' loads wait for one another's stores; on 512 x 256 x 256
-// chunks 1, 2, 4, 16 took 1371, 1379, 1402, 1438 us, on 256 x 128 x 128 165,
-// 161, 160, 173, on 48 x 40 x 36 chunks 1, 2 took 9.1, 10.0.
-static int update_chunk(const Geo &g) {
-    const long cols = (long)((g.nx + 63) / 64) * ((g.ny + 3) / 4);
-    return cols * ((g.nz + 1) / 2) >= 2048 ? 2 : 1;
-}
-static dim3 update_grid(const Geo &g, int chunk) {
-    return dim3((g.nx + 63) / 64, (g.ny + 3) / 4, (g.nz + chunk - 1) / chunk);
-}
+static dim3 update_grid(const Geo &g) { return dim3((g.nx + 63) / 64, (g.ny + 3) / 4, g.nz); }
 static int nblocks(const dim3 &d) { return (int)(d.x * d.y * d.z); }
 
 // Doubles of the reduction scratch: [0, flux) the block sums of k_flux (or of
-// k_update_div), [dt, dt + blocks) the CFL maxima of the aux pass, then the
-// second-level values of k_weno_items.
+// k_update_div), [dt, dt + blocks) the CFL maxima of k_flux (of the aux pass
+// elsewhere), then the second-level values of k_weno_items.
 int one_pass_flux_slots(const Geo &g, bool mixed) { return 5 * nblocks(flux_grid(g, flux_chunk(g, mixed))); }
-int one_pass_update_blocks(const Geo &g) { return nblocks(update_grid(g, update_chunk(g))); }
+int one_pass_dt_slots(const Geo &g) {
+    const int f = nblocks(flux_grid(g, 1)), a = aux_dt_blocks(g);
+    return f > a ? f : a;
+}
+int one_pass_update_blocks(const Geo &g) { return nblocks(update_grid(g)); }
 
 static int item_segments(const Geo &g, int *wpt) {
     const long nwords = (long)rec_per_row(g) * g.ny * g.nz;
@@ -1522,7 +1597,7 @@ hipError_t launch_hot_items(st_solver *s) {
     return hipGetLastError();
 }
 
-hipError_t launch_flux(st_solver *s, void *fl, int stage) {
+hipError_t launch_flux(st_solver *s, void *fl, int stage, bool dt) {
     const Geo &g = s->g;
     const bool sums = s->p.channel_case != 0, cons = s->p.conservative_viscous == 1;
     // with the bulk sums the chunk is a function of the grid alone: they are
@@ -1543,6 +1618,8 @@ hipError_t launch_flux(st_solver *s, void *fl, int stage) {
     F.chunk = chunk;
     F.last = stage == 2;
     if (sums) s->force_nblk = nblocks(grid);
+    F.dtpart = dt && !s->mixed ? s->dtpart : nullptr;
+    if (dt) s->dt_nblk = s->mixed ? aux_dt_blocks(g) : nblocks(grid);
 #define ST_LAUNCH_FX(C_, S_) \
     ST_DISPATCH(ST_GO(k_flux, ST_T(R, C_, S_), 256, kFluxWaves<R>, grid, dim3(kFluxTX, kFluxTY), g, s->kp, (R *)s->w_aux, (R *)fl, F))
     if (cons && sums) ST_LAUNCH_FX(true, true);
@@ -1567,7 +1644,7 @@ hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt) {
     A.partials = s->partials;
     A.nblk = s->force_nblk;
     A.dtpart = s->dtpart;
-    A.ndt = dt ? aux_dt_blocks(g) : 0;
+    A.ndt = dt ? s->dt_nblk : 0;
     A.stage2 = s->stage2;
     A.ticket = s->counters + 1;
     A.ds = s->ds;
@@ -1579,12 +1656,11 @@ hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt) {
     // one workgroup per 8192 cells, at most what the chip holds at once
     long nb = (long)((g.nint + 8191) / 8192);
     nb = nb < 1 ? 1 : (nb > kItemBlocks ? kItemBlocks : nb);
-    ST_DISPATCH(ST_GO(k_weno_items, ST_T(R), 256, 2, dim3((unsigned)nb), dim3(256), g, s->kp, (const R *)s->w_aux, s->w,
-                      (R *)fl, A));
+    ST_DISPATCH(ST_GO(k_weno_items, ST_T(R), 256, 2, dim3((unsigned)nb), dim3(256), g, s->kp, s->w, (R *)fl, A));
     return hipGetLastError();
 }
 
-hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last) {
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last, bool mu) {
     const Geo &g = s->g;
     const bool fv = s->p.channel_case && s->p.theta_wall >= -1.0, o2 = s->p.conservative_viscous == 1;
     UpdArgs U{};
@@ -1594,14 +1670,14 @@ hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int st
     U.rkr = s->rhork[stage];
     U.rkg = s->gamrk[stage];
     U.channel = s->p.channel_case;
-    U.chunk = update_chunk(g);
     // the first two stages' are F[prev] of the next; the third's has no reader
     // but the caller, and is left out (32 of 184 B a cell) while further steps
     // of the call follow: 512x256x256 1380 -> 1307 us a stage over three stages
     U.keep = stage < 2 || last;
+    U.mu = mu && !fv;
     U.step_end = step_end ? 1 : 0;
     U.partials = s->partials;
-    const dim3 grid = update_grid(g, U.chunk);
+    const dim3 grid = update_grid(g);
 #define ST_LAUNCH_UD(F_, O_)                                                                                  \
     ST_DISPATCH(ST_GO(k_update_div, ST_T(R, F_, O_), 256, 0, grid, dim3(64, 4), g, s->kp, s->w, (R *)s->w_aux, \
                       (const R *)fl_prev, (R *)fl, U))
