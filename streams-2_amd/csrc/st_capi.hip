@@ -294,14 +294,21 @@ bool fp64_sensor(const st_solver *s) { return s->mixed && s->p.conservative_visc
 // one RK stage of rk_sync in three launches (st_stage.hip), plus the step's
 // WENO masks at its first stage; first, last: the first and last stage of a
 // call, where w_aux comes from and goes to the caller; end: the last stage of
-// a st_advance step; stay: no step of the call follows
-int stage_one_pass(st_solver *s, int istep, bool end, bool first, bool stay) {
+// a st_advance step; stay: no step of the call follows; next_dt: one follows
+// that recomputes dt
+int stage_one_pass(st_solver *s, int istep, bool end, bool first, bool stay, bool next_dt) {
     using namespace st;
     void *fprev = s->F[s->cur], *fcur = s->F[s->cur ^ 1];
     const Geo &g = s->g;
     const bool dt = istep == 0 && s->dt_in_stage && s->p.cfl > 0, last = stay && istep == 2;
     if (istep == 0) TIMED(ST_K_WENO_FIX, launch_hot_items(s));
-    const bool aux_dt = dt && s->mixed;  // (k_flux takes the radii in FP64)
+    // the CFL radii: in FP64 k_flux takes them; in the mixed form the last step's
+    // update, where nothing changes its state any more, or the aux pass
+    if (first && istep == 0) s->dt_waits = false;
+    const bool aux_dt = dt && s->mixed && !s->dt_waits;
+    const bool fv = s->p.channel_case && s->p.theta_wall >= -1.0;
+    const bool feeds = next_dt && istep == 2 && s->mixed && !fv && !s->general_bc;
+    if (aux_dt) s->dt_nblk = aux_dt_blocks(g);
     if ((first && istep == 0) || last || aux_dt)
         TIMED(ST_K_AUX, launch_aux(s, 1 - g.ng, g.nx + g.ng, 1 - g.ng, g.ny + g.ng, 1 - g.ng, g.nz + g.ng, true, aux_dt,
                                    true, last));
@@ -310,8 +317,9 @@ int stage_one_pass(st_solver *s, int istep, bool end, bool first, bool stay) {
     if (istep == 2 && fp64_sensor(s)) TIMED(ST_K_SENSOR, launch_sensor_refine(s, false, true));
     TIMED(ST_K_WENO_FIX, launch_weno_items(s, fcur, istep, dt));
     if (s->has_nr) TIMED(ST_K_BC, launch_bc_nr(s, fcur, true));
-    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end, stay, !last));
-    if (s->p.channel_case && s->p.theta_wall >= -1.0)
+    TIMED(ST_K_UPDATE, launch_update_div(s, fprev, fcur, istep, end, stay, !last, feeds));
+    s->dt_waits = feeds;
+    if (fv)
         TIMED(ST_K_FORCE_VAR, launch_force_var(s, one_pass_update_blocks(g), !last));
     if (s->general_bc) TIMED(ST_K_BC, launch_physical_ghosts(s, true, !last));
     s->cur ^= 1;
@@ -384,11 +392,12 @@ int stage(st_solver *s, int istep) {
 }
 
 // end: the step of st_advance, which also moves time and the step counter;
-// first, last: no step of the same call before it, after it
-int do_rk_sync(st_solver *s, bool end, bool first, bool last) {
+// first, last: no step of the same call before it, after it; next_dt as in
+// stage_one_pass
+int do_rk_sync(st_solver *s, bool end, bool first, bool last, bool next_dt) {
     const bool one = st::one_pass_stage(s);
     for (int istep = 0; istep < 3; istep++) {
-        int rc = one ? stage_one_pass(s, istep, end && istep == 2, first, last) : stage(s, istep);
+        int rc = one ? stage_one_pass(s, istep, end && istep == 2, first, last, next_dt) : stage(s, istep);
         if (rc) return rc;
     }
     if (end && !one) TIMED(ST_K_STEP_END, st::launch_step_end(s));
@@ -1163,7 +1172,7 @@ int st_rk_sync(st_solver *s) {
         if (rc) return rc;
         return rk_sync_pieces(s, s->hs->dt);
     }
-    return do_rk_sync(s, false, true, true);
+    return do_rk_sync(s, false, true, true, false);
 }
 
 int st_advance(st_solver *s, int32_t nsteps) {
@@ -1185,13 +1194,14 @@ int st_advance(st_solver *s, int32_t nsteps) {
             HIPCHK(st::launch_step_end(s));
             continue;
         }
-        if (s->p.cfl > 0 && ((s->icyc - s->icyc0) % iter_dt) == 0) {
+        auto takes_dt = [&](int64_t icyc) { return s->p.cfl > 0 && ((icyc - s->icyc0) % iter_dt) == 0; };
+        if (takes_dt(s->icyc)) {
             // compute_aux(central) + compute_dt of the step start form the
             // same primitives of the same w as the first stage's aux, which
             // therefore takes the reduction
             s->dt_in_stage = true;
         }
-        int rc = do_rk_sync(s, true, n == 0, n + 1 == nsteps);
+        int rc = do_rk_sync(s, true, n == 0, n + 1 == nsteps, n + 1 < nsteps && takes_dt(s->icyc + 1));
         if (rc) return rc;
     }
     return ST_OK;

@@ -81,6 +81,23 @@ __device__ __forceinline__ double mu_of(const KPar &P, const double (&c)[5]) {
     return viscosity_of(P, temperature_from_e(P, ee, P.t0));
 }
 
+// The largest spectral radius of compute_dt_subroutine (kernels_cpu.F90:
+// 6814-6880) at a point with the Euler metrics a and the viscous ones s, by
+// the operations of k_aux as mu_of.
+__device__ __forceinline__ double cfl_radius(const KPar &P, const double (&c)[5], const double (&a)[3],
+                                             const double (&s)[3]) {
+    const double ri = 1.0 / c[0];
+    const double uu = c[1] * ri, vv = c[2] * ri, ww = c[3] * ri;
+    const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
+    const double ee = c[4] / c[0] - qq;
+    const double tt = temperature_from_e(P, ee, P.t0);
+    const double nu = ri * viscosity_of(P, tt), kor = nu / P.prandtl;
+    const double cs = sqrt(gamloc_of(P, tt) * P.rgas0 * tt);
+    double mx = fmax(fmax((fabs(uu) + cs) * a[0], (fabs(vv) + cs) * a[1]), (fabs(ww) + cs) * a[2]);
+    mx = fmax(mx, fmax(nu * s[0], fmax(nu * s[1], nu * s[2])));
+    return fmax(mx, fmax(kor * s[0], fmax(kor * s[1], kor * s[2])));
+}
+
 // bcwall_staggered_subroutine (kernels_cpu.F90:6612-6678): the ghost state d
 // that mirrors the state c about an isothermal wall (t_start as in
 // temperature_from_e).

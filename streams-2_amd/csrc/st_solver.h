@@ -68,7 +68,8 @@ struct st_solver {
     bool dt_in_stage;   // the CFL reduction of this step rides on the first stage's aux
     int visc_chunk;     // planes per tile of the z-marching viscous kernel (0: automatic)
     int march_chunk;    // points per thread of the y/z flux marches (0: automatic)
-    int dt_nblk;        // CFL block maxima of the last launch_flux that took them
+    int dt_nblk;        // CFL block maxima that wait in dtpart
+    bool dt_waits;      // the last update left those of its new state
     bool x_uniform;     // dcsidx is one value (set by st_set_grid)
     bool fuse_xy;       // x and y Euler fluxes in one pass
     bool fuse_zv;       // viscous divergence terms folded into the z march (Laplacian form)
@@ -256,7 +257,7 @@ hipError_t launch_flux(st_solver *s, void *fl, int stage, bool dt);
 // WENO faces; bulk sums of force_rhs and, with dt, the CFL step finished
 hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt);
 // grad(div/3), update_flux, update_field, wall ghosts; the end of the step
-hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last, bool mu);
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last, bool mu, bool dt);
 hipError_t launch_dt(st_solver *s);
 hipError_t launch_step_end(st_solver *s);
 hipError_t launch_residual(st_solver *s);

@@ -424,7 +424,8 @@ constexpr int kFluxWaves = sizeof(R) == sizeof(double) ? 2 : 3;
 
 constexpr int kFluxMaxChunk = 32;
 // FP64 also takes the CFL radii, from the point it holds; the mixed form's
-// points are rounded, and its radii are those of an aux pass in FP64
+// points are rounded, and it takes them from w in FP64, where w was last written
+// or in the aux pass
 template <typename R>
 constexpr bool kFluxDt = sizeof(R) == sizeof(double);
 
@@ -1365,6 +1366,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // ============================================================ update
 struct UpdArgs {
     const double *dx1, *dy1, *dz1, *xc, *yc, *zc, *yn;
+    const double *dxs, *dys, *dzs;  // viscous metrics of the CFL radii
     DevScalars *ds;
     double rkr, rkg;
     int channel;
@@ -1372,6 +1374,7 @@ struct UpdArgs {
     int mu;            // the next stage reads the viscosity of the new state: store it
     int step_end;      // third stage of st_advance: icyc += 1, time += dt
     double *partials;  // block sums of rho u T dy (FV)
+    double *dtpart;    // block maxima of the CFL radii of the new state (null: not wanted)
 };
 
 // visflx_div (kernels_cpu.F90:3484-3532, or its second-order form with O2,
@@ -1493,12 +1496,26 @@ __device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim
                 }
                 if (U.mu) wa[6 * nv + d] = R(mu_of(P, x));
             }
+            if (!kFluxDt<R> && U.dtpart) {
+                const double a[3] = {U.dx1[i - 1], U.dy1[j - 1], U.dz1[k - 1]};
+                const double s[3] = {U.dxs[i - 1], U.dys[j - 1], U.dzs[k - 1]};
+                acc[0] = cfl_radius(P, wn, a, s);
+            }
         }
     }
     if (FV) {
         block_sum<1>(acc, lds);
         if (flat_thread() == 0)
             U.partials[(int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z))] = acc[0];
+    }
+    if (!FV && !kFluxDt<R> && U.dtpart) {
+        const int ft = flat_thread();
+        const double mx = wave_max(acc[0]);
+        if ((ft & 63) == 0) lds[ft >> 6][0] = mx;
+        __syncthreads();
+        if (ft == 0)
+            U.dtpart[(int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z))] =
+                fmax(fmax(lds[0][0], lds[1][0]), fmax(lds[2][0], lds[3][0]));
     }
     // run()'s loop end (singleideal_cpu.F90:1604,1642); nothing else of this
     // launch reads time or icyc
@@ -1571,11 +1588,11 @@ static int nblocks(const dim3 &d) { return (int)(d.x * d.y * d.z); }
 // k_update_div), [dt, dt + blocks) the CFL maxima of k_flux (of the aux pass
 // elsewhere), then the second-level values of k_weno_items.
 int one_pass_flux_slots(const Geo &g, bool mixed) { return 5 * nblocks(flux_grid(g, flux_chunk(g, mixed))); }
-int one_pass_dt_slots(const Geo &g) {
-    const int f = nblocks(flux_grid(g, 1)), a = aux_dt_blocks(g);
-    return f > a ? f : a;
-}
 int one_pass_update_blocks(const Geo &g) { return nblocks(update_grid(g)); }
+int one_pass_dt_slots(const Geo &g) {
+    const int f = nblocks(flux_grid(g, 1)), a = aux_dt_blocks(g), u = one_pass_update_blocks(g);
+    return f > a ? (f > u ? f : u) : (a > u ? a : u);
+}
 
 static int item_segments(const Geo &g, int *wpt) {
     const long nwords = (long)rec_per_row(g) * g.ny * g.nz;
@@ -1619,7 +1636,7 @@ hipError_t launch_flux(st_solver *s, void *fl, int stage, bool dt) {
     F.last = stage == 2;
     if (sums) s->force_nblk = nblocks(grid);
     F.dtpart = dt && !s->mixed ? s->dtpart : nullptr;
-    if (dt) s->dt_nblk = s->mixed ? aux_dt_blocks(g) : nblocks(grid);
+    if (F.dtpart) s->dt_nblk = nblocks(grid);
 #define ST_LAUNCH_FX(C_, S_) \
     ST_DISPATCH(ST_GO(k_flux, ST_T(R, C_, S_), 256, kFluxWaves<R>, grid, dim3(kFluxTX, kFluxTY), g, s->kp, (R *)s->w_aux, (R *)fl, F))
     if (cons && sums) ST_LAUNCH_FX(true, true);
@@ -1660,7 +1677,7 @@ hipError_t launch_weno_items(st_solver *s, void *fl, int stage, bool dt) {
     return hipGetLastError();
 }
 
-hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last, bool mu) {
+hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int stage, bool step_end, bool last, bool mu, bool dt) {
     const Geo &g = s->g;
     const bool fv = s->p.channel_case && s->p.theta_wall >= -1.0, o2 = s->p.conservative_viscous == 1;
     UpdArgs U{};
@@ -1675,6 +1692,9 @@ hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int st
     // of the call follow: 512x256x256 1380 -> 1307 us a stage over three stages
     U.keep = stage < 2 || last;
     U.mu = mu && !fv;
+    U.dxs = s->dcsidxs; U.dys = s->detadys; U.dzs = s->dzitdzs;
+    U.dtpart = dt ? s->dtpart : nullptr;
+    if (dt) s->dt_nblk = one_pass_update_blocks(g);
     U.step_end = step_end ? 1 : 0;
     U.partials = s->partials;
     const dim3 grid = update_grid(g);
