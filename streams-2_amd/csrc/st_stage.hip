@@ -1151,11 +1151,12 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
     };
     ItemConst C;
     C.eb = cvc(P, 0);
-    C.ea = P.t0 * (cvc(P, P.indx_cp_r + 1) - C.eb);
+    C.ea = uniform(P.t0 * (cvc(P, P.indx_cp_r + 1) - C.eb));
     C.rg = P.rgas0;
-    C.gam = cpc(P, 0) / (cpc(P, 0) - P.rgas0);
-    C.tb = 1.0 / cpc(P, 0);
-    C.ta = P.t0 - cpc(P, P.indx_cp_r + 1) * P.t0 * C.tb;
+    C.gam = uniform(cpc(P, 0) / (cpc(P, 0) - P.rgas0));
+    C.tb = uniform(1.0 / cpc(P, 0));
+    C.ta = uniform(P.t0 - cpc(P, P.indx_cp_r + 1) * P.t0 * C.tb);
+    const double te = uniform(1.0 / C.eb), t0e = uniform(P.t0 - cvc(P, P.indx_cp_r + 1) * P.t0 * te);  // T = t0e + te e
     const int wave = (blockIdx.x * blockDim.x + t) >> 6;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
     for (int base = wave * 62; base < total; base += nwaves * 62) {
@@ -1201,7 +1202,7 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
                 q[s].a *= ri;
                 q[s].b *= ri;
                 const double qq = 0.5 * (q[s].n * q[s].n + q[s].a * q[s].a + q[s].b * q[s].b);
-                q[s].t = temperature_from_e(P, re[s] / q[s].r - qq, 0.0);
+                q[s].t = t0e + te * (re[s] * ri - qq);
             }
             const int elo = eoc[c - 1], ehi = eoc[c];
             const double mt = met[c - 1];
