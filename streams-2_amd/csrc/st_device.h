@@ -117,11 +117,10 @@ __device__ __forceinline__ void wall_ghost_of(const KPar &P, const double (&c)[5
     d[3] = -rho * ww;
     d[4] = rho * (ee + qq);
 }
-// for one ghost point: the mirror of interior point js, written at jg; with mu
-// its viscosity too
+// for one ghost point: the mirror of interior point js, written at jg
 template <typename R>
-__device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *__restrict__ w, R *__restrict__ wa, int i,
-                                           int js, int jg, int k, bool mu) {
+__device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *__restrict__ w, const R *__restrict__ wa,
+                                           int i, int js, int jg, int k) {
     const int s = gidx(g, i, js, k), d = gidx(g, i, jg, k);
     const size_t nv = g.nvol;
     double c[5], x[5];
@@ -130,7 +129,6 @@ __device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *
     wall_ghost_of(P, c, double(wa[5 * nv + s]), x);
 #pragma unroll
     for (int m = 0; m < 5; m++) w[m * nv + d] = x[m];
-    if (mu) wa[6 * nv + d] = R(mu_of(P, x));
 }
 
 // exclusive prefix over the block's 256 threads of v; *total receives the sum

@@ -95,7 +95,7 @@ __global__ void k_extrapolate_var(Geo g, T *__restrict__ a) {
 }
 
 template <typename R>
-__global__ void k_wall_ghosts(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa, int mu) {
+__global__ void k_wall_ghosts(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa) {
     const int tot = 2 * g.ng * g.nx * g.nz;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
         const int i = t % g.nx + 1;
@@ -103,10 +103,10 @@ __global__ void k_wall_ghosts(Geo g, KPar P, double *__restrict__ w, R *__restri
         const int l = r % (2 * g.ng);
         const int k = r / (2 * g.ng) + 1;
         if (l < g.ng) {
-            if (P.wall_stag[0]) wall_ghost(g, P, w, wa, i, l + 1, -l, k, mu != 0);
+            if (P.wall_stag[0]) wall_ghost(g, P, w, wa, i, l + 1, -l, k);
         } else {
             const int ll = l - g.ng + 1;
-            if (P.wall_stag[1]) wall_ghost(g, P, w, wa, i, g.ny + 1 - ll, g.ny + ll, k, mu != 0);
+            if (P.wall_stag[1]) wall_ghost(g, P, w, wa, i, g.ny + 1 - ll, g.ny + ll, k);
         }
     }
 }
@@ -234,8 +234,8 @@ __device__ __forceinline__ void bc_point(const Geo &g, const KPar &P, double *__
         }
     } else if (tag == 6 && staggered) {
         for (int l = 1; l <= ng; l++) {
-            if (ilat == 3) wall_ghost(g, P, w, wa, a, l, 1 - l, b, false);
-            else if (ilat == 4) wall_ghost(g, P, w, wa, a, g.ny + 1 - l, g.ny + l, b, false);
+            if (ilat == 3) wall_ghost(g, P, w, wa, a, l, 1 - l, b);
+            else if (ilat == 4) wall_ghost(g, P, w, wa, a, g.ny + 1 - l, g.ny + l, b);
         }
     } else if (tag == 6 && ilat == 3) {
         const int c1 = gidx(g, a, 1, b);
@@ -260,7 +260,7 @@ __device__ __forceinline__ void bc_point(const Geo &g, const KPar &P, double *__
 #pragma unroll
             for (int m = 0; m < 5; m++) w[m * nv + gidx(g, a, -l, b)] = x[m];
         }
-        for (int l = 4; l <= ng; l++) wall_ghost(g, P, w, wa, a, 1 + l, 1 - l, b, false);
+        for (int l = 4; l <= ng; l++) wall_ghost(g, P, w, wa, a, 1 + l, 1 - l, b);
     } else if (tag == 7 && ilat == 4) {
         const double tanhlen = 8.0 * P.tanhfacs;
         const int i = a, k = b;
@@ -2821,8 +2821,8 @@ __device__ __forceinline__ void k_update_body(const dim3 blockIdx, const dim3 gr
             wa[5 * nv + c] = R(tt);
             acc[0] = wn[1] * tt * dy;
         } else {
-            if (P.wall_stag[0] && j <= g.ng) wall_ghost(g, P, w, wa, i, j, 1 - j, k, false);
-            if (P.wall_stag[1] && j > g.ny - g.ng) wall_ghost(g, P, w, wa, i, j, 2 * g.ny + 1 - j, k, false);
+            if (P.wall_stag[0] && j <= g.ng) wall_ghost(g, P, w, wa, i, j, 1 - j, k);
+            if (P.wall_stag[1] && j > g.ny - g.ng) wall_ghost(g, P, w, wa, i, j, 2 * g.ny + 1 - j, k);
         }
     }
     if (FORCE_VAR) {
@@ -2852,10 +2852,12 @@ __global__ __launch_bounds__(RED_THREADS) void k_force_var_finish(KPar P, const 
     }
 }
 
-// force_var_2_subroutine (kernels_cpu.F90:3282-3314) + wall ghosts
+// force_var_2_subroutine (kernels_cpu.F90:3282-3314), and with walls the
+// staggered wall ghosts of the new state (a launch of their own cost 4.3 us a
+// stage on 45 x 33 x 21); mu as in k_bc_faces
 template <typename R>
 __global__ __launch_bounds__(256) void k_force_var2(Geo g, KPar P, double *__restrict__ w, R *__restrict__ wa,
-                                                    const DevScalars *__restrict__ ds, int mu) {
+                                                    const DevScalars *__restrict__ ds, int walls, int mu) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
@@ -2863,11 +2865,22 @@ __global__ __launch_bounds__(256) void k_force_var2(Geo g, KPar P, double *__res
     const size_t nv = g.nvol;
     const int c = gidx(g, i, j, k);
     const double rho = w[c], rhou = w[nv + c], rhov = w[2 * nv + c], rhow = w[3 * nv + c];
-    const double ttnew = double(wa[5 * nv + c]) + ds->bulkt;
+    const double tt = double(wa[5 * nv + c]), ttnew = tt + ds->bulkt;
     const double ee = e_from_temperature(P, ttnew);
     const double x[5] = {rho, rhou, rhov, rhow, rho * ee + 0.5 * (rhou * rhou + rhov * rhov + rhow * rhow) / rho};
     w[4 * nv + c] = x[4];
     if (mu) wa[6 * nv + c] = R(mu_of(P, x));
+    if (!walls) return;
+#pragma unroll 1
+    for (int side = 0; side < 2; side++) {
+        if (!P.wall_stag[side] || (side ? j <= g.ny - g.ng : j > g.ng)) continue;
+        double y[5];
+        wall_ghost_of(P, x, tt, y);
+        const int d = gidx(g, i, side ? 2 * g.ny + 1 - j : 1 - j, k);
+#pragma unroll
+        for (int m = 0; m < 5; m++) w[m * nv + d] = y[m];
+        if (mu) wa[6 * nv + d] = R(mu_of(P, y));
+    }
 }
 
 // ------------------------------------------------------------ statistics
@@ -3464,13 +3477,13 @@ hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int 
     return hipGetLastError();
 }
 
-hipError_t launch_wall_ghosts(st_solver *s, bool mu) {
+hipError_t launch_wall_ghosts(st_solver *s) {
     ST_NOREC();
     const Geo &g = s->g;
     if (!s->kp.wall_stag[0] && !s->kp.wall_stag[1]) return hipSuccess;
     size_t tot = (size_t)2 * g.ng * g.nx * g.nz;
     ST_DISPATCH(hipLaunchKernelGGL(k_wall_ghosts<R>, dim3(grid1d(tot, 256)), dim3(256), 0, s->stream, g, s->kp, s->w,
-                                   (R *)s->w_aux, mu ? 1 : 0));
+                                   (R *)s->w_aux));
     return hipGetLastError();
 }
 
@@ -3871,8 +3884,8 @@ hipError_t launch_force_var(st_solver *s, int nblk, bool mu) {
     hipLaunchKernelGGL(k_force_var_finish, dim3(red_blocks(nblk)), dim3(RED_THREADS), 0, s->stream, s->kp,
                        s->partials, nblk, s->partials + s->npart - RB * 8, s->counters + 1, s->ds);
     ST_DISPATCH(hipLaunchKernelGGL(k_force_var2<R>, cell_grid(g), kCellBlock, 0, s->stream, g, s->kp, s->w,
-                                   (R *)s->w_aux, s->ds, mu ? 1 : 0));
-    return launch_wall_ghosts(s, mu);
+                                   (R *)s->w_aux, s->ds, 1, mu ? 1 : 0));
+    return hipGetLastError();
 }
 
 int dt_blocks_per_plane(const Geo &g) { return ((g.nx + 63) / 64) * ((g.ny + 3) / 4); }
@@ -4040,7 +4053,7 @@ hipError_t launch_force_var_piece(st_solver *s) {
     hipLaunchKernelGGL(k_force_var_finish, dim3(red_blocks(cell_blocks(g))), dim3(RED_THREADS), 0, s->stream, s->kp,
                        s->partials, cell_blocks(g), s->partials + s->npart - RB * 8, s->counters + 1, s->ds);
     ST_DISPATCH(hipLaunchKernelGGL(k_force_var2<R>, cell_grid(g), kCellBlock, 0, s->stream, g, s->kp, s->w,
-                                   (R *)s->w_aux, s->ds, 0));
+                                   (R *)s->w_aux, s->ds, 0, 0));
     return hipGetLastError();
 }
 

@@ -197,11 +197,11 @@ hipError_t launch_extrapolate_aux(st_solver *s, int var);
 hipError_t launch_aux(st_solver *s, int i0, int i1, int j0, int j1, int k0, int k1, bool image,
                       bool dt = false, bool defer_dt = false, bool enthalpy = true);
 int aux_dt_blocks(const Geo &g);  // block maxima of an aux pass over the ghosted box
-hipError_t launch_wall_ghosts(st_solver *s, bool mu = false);
+hipError_t launch_wall_ghosts(st_solver *s);
 // physical ghosts of every non-periodic face in the order xmin..zmax
 // (update_ghost without the periodic swap), recyc_exchange and the recycled
 // inflow included; draws: first redraw the random inflow plane; mu: also
-// w_aux(7) of the points written (as in the wall ghosts and force_var)
+// w_aux(7) of the points written (as in force_var)
 hipError_t launch_physical_ghosts(st_solver *s, bool draws, bool mu = false);
 // characteristic boundary treatment added to fl (bc_nr)
 hipError_t launch_bc_nr(st_solver *s, void *fl, bool from_w = false);
@@ -238,7 +238,8 @@ hipError_t launch_sensor(st_solver *s, bool ghost_images);
 hipError_t launch_visc_div(st_solver *s, void *fl, const void *fl_prev, int stage, bool reduce, bool ord2);
 hipError_t launch_force_finish(st_solver *s, int stage);
 hipError_t launch_update(st_solver *s, const void *fl_prev, const void *fl, int stage);
-// nblk block sums of rho*u*T*dy from the update
+// nblk block sums of rho*u*T*dy from the update, then force_var_2 and the wall
+// ghosts
 hipError_t launch_force_var(st_solver *s, int nblk, bool mu = false);
 int update_blocks(const Geo &g);
 // ---- one-pass stage (st_stage.hip)
