@@ -12,11 +12,11 @@ metric: Gcell-updates/s per RK stage = nx*ny*nz * 3 * steps / seconds / 1e9.
 
 Prints one JSON line.  The roofline object covers the kernel with the
 largest total time among those with a byte count (one launch per stage: the
-z flux march, its WENO fix-up timed apart as "weno_fix"), from HIP events
-recorded on the solver's own stream around every launch (the CFL reduction
-of each step rides on the first stage's aux pass, so it is timed within
-"aux"); its traffic comes from the committed rocprofv3 FETCH_SIZE/WRITE_SIZE
-summary of the same workload.  The CPU baseline times the oracle (a
+one-pass flux, "euler_xy", or the update; the WENO items and the step's masks
+are timed apart as "weno_fix"), from HIP events recorded on the solver's own
+stream around every launch (the CFL reduction of each step rides on the first
+stage's flux pass); its traffic comes from the committed rocprofv3
+FETCH_SIZE/WRITE_SIZE summary of the same workload.  The CPU baseline times the oracle (a
 restatement of the reference CPU kernels) on a bounded sample of the same
 workload, on every core the process may use.
 
@@ -58,7 +58,9 @@ HBM_PEAK_GBS = 8000.0
 ALGO_BYTES = {
     "aux": (96.0, "point"),      # read w(5) 40 B + write w_aux(1:7) 56 B
     "euler_x": (96.0, "cell"),   # read w_aux(1:6,8) 56 B + write fl(5) 40 B
-    "euler_xy": (96.0, "cell"),  # x and y in one pass: read w_aux(1:6,8) 56 B + write fl(5) 40 B
+    # the one-pass flux: read w(5) 40 B + mu 8 B, write fl(5) 40 B + div/3 8 B; the
+    # third stage also |omega| and the sensor: 96 + 16 / 3
+    "euler_xy": (304.0 / 3.0, "cell"),
     "visc": (120.0, "cell"),     # read w_aux(2,3,4,6,7) 40 B + fl(2:5) rw 64 B + write w_aux(9,10) 16 B
     "euler_y": (136.0, "cell"),  # read w_aux(1:6,8) 56 B + fl(5) rw 80 B
     "euler_z": (136.0, "cell"),
@@ -66,9 +68,10 @@ ALGO_BYTES = {
     "euler_zv": (184.0, "cell"),
     "sensor": (24.0, "cell"),    # read w_aux(9,10) + write w_aux(8)
     "visc_div": (144.0, "cell"), # w_aux(2,3,4,7,10) 40 + fl(2:5) rw 64 + fl_prev(1,2) 16 + w(1,2) 16 + T 8
-    # fl_prev 40 + fl 40 + w rw 80; the first Wray stage (rho = 0) skips fl_prev:
-    # (120 + 160 + 160) / 3 per launch over the three stages of a step
-    "update": (440.0 / 3.0, "cell"),
+    # with the grad(div/3) terms: fl 40 + w rw 80 + mu rw 16 + div/3 8, fl_prev 40 but
+    # at the first Wray stage (rho = 0), fl(2:5) 32 written but at the third:
+    # (176 + 216 + 184) / 3 per launch over the three stages of a step
+    "update": (192.0, "cell"),
     "dt": (40.0, "cell"),        # read w(5)
 }
 
@@ -192,8 +195,8 @@ def sbli_workload(args):
         res = g.compute_residual()
         kt = g.kernel_times(3)
         # FP64 byte counts; without channel forcing the viscous divergence
-        # terms need no force_rhs inputs (104 B/cell alone, 152 B/cell folded
-        # into the z march)
+        # terms of the separate sweeps need no force_rhs inputs (104 B/cell
+        # alone, 152 B/cell folded into the z march)
         nbytes = dict(ALGO_BYTES, visc_div=(104.0, "cell"), euler_zv=(152.0, "cell"))
         nvol = (nx + 6) * (ny + 6) * (nz + 6)
 

@@ -304,8 +304,8 @@ int st_compute_dt_noalloc(const st_params *p, void *hip_stream, const double *w,
 #define ST_K_DT         10
 #define ST_K_STEP_END   11
 #define ST_K_BC         12   /* physical ghost faces and characteristic boundaries */
-#define ST_K_EULER_XY   13   /* x and y Euler fluxes in one pass (y range spanning all rows) */
-#define ST_K_WENO_FIX   14   /* WENO faces of the Euler sweeps (list compaction + fix-up) */
+#define ST_K_EULER_XY   13   /* one-pass stage: every central flux and viscous term but grad(div/3); else x and y Euler fluxes in one pass */
+#define ST_K_WENO_FIX   14   /* WENO faces (one-pass stage: the step's masks + work items; else list compaction + fix-up) */
 #define ST_K_EULER_ZV   15   /* z Euler fluxes + viscous divergence terms + force_rhs partials (its z fix-up counts under ST_K_WENO_FIX) */
 #define ST_NKFAM        16
 int st_kernel_times(st_solver *s, int32_t nsteps, double ms[ST_NKFAM], int32_t count[ST_NKFAM]);

@@ -673,9 +673,8 @@ __global__ void k_rng_reset(Win31 seeded, uint32_t *__restrict__ win2, int *__re
 // dt evaluates the same primitives of the same w as compute_dt's own
 // compute_aux(central=1) at the start of the step.
 // Bound by HBM: 40 B read and 56 B written a point.  image & 2 leaves the
-// enthalpy out (8 B of 96): the one-pass stage forms it from the other
-// primitives, so only the last stage of a call (whose w_aux the caller can
-// read) and bc_nr want it.
+// enthalpy out (8 B of 96), which the one-pass stage reads nowhere: there only
+// the last stage of a call, whose w_aux the caller can read, wants it.
 template <typename R, bool DT = false>
 __device__ __forceinline__ void k_aux_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P, const double *__restrict__ w, R *__restrict__ wa,
                                              int i0, int ni, int j0, int nj, int k0, int nk, int image,

@@ -65,7 +65,7 @@ struct st_solver {
     int *rng_ctl;       // [0] window in use, [1] ticket of the draw kernel
     uint32_t rng_seeded[31];  // window right after seeding
     double *w_stat;     // running statistics w_stat(1:70, 1:nx, 1:ny), allocated on first use
-    bool dt_in_stage;   // the CFL reduction of this step rides on the first stage's aux
+    bool dt_in_stage;   // the CFL reduction of this step rides on its first stage
     int visc_chunk;     // planes per tile of the z-marching viscous kernel (0: automatic)
     int march_chunk;    // points per thread of the y/z flux marches (0: automatic)
     int dt_nblk;        // CFL block maxima that wait in dtpart
