@@ -82,16 +82,16 @@ __device__ __forceinline__ double mu_of(const KPar &P, const double (&c)[5]) {
 }
 
 // The largest spectral radius of compute_dt_subroutine (kernels_cpu.F90:
-// 6814-6880) at a point with the Euler metrics a and the viscous ones s, by
-// the operations of k_aux as mu_of.
-__device__ __forceinline__ double cfl_radius(const KPar &P, const double (&c)[5], const double (&a)[3],
+// 6814-6880) at a point of viscosity mu with the Euler metrics a and the
+// viscous ones s, by the operations of k_aux as mu_of.
+__device__ __forceinline__ double cfl_radius(const KPar &P, const double (&c)[5], double mu, const double (&a)[3],
                                              const double (&s)[3]) {
     const double ri = 1.0 / c[0];
     const double uu = c[1] * ri, vv = c[2] * ri, ww = c[3] * ri;
     const double qq = 0.5 * (uu * uu + vv * vv + ww * ww);
     const double ee = c[4] / c[0] - qq;
     const double tt = temperature_from_e(P, ee, P.t0);
-    const double nu = ri * viscosity_of(P, tt), kor = nu / P.prandtl;
+    const double nu = ri * mu, kor = nu / P.prandtl;
     const double cs = sqrt(gamloc_of(P, tt) * P.rgas0 * tt);
     double mx = fmax(fmax((fabs(uu) + cs) * a[0], (fabs(vv) + cs) * a[1]), (fabs(ww) + cs) * a[2]);
     mx = fmax(mx, fmax(nu * s[0], fmax(nu * s[1], nu * s[2])));

@@ -1375,7 +1375,7 @@ struct UpdArgs {
     int mu;            // the next stage reads the viscosity of the new state: store it
     int step_end;      // third stage of st_advance: icyc += 1, time += dt
     double *partials;  // block sums of rho u T dy (FV)
-    double *dtpart;    // block maxima of the CFL radii of the new state (null: not wanted)
+    double *dtpart;    // block maxima of the CFL radii of the new state (with mu; null: not wanted)
 };
 
 // visflx_div (kernels_cpu.F90:3484-3532, or its second-order form with O2,
@@ -1479,6 +1479,7 @@ __device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim
             wa[5 * nv + c] = R(tt);
             acc[0] += wn[1] * tt * dy;
         } else {
+            double mu_new = 0.0;
             // the cell's viscosity, and bcwall_staggered (kernels_cpu.F90:
             // 6612-6678) with the ghosts' at either wall
 #pragma unroll 1
@@ -1495,12 +1496,15 @@ __device__ __forceinline__ void k_update_div_body(const dim3 blockIdx, const dim
 #pragma unroll
                     for (int m = 0; m < 5; m++) w[m * nv + d] = x[m];
                 }
-                if (U.mu) wa[6 * nv + d] = R(mu_of(P, x));
+                if (!U.mu) continue;
+                const double m = mu_of(P, x);
+                wa[6 * nv + d] = R(m);
+                if (o == 0) mu_new = m;
             }
             if (!kFluxDt<R> && U.dtpart) {
                 const double a[3] = {U.dx1[i - 1], U.dy1[j - 1], U.dz1[k - 1]};
                 const double s[3] = {U.dxs[i - 1], U.dys[j - 1], U.dzs[k - 1]};
-                acc[0] = cfl_radius(P, wn, a, s);
+                acc[0] = cfl_radius(P, wn, mu_new, a, s);
             }
         }
     }
@@ -1558,12 +1562,12 @@ bool one_pass_stage(const st_solver *s) {
 static const int kFluxTX = 32, kFluxTY = 8;
 
 // Planes per workgroup of k_flux.  The chip holds two (FP64) or three (mixed)
-// workgroups a CU, and a round of them takes about chunk + 1.1 plane times
-// (4.7 us a plane and 5.2 us for the stencil's first planes and the launch, on
-// 512 x 256 x 256 at chunks 4, 8 and 16; with a CU to itself a workgroup takes
-// 3.4 us a plane).  Long chunks spare the start-up, short ones fill the chip
+// workgroups a CU, and a round of them takes about chunk + 1.3 plane times
+// (4.9 us a plane and 6.4 us for the stencil's first planes and the launch, on
+// 512 x 256 x 256 at chunks 1 to 32; with a CU to itself a workgroup takes
+// 3.8 us a plane).  Long chunks spare the start-up, short ones fill the chip
 // and its last round: the chunk with the least rounds x round time.  On
-// 128 x 96 x 64 chunks 2, 4, 8, 16 took 50, 47, 51, 66 us.
+// 128 x 96 x 64 chunks 2, 4, 8, 16 took 57, 54, 56, 73 us (7 is taken: 53).
 static int flux_chunk(const Geo &g, bool mixed) {
     const long tiles = (long)((g.nx + kFluxTX - 1) / kFluxTX) * ((g.ny + kFluxTY - 1) / kFluxTY);
     const int cus = 256, slots = cus * (mixed ? 3 : 2);
@@ -1571,7 +1575,7 @@ static int flux_chunk(const Geo &g, bool mixed) {
     double least = 0.0;
     for (int c = 1; c <= kFluxMaxChunk && c <= g.nz; c++) {
         const long blocks = tiles * ((g.nz + c - 1) / c);
-        const double t = blocks <= cus ? 1.1 + 0.73 * c : (double)((blocks + slots - 1) / slots) * (1.1 + c);
+        const double t = blocks <= cus ? 1.3 + 0.77 * c : (double)((blocks + slots - 1) / slots) * (1.3 + c);
         if (c == 1 || t < least) {
             least = t;
             best = c;
