@@ -132,17 +132,18 @@ __device__ __forceinline__ void wall_ghost(const Geo &g, const KPar &P, double *
 }
 
 // exclusive prefix over the block's 256 threads of v; *total receives the sum
-__device__ __forceinline__ int block_excl_scan256(int v, int *wsum, int *total) {
+template <typename T>
+__device__ __forceinline__ T block_excl_scan256(T v, T *wsum, T *total) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int x = v;
+    T x = v;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d, 64);
+        const T y = __shfl_up(x, d, 64);
         if (lane >= d) x += y;
     }
     if (lane == 63) wsum[wv] = x;
     __syncthreads();
-    int before = 0, tot = 0;
+    T before = 0, tot = 0;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         if (q < wv) before += wsum[q];

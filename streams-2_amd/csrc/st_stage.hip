@@ -22,6 +22,7 @@
 // have set.
 #include "st_device.h"
 #include "st_flux.h"
+#include "st_items.h"
 #include "st_solver.h"
 
 namespace st {
@@ -34,16 +35,10 @@ namespace st {
 // window of the reference kernels, kernels_cpu.F90:466-470).
 //
 // Layouts: hot bits, ceil(rx/64) words per ghosted row, bit e of a row the
-// point i = e + 1 - ng.  Cell records, one per 64 cells of an interior row
-// (row-major over j, k): words 2d and 2d+1 hold the lower-face and
-// upper-face bits of direction d (words 6, 7 unused: a record is one 64-byte
-// sector).
-constexpr int kRecWords = 8;
-constexpr int kItemSeg = 4096;       // list segments at most
+// point i = e + 1 - ng.  Cell records and list segments: st_items.h.
 constexpr int kItemBlocks = 512;     // workgroups of the item kernel at most (two per CU)
 
 __host__ __device__ __forceinline__ int hot_words(const Geo &g) { return (g.rx + 63) / 64; }
-__host__ __device__ __forceinline__ int rec_per_row(const Geo &g) { return (g.nx + 63) / 64; }
 
 // the cells with a WENO face, 32 cells of a row per entry, one word a direction
 __host__ __device__ __forceinline__ int dirty_per_row(const Geo &g) { return (g.nx + 31) / 32; }
@@ -90,10 +85,6 @@ __global__ __launch_bounds__(256) void k_hot_bits(Geo g, KPar P, const R *__rest
 // The list of a segment starts at its first cell's index, so it has room for
 // one item per cell; a segment with more writes none and reports -3 * cells:
 // its items are then all (cell, direction) pairs, read from the records.
-__device__ __forceinline__ int seg_first_cell(const Geo &g, int nwx, int wd, int nwords) {
-    return wd >= nwords ? (int)g.nint : (wd / nwx) * g.nx + 64 * (wd % nwx);
-}
-
 __device__ __forceinline__ void k_hot_items_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
                                                  const uint64_t *__restrict__ hot, uint64_t *__restrict__ rec,
                                                  uint3 *__restrict__ dirty, int wpt, int *__restrict__ list, int *__restrict__ counts) {
@@ -151,9 +142,9 @@ __device__ __forceinline__ void k_hot_items_body(const dim3 blockIdx, const dim3
     }
     int total;
     int off = block_excl_scan256(c, wsum, &total);
-    const bool dense = total > S1 - S0;
-    if (threadIdx.x == 0) counts[blockIdx.x] = dense ? -3 * (S1 - S0) : total;
-    if (c == 0 || dense) return;
+    const int report = segment_report(total, S1 - S0);
+    if (threadIdx.x == 0) counts[blockIdx.x] = report;
+    if (c == 0 || report < 0) return;
     int *seg = list + S0;
     for (int wd = wa0; wd < wa1; wd++) {
         const uint64_t *o = rec + (size_t)kRecWords * wd;
@@ -1101,22 +1092,22 @@ struct ItemArgs {
 template <typename R>
 __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim3 gridDim, Geo g, KPar P,
                                                   const double *__restrict__ w, R *__restrict__ fl, ItemArgs A) {
-    __shared__ int pre[kItemSeg + 1];
-    __shared__ int wsum[4];
+    __shared__ pair_t pre[kItemSeg + 1];
+    __shared__ pair_t wsum[4];
     __shared__ double lds[4][6];
     __shared__ bool last;
     const int t = threadIdx.x, lane = t & 63;
     double red[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    int total;
+    pair_t total;
     {
-        int cs[16], sum = 0;
+        pair_t cs[16], sum = 0;
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const int sgi = 16 * t + q;
-            cs[q] = sgi < A.nseg ? abs(A.counts[sgi]) : 0;
+            cs[q] = sgi < A.nseg ? segment_pairs(A.counts[sgi]) : 0;
             sum += cs[q];
         }
-        int run = block_excl_scan256(sum, wsum, &total);
+        pair_t run = block_excl_scan256(sum, wsum, &total);
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const int sgi = 16 * t + q;
@@ -1128,18 +1119,15 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
     }
     const size_t nv = g.nvol, ni = g.nint;
     const int nwx = rec_per_row(g), nwords = nwx * g.ny * g.nz;
-    // item e: its cell (linear) and code; in a segment without a list the
-    // (cell, direction) pairs in order, their masks from the records
-    auto item = [&](int e, int &cell, int &code) {
-        int lo = 0, hi = A.nseg;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (pre[mid] <= e) lo = mid;
-            else hi = mid;
-        }
+    // item `odd` of pair e: its cell (linear) and code, both left alone for a
+    // blank; in a segment without a list the (cell, direction) pairs in order,
+    // their masks from the records
+    auto item = [&](pair_t e, int odd, int &cell, int &code) {
+        const int lo = pair_segment(pre, A.nseg, e);
         const int S0 = seg_first_cell(g, nwx, lo * 256 * A.wpt, nwords);
-        const int x = e - pre[lo];
-        if (A.counts[lo] >= 0) {
+        const int x = 2 * (int)(e - pre[lo]) + odd, report = A.counts[lo];
+        if (x >= segment_items(report)) return;
+        if (report >= 0) {
             code = A.list[S0 + x];
             cell = S0 + (code & 0xffffff);
         } else {
@@ -1157,12 +1145,12 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
     C.tb = uniform(1.0 / cpc(P, 0));
     C.ta = uniform(P.t0 - cpc(P, P.indx_cp_r + 1) * P.t0 * C.tb);
     const double te = uniform(1.0 / C.eb), t0e = uniform(P.t0 - cvc(P, P.indx_cp_r + 1) * P.t0 * te);  // T = t0e + te e
-    const int wave = (blockIdx.x * blockDim.x + t) >> 6;
-    const int nwaves = (gridDim.x * blockDim.x) >> 6;
-    for (int base = wave * 62; base < total; base += nwaves * 62) {
-        const int e = base + lane;
+    const unsigned wave = (blockIdx.x * blockDim.x + t) >> 6;
+    const unsigned nwaves = (gridDim.x * blockDim.x) >> 6;
+    for (pair_t base = wave * 31; base < total; base += nwaves * 31) {
+        const pair_t e = base + (lane >> 1);
         int cell = -1, code = 0;
-        if (e < total) item(e, cell, code);
+        if (e < total) item(e, lane & 1, cell, code);
         const bool lo_hot = (code >> 26) & 1, hi_hot = (code >> 27) & 1;
         const bool work = cell >= 0 && (lo_hot || hi_hot);
         double d[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -1249,7 +1237,7 @@ __device__ __forceinline__ void k_weno_items_body(const dim3 blockIdx, const dim
         if (lane == 0) {
             cm = -1;
             int cd;
-            if (base > 0) item(base - 1, cm, cd);
+            if (base > 0) item(base - 1, 1, cm, cd);
         }
 #pragma unroll
         for (int m = 0; m < 5; m++) {
@@ -1597,14 +1585,6 @@ int one_pass_update_blocks(const Geo &g) { return nblocks(update_grid(g)); }
 int one_pass_dt_slots(const Geo &g) {
     const int f = nblocks(flux_grid(g, 1)), a = aux_dt_blocks(g), u = one_pass_update_blocks(g);
     return f > a ? (f > u ? f : u) : (a > u ? a : u);
-}
-
-static int item_segments(const Geo &g, int *wpt) {
-    const long nwords = (long)rec_per_row(g) * g.ny * g.nz;
-    long per = (nwords + 256L * kItemSeg - 1) / (256L * kItemSeg);
-    if (per < 1) per = 1;
-    *wpt = (int)per;
-    return (int)((nwords + 256 * per - 1) / (256 * per));
 }
 
 hipError_t launch_hot_items(st_solver *s) {
