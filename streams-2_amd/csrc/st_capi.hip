@@ -639,9 +639,16 @@ int st_set_grid(st_solver *s, const double *x, const double *y, const double *z,
     s->jbl = 0;
     for (int j = 1; j <= g.ny; j++)
         if (s->p.l0 > y[j + g.ng - 1]) s->jbl = j;
-    // the metric of equal nodes agrees to their round-off
+    // the x metric of equal nodes agrees to their round-off
     s->x_uniform = true;
     for (int i = 1; i < g.nx; i++) s->x_uniform = s->x_uniform && std::fabs(dcsidx[i] / dcsidx[0] - 1.0) <= 1e-11;
+    if (s->p.conservative_viscous == 1) {
+        // this form's derivatives divide by x(i+1) - x(i-1) instead, which
+        // carries the coordinates' own round-off too
+        const double *xi = x + g.ng - 1, d = xi[2] - xi[0];
+        const double tol = 1e-11 * std::fabs(d) + 1e-15 * std::fmax(std::fabs(xi[0]), std::fabs(xi[g.nx + 1]));
+        for (int i = 2; i <= g.nx; i++) s->x_uniform = s->x_uniform && std::fabs(xi[i + 1] - xi[i - 1] - d) <= tol;
+    }
     s->grid_set = true;
     return ST_OK;
 }

@@ -70,7 +70,7 @@ struct st_solver {
     int march_chunk;    // points per thread of the y/z flux marches (0: automatic)
     int dt_nblk;        // CFL block maxima that wait in dtpart
     bool dt_waits;      // the last update left those of its new state
-    bool x_uniform;     // dcsidx is one value (set by st_set_grid)
+    bool x_uniform;     // dcsidx, and in the conservative form the node spacing, is one value (set by st_set_grid)
     bool fuse_xy;       // x and y Euler fluxes in one pass
     bool fuse_zv;       // viscous divergence terms folded into the z march (Laplacian form)
     int force_nblk;     // force_rhs partials written in this stage (visc_div blocks, or z march + fix-up)
