@@ -85,7 +85,9 @@ struct Job {
     }
     bool wait(int q) { return ok(ev ? hipEventSynchronize(ev[q]) : hipStreamSynchronize(s->stream)); }
     // Two buffers a thread: one on the link while the other is re-spaced.
-    // Every chunk is waited for before its buffer or this thread goes away.
+    // Every chunk is waited for before its buffer or this thread goes away: out
+    // says whether one may be in flight, also where its event could not be
+    // recorded or waited for.
     void run(int t) {
         char *b[2] = {mem + 2 * t * bytes, mem + (2 * t + 1) * bytes};
         bool out[2] = {false, false};
@@ -95,17 +97,17 @@ struct Job {
             const bool more = c < chunks;
             if (more) {
                 if (out[q]) {  // in: the buffer's last chunk
-                    out[q] = false;
                     if (!wait(2 * t + q)) break;
+                    out[q] = false;
                 }
                 if (in) pack(b[q], c);
-                if (!issue(b[q], c, 2 * t + q)) break;
                 out[q] = true;
+                if (!issue(b[q], c, 2 * t + q)) break;
                 held[q] = c;
             }
             if (!in && out[q ^ 1]) {
-                out[q ^ 1] = false;
                 if (!wait(2 * t + (q ^ 1))) break;
+                out[q ^ 1] = false;
                 unpack(b[q ^ 1], held[q ^ 1]);
             }
             if (!more && !(out[0] && !in) && !(out[1] && !in)) break;

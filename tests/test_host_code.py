@@ -24,3 +24,8 @@ def _run(tmp_path, *sources):
 def test_work_items_are_numbered_past_32_bits(tmp_path):
     r = _run(tmp_path, os.path.join(HOST, "items_host.hip"))
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_field_copies_leave_nothing_in_flight(tmp_path):
+    r = _run(tmp_path, os.path.join(HOST, "copy_host.hip"), os.path.join(ROOT, "streams-2_amd", "csrc", "st_copy.hip"))
+    assert r.returncode == 0, r.stdout + r.stderr
