@@ -469,9 +469,8 @@ int create_solver(const st_params *p, const st::SlotMem *mem, st_solver **out) {
     *out = nullptr;
     int rc = validate(p);
     if (rc) return rc;
-    st_solver *s = new (std::nothrow) st_solver();
+    st_solver *s = new (std::nothrow) st_solver();  // value-initialised: zeros, and the staging's own members
     if (!s) return fail(ST_ERR_NOMEM, "host allocation failed");
-    std::memset((void *)s, 0, sizeof(st_solver));
     s->p = *p;
     s->fuse_xy = true;
     s->fuse_zv = true;
