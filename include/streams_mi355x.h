@@ -310,11 +310,16 @@ int st_compute_dt_noalloc(const st_params *p, void *hip_stream, const double *w,
 #define ST_NKFAM        16
 int st_kernel_times(st_solver *s, int32_t nsteps, double ms[ST_NKFAM], int32_t count[ST_NKFAM]);
 
-/* Stream used by every launch of this solver (NULL = the library's own). */
-/* Launch shapes (no reference counterpart; tuning only): planes per tile
- * of the z-marching viscous kernel and points per thread of the y/z flux
- * marches, 0 = automatic.  Results do not depend on them. */
+/* Launch shapes (no reference counterpart; tuning only), 0 = automatic.
+ * Results do not depend on them.  Where the stage runs in one pass (KEEP
+ * split with nkeep 0, calorically perfect gas, Roe WENO split, periodic
+ * span; a channel also periodic and equally spaced in x) visc_chunk is the
+ * planes per workgroup of its flux kernel (32 at most) if there are no bulk
+ * sums to group by them, and both are without effect in a channel.
+ * Elsewhere: planes per tile of the z-marching viscous kernel, and points
+ * per thread of the y/z flux marches. */
 int st_set_tuning(st_solver *s, int32_t visc_chunk, int32_t march_chunk);
+/* Stream used by every launch of this solver (NULL = the library's own). */
 int st_set_stream(st_solver *s, void *hip_stream);
 int st_synchronize(st_solver *s);
 
@@ -326,10 +331,12 @@ const char *st_version(void);
  * admitted in arrival order as slots and HBM free up (the server holds
  * hbm_capacity_bytes as one device pool from its creation and carves each
  * solve's st_solver_footprint out of it: no allocation while solves run),
- * each runs on its own stream from a HIP graph of steps_per_graph steps
- * (0: no graph), and their work overlaps on the device.  autotune != 0
+ * each runs on its own stream, from a HIP graph of steps_per_graph steps
+ * where five such chunks or more are left (0: no graph), and their work
+ * overlaps on the device.  autotune != 0
  * times launch shapes (st_set_tuning) on the first solves of each
- * grid-shape class, during their own steps, and keeps the fastest.  A
+ * grid-shape class, during their own steps, and keeps the fastest; a class
+ * with one launch shape (a channel in one pass) is settled from the start.  A
  * result is identical to the same solve run alone through st_advance. */
 typedef struct st_server st_server;
 int st_server_create(int64_t hbm_capacity_bytes, int32_t max_slots, int32_t steps_per_graph, int32_t autotune,

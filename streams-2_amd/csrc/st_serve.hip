@@ -17,20 +17,22 @@
 // Threads.  The scheduler thread never waits on the device: it admits
 // requests (pool block + slot), launches chunks of K steps on each active
 // slot's stream (from a captured HIP graph once the class's launch shape
-// is settled), keeps two chunks in flight per slot and polls their events.
-// A worker thread does what blocks: the set-up of an admitted solve on its
+// is settled and where enough of the solve is left), keeps two chunks in
+// flight per slot and polls their events.  A worker thread does what blocks: the set-up of an admitted solve on its
 // slot (tables, grid and field copies, start of run), the hand-back of a
 // finished one (residual, field copy, pool block and slot released) and
 // the writing of checkpoint files.  The work of all active solves overlaps
 // on the device.
 //
 // Launch shapes are tuned online per grid-shape class (each extent rounded
-// up to a power of two, precision, viscous form): the first chunks of the
-// first solves of a class run with the candidate shapes in turn, timed by
-// events on their own streams, and once every candidate has a time the
-// fastest is kept for the class.  Results do not depend on the launch
-// shape, so the tuning chunks are ordinary steps of the solves: no step is
-// run twice and no solve waits for the tuner.
+// up to a power of two, precision, viscous form, and which chunks shape a
+// launch of its steps): the first chunks of the first solves of a class run
+// with the candidate shapes in turn, timed by events on their own streams,
+// and once every candidate has a time the fastest is kept for the class.
+// Results do not depend on the launch shape, so the tuning chunks are
+// ordinary steps of the solves: no step is run twice and no solve waits for
+// the tuner.  A class whose launches are fixed by its grids (the one-pass
+// stage with bulk sums) is settled from the start.
 //
 // Checkpoints (the restart files of a request, rst.bin + field_info0.dat
 // in the formats of field.F90:1853-1966 and singleideal.F90:2546-2659):
@@ -123,7 +125,7 @@ enum SlotState { kFree, kSetup, kRunning, kDraining };
 
 constexpr int kTabInts = 1 << 16;  // pinned table staging: nx + ny + nz + 3 ints at most
 
-using TuneKey = std::tuple<int, int, int, int, int>;
+using TuneKey = std::tuple<int, int, int, int, int, int>;  // the last one launch_shapes, known after set-up
 
 struct Tune {
     std::vector<std::pair<int, int>> cand;  // (visc_chunk, march_chunk)
@@ -227,6 +229,13 @@ struct Batcher {
 constexpr size_t kBatchTabBytes = (size_t)32 << 20;  // per table buffer
 constexpr int kMaxLanes = 8;
 
+// A solve captures its graph while at least this many whole chunks are left:
+// the capture takes the scheduler, which launches for every solve, about as
+// long as four plain chunks.  16 solves of 32 to 64 cells a side, chunks of 10
+// steps, with a graph always / from five chunks on, ms: 20 steps 42 / 35, 40
+// steps 60 / 51 (in two batch lanes 78 / 63), 80 steps 98 / 94, 200 steps the
+// same.
+constexpr int kGraphChunks = 5;
 constexpr int kPlainChunk = 10;  // steps per chunk of a server without graphs (steps_per_graph 0 or 1)
 
 enum JobKind { kSetupJob, kFinishJob, kCheckpointJob };
@@ -321,6 +330,7 @@ int setup(st_server *sv, Slot &sl) {
                           gd[6].data(), gd[7].data(), gd[8].data(), gd[9].data(), gd[10].data(), gd[11].data(),
                           gd[12].data())))
         return rc;
+    std::get<5>(sl.key) = st::launch_shapes(sl.s);
     if ((rc = st_copy_from_field(sl.s, r->w0.data())) || (rc = st_init_run(sl.s))) return rc;
     // whether a chunk of its steps records in body form, and its launch
     // sequence (solves whose sequences agree are batched together)
@@ -495,13 +505,25 @@ void push_job(st_server *sv, JobKind k, int slot) {
     sv->cv_job.notify_all();
 }
 
-// Scheduler: the candidate shapes of a class.
-Tune make_tune() {
+// Scheduler: the class of a solve, made on first sight (the caller holds
+// sv->mu).  Its candidates differ in a launch of the solve's steps; a class
+// with one alone is settled.
+Tune &tune_of(st_server *sv, const Slot &sl) {
+    auto it = sv->tune.find(sl.key);
+    if (it != sv->tune.end()) return it->second;
     Tune t;
-    t.cand = {{0, 0}, {8, 8}, {8, 16}, {16, 16}, {16, 32}, {32, 16}, {32, 32}, {8, 32}, {32, 8}};
+    const int shapes = std::get<5>(sl.key);
+    if (shapes & st::kShapeMarch)
+        t.cand = {{0, 0}, {8, 8}, {8, 16}, {16, 16}, {16, 32}, {32, 16}, {32, 32}, {8, 32}, {32, 8}};
+    else if (shapes & st::kShapeVisc) t.cand = {{0, 0}, {8, 0}, {16, 0}, {32, 0}};
+    else t.cand = {{0, 0}};
     t.ms.assign(t.cand.size(), -1.f);
     t.assigned.assign(t.cand.size(), 0);
-    return t;
+    if (t.cand.size() == 1) {
+        t.done = true;
+        sv->tuned_classes++;
+    }
+    return sv->tune.emplace(sl.key, std::move(t)).first->second;
 }
 
 // Scheduler: enqueue the next chunk of steps of a slot and record its
@@ -517,9 +539,7 @@ int launch_chunk(st_server *sv, Slot &sl) {
     Tune *t = nullptr;
     if (sv->autotune) {
         std::lock_guard<std::mutex> lk(sv->mu);
-        auto it = sv->tune.find(sl.key);
-        if (it == sv->tune.end()) it = sv->tune.emplace(sl.key, make_tune()).first;
-        t = &it->second;
+        t = &tune_of(sv, sl);
         if (!t->done && n == per) {
             for (size_t q = 0; q < t->cand.size(); q++)
                 if (!t->assigned[q]) {
@@ -538,7 +558,7 @@ int launch_chunk(st_server *sv, Slot &sl) {
     } else {
         bool use_graph = false;
         if (n == sv->K && graphable(sv, r)) {
-            if (!sl.exec && (!t || t->done)) {
+            if (!sl.exec && (!t || t->done) && left >= kGraphChunks * per) {
                 if (t && (rc = st_set_tuning(s, t->best.first, t->best.second))) return rc;
                 if ((rc = capture(sv, sl))) return rc;
             }
@@ -620,10 +640,9 @@ void drop_candidates(st_server *sv, Slot &sl) {
 bool class_done(st_server *sv, const Slot &sl, Tune *best = nullptr) {
     if (!sv->autotune) return true;
     std::lock_guard<std::mutex> lk(sv->mu);
-    auto it = sv->tune.find(sl.key);
-    if (it == sv->tune.end() || !it->second.done) return false;
-    if (best) *best = it->second;
-    return true;
+    const Tune &t = tune_of(sv, sl);
+    if (t.done && best) *best = t;
+    return t.done;
 }
 
 // Scheduler: a solve whose next chunk belongs in a batch (it shares its
@@ -954,7 +973,7 @@ void serve_loop(st_server *sv) {
                 sl.off = off;
                 sl.rc = ST_OK;
                 sl.key = TuneKey{pow2_ceil(r->p.nx), pow2_ceil(r->p.ny), pow2_ceil(r->p.nz), r->p.precision,
-                                 r->p.conservative_viscous};
+                                 r->p.conservative_viscous, 0};
                 sl.tcand[0] = sl.tcand[1] = -1;
                 sv->used += r->bytes;
                 r->state = 1;

@@ -66,8 +66,8 @@ struct st_solver {
     uint32_t rng_seeded[31];  // window right after seeding
     double *w_stat;     // running statistics w_stat(1:70, 1:nx, 1:ny), allocated on first use
     bool dt_in_stage;   // the CFL reduction of this step rides on its first stage
-    int visc_chunk;     // planes per tile of the z-marching viscous kernel (0: automatic)
-    int march_chunk;    // points per thread of the y/z flux marches (0: automatic)
+    int visc_chunk;     // planes per workgroup of k_flux (without bulk sums, kFluxMaxChunk at most) or per tile of the viscous march (0: automatic)
+    int march_chunk;    // points per thread of the y/z flux marches of the separate sweeps (0: automatic)
     int dt_nblk;        // CFL block maxima that wait in dtpart
     bool dt_waits;      // the last update left those of its new state
     bool x_uniform;     // dcsidx, and in the conservative form the node spacing, is one value (set by st_set_grid)
@@ -244,6 +244,9 @@ hipError_t launch_force_var(st_solver *s, int nblk, bool mu = false);
 int update_blocks(const Geo &g);
 // ---- one-pass stage (st_stage.hip)
 bool one_pass_stage(const st_solver *s);
+// which of st_set_tuning's chunks shape a launch of the solver's steps
+constexpr int kShapeVisc = 1, kShapeMarch = 2;
+int launch_shapes(const st_solver *s);
 size_t hot_bits_bytes(const Geo &g);
 size_t hot_rec_bytes(const Geo &g);
 size_t hot_dirty_bytes(const Geo &g);

@@ -1547,6 +1547,13 @@ bool one_pass_stage(const st_solver *s) {
            (!p.channel_case || (s->kp.periodic[0] && s->x_uniform));
 }
 
+// With the bulk sums launch_flux fixes the chunk by the grid, without them
+// visc_chunk sets it; the separate sweeps take both.
+int launch_shapes(const st_solver *s) {
+    if (!one_pass_stage(s)) return kShapeVisc | kShapeMarch;
+    return s->p.channel_case ? 0 : kShapeVisc;
+}
+
 static const int kFluxTX = 32, kFluxTY = 8;
 
 // Planes per workgroup of k_flux.  The chip holds two (FP64) or three (mixed)

@@ -303,3 +303,39 @@ def test_closing_with_batched_chunks_in_flight():
                       want_fields=True, timeout=120.0, batch=1)
     for n, (a, b) in enumerate(zip(seq["results"], srv["results"])):
         assert np.array_equal(interior(a["w"]), interior(b["w"])), n
+
+
+@pytest.mark.parametrize("bulk_sums", [True, False])
+def test_the_tuner_times_only_launch_shapes_that_differ(bulk_sums):
+    """Four requests of one class, two chunks each: fewer chunks than the nine
+    candidates of the separate sweeps.  A channel in one pass has one launch
+    shape, so its class is settled at once and its solves share a batch; without
+    bulk sums there are four, which these chunks can time."""
+    from streams_mi355x.cases import make_bl_box
+
+    if bulk_sums:
+        reqs = [Request(make_channel(nx=40, ny=24, nz=20, seed=n), 80, 0.0) for n in range(4)]
+    else:
+        reqs = [Request(make_bl_box(nx=40, ny=24, nz=20, seed=n, bctags=(1, 4, 6, 4, 0, 0), bctags_nr=(0,) * 6), 80, 0.0)
+                for n in range(4)]
+    seq = run_sequential(reqs, want_fields=True)
+    srv = run_serving(reqs, hbm_bytes=8 << 30, max_slots=4, steps_per_graph=40, autotune=True, want_fields=True,
+                      timeout=60.0, batch=1)
+    assert srv["stats"]["tuned_classes"] == 1
+    assert (srv["stats"]["batched_chunks"] > 0) == bulk_sums
+    for n, (a, b) in enumerate(zip(seq["results"], srv["results"])):
+        assert b["error"] is None, (n, b["error"])
+        assert np.array_equal(interior(a["w"]), interior(b["w"])), n
+
+
+@pytest.mark.parametrize("nsteps", [18, 20, 22])
+def test_solves_on_either_side_of_the_graph_capture(nsteps):
+    """A solve captures its graph while five whole chunks are left: none, one
+    replayed to the end and one followed by a shorter chunk."""
+    reqs = [Request(r.case, nsteps, 0.0) for r in _requests()[:3]]
+    seq = run_sequential(reqs, want_fields=True)
+    srv = run_serving(reqs, hbm_bytes=8 << 30, max_slots=3, steps_per_graph=4, autotune=True, want_fields=True,
+                      timeout=60.0)
+    for n, (a, b) in enumerate(zip(seq["results"], srv["results"])):
+        assert np.array_equal(interior(a["w"]), interior(b["w"])), n
+        assert b["scalars"]["icyc"] == nsteps
