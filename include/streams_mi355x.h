@@ -129,7 +129,9 @@ typedef struct st_solver st_solver;
 /* ---- lifecycle: device allocation owned by the library -------------------
  * Replaces the hipfort hipMalloc of the backend arrays
  * (base_amd.F90:1211-1413, singleideal_amd.F90:1268-1327) and the setup of
- * bc_preproc / correct_bc_order (singleideal.F90:4703-4750, 946-993). */
+ * bc_preproc / correct_bc_order (singleideal.F90:4703-4750, 946-993).
+ * A solver also holds pinned host memory, the staging of its field copies:
+ * as much as its field, 32 MiB at most (solves inside a server share one). */
 int st_solver_create(const st_params *p, st_solver **out);
 int st_solver_destroy(st_solver *s);
 /* Bytes of HBM one solve of these sizes occupies (admission control). */

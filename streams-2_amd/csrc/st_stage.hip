@@ -447,9 +447,11 @@ struct FluxArgs {
 // The primitives are formed from w as a point enters the window or the halo,
 // about 20 operations each for two points a lane and plane: 512 x 256 x 256
 // 1.25 -> 1.36 ms, for the aux pass of 0.60 ms and half of the reads.
-// Bound by FP64 issue: ~870 vector instructions a wave and plane, 4.4 cycles
-// each at the ~2.0 GHz of a loaded chip (59 TFLOP/s of FMAs measured), 77 % of
-// the kernel's time.  512 x 256 x 256, with the bulk sums: 1.36 ms, where the
+// Bound by vector issue and what two waves cannot hide of the waits: ~770
+// vector instructions a wave and plane with the start-up planes (77 % of them
+// FP64), which keep the vector units busy for 57 % of the cycles at the 2.0 GHz
+// of a loaded chip; the waves wait for 30 % of theirs (counters on
+// 512 x 256 x 256).  There, with the bulk sums: 1.36 to 1.41 ms, where the
 // passes it replaces took 0.64 + 0.85 + 0.99 + 1.37; 128 x 96 x 64: 52 us for
 // 20 + 38 + 35 + 41.  Mixed, 256 x 192 x 128: 203 us for 131 + 124 + 115 + 175.
 template <typename T>
@@ -1080,9 +1082,9 @@ struct ItemArgs {
 // the first 62.  All directions share one launch, and every face is hybrid
 // per lane; bound by the latency of the scattered stencil loads and, where
 // WENO cells are many, by the arithmetic of the faces.  On 384 x 128 x 96 with
-// a shock (1.6 % WENO faces) 69 us a stage, with the general characteristic
-// routines of st_flux.h at one wave per SIMD 125; on 512 x 256 x 256 after 25
-// steps 0.32 ms for 0.43.
+// a shock (1.6 % WENO faces) 71 us a stage, with the general characteristic
+// routines of st_flux.h at one wave per SIMD 125; on 512 x 256 x 256 0.29 ms
+// after 25 steps (0.54 % of the faces; 0.54 ms averaged over them).
 //
 // The workgroups then finish the reductions of the stage (two levels, fixed
 // order): the bulk sums of k_flux with the items' changes, giving b1, b2,
@@ -1380,7 +1382,9 @@ struct UpdArgs {
 // wave per SIMD less and 4 % slower (and without it no faster, 1379 against
 // 1371 us).  Bound by HBM: 40 + 40 + 40 + 8 + 8 B read and 32 + 40 + 8 B
 // written a cell (the third stage mostly without the 32), 1.33 ms a stage on
-// 512 x 256 x 256 (5.2 TB/s), 34 us on 128 x 96 x 64.  The right-hand sides are
+// 512 x 256 x 256 (5.1 TB/s in the bytes moved, where k_aux moves 5.6; 112
+// registers leave four waves per SIMD, whose vector units are busy for 37 % of
+// the cycles), 34 us on 128 x 96 x 64.  The right-hand sides are
 // read with the non-temporal hint: neither is read again before a full stage of
 // traffic has passed.
 template <typename R, bool FV, bool O2>
@@ -1680,7 +1684,7 @@ hipError_t launch_update_div(st_solver *s, const void *fl_prev, void *fl, int st
     U.rkg = s->gamrk[stage];
     U.channel = s->p.channel_case;
     // the first two stages' are F[prev] of the next; the third's has no reader
-    // but the caller, and is left out (32 of 184 B a cell) while further steps
+    // but the caller, and is left out (32 of 216 B a cell) while further steps
     // of the call follow: 512x256x256 1380 -> 1307 us a stage over three stages
     U.keep = stage < 2 || last;
     U.mu = mu && !fv;
