@@ -16,8 +16,8 @@ constexpr int kItemSeg = 4096;  // list segments at most
 // A launch numbers its items in pairs, a segment of an odd number ending in a
 // blank.  A cell has up to three items: a grid of 2^31 points, the largest a
 // solver takes, has 3.2e9 pairs at most, where the items themselves would not
-// fit 32 bits.  (64-bit numbers in the kernel's search and prefix took 269 us
-// for the 262 of this on 512 x 256 x 256.)
+// fit 32 bits.  (64-bit numbers in the kernel's search and prefix: 269 us for
+// the 262 of this on 512 x 256 x 256, the masks of the step averaged in.)
 using pair_t = unsigned;
 
 __host__ __device__ __forceinline__ int rec_per_row(const Geo &g) { return (g.nx + 63) / 64; }

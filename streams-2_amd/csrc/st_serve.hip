@@ -569,7 +569,8 @@ int launch_chunk(st_server *sv, Slot &sl) {
             s->icyc += n;
             s->last_stage = 2;
         } else {
-            if (t && !t->done && (rc = st_set_tuning(s, 0, 0))) return rc;
+            // (automatic while the class is not settled)
+            if (t && (rc = st_set_tuning(s, t->best.first, t->best.second))) return rc;
             if ((rc = st_advance(s, n))) return rc;
         }
     }
